@@ -201,6 +201,8 @@ uint64_t gdn_bytes(const GdnArgs& g) {
     return 2 * vh * sd * sd * 4 + (2 * kh * sd + vh * sd) * 4 + vh * sd * 4 * 2 + vh * 8;
 }
 
+constexpr uint64_t kMatvecMaxCols = 12288 + 4096;  // inputs that a workgroup stages in LDS
+
 bool is_matrix(const Weight* w) { return w && w->rows >= 1 && w->cols >= 1; }
 
 // Grouped matvec over weights with one input; splits the list into runs of equal type.
@@ -226,7 +228,7 @@ emprise_status run_matvec(emprise_hip* h, const Proj* p, int n, int mode, const 
     const uint64_t cols = p[0].w->cols;
     for (int i = 0; i < n; ++i)
         if (p[i].w->cols != cols) return fail(EMPRISE_EINVAL, "projections sharing an input need equal columns");
-    if (cols > 12288 + 4096) return fail(EMPRISE_EINVAL, "input width %llu exceeds the staged-input limit", (unsigned long long)cols);
+    if (cols > kMatvecMaxCols) return fail(EMPRISE_EINVAL, "input width %llu exceeds the staged-input limit", (unsigned long long)cols);
     bool first = true;
     for (int i = 0; i < n;) {
         int j = i + 1;
@@ -566,8 +568,7 @@ emprise_status emprise_hip_linear_norm(emprise_hip* h, const emprise_hip_input* 
     return run_matvec(h, p, n, kMvPlain, in, nullptr, nullptr, nullptr, 0, nullptr);
 }
 
-// Batches of at least this many tokens run as a GEMM on the matrix cores; smaller ones
-// as matvecs, which read the weights once per token at full HBM speed.
+// Batches of at least this many tokens run as a GEMM whatever the weights (on_gemm).
 constexpr int kGemmMinBatch = 8;
 constexpr size_t kGemmScratchBytes = size_t(256) << 20;  // dequantised weight rows per GEMM pass
 
@@ -577,34 +578,115 @@ emprise_status emprise_hip_linear_batch(emprise_hip* h, emprise_weight w, empris
     return emprise_hip_linear_batch_strided(h, w, X, wt->cols, Y, wt->rows, K);
 }
 
-// Y[k] = [W_0; W_1; ...] X[k]: the weights' rows side by side in Y, for K rows of X. From
-// kGemmMinBatch rows up the projections run as GEMMs on the matrix cores -- chunked
-// Q6_K/Q4_K weights on exact fp16 pieces, consecutive weights of one type (q|k|v, the
-// recurrent in-projections) sharing a launch and its full tiles; other weights
-// dequantised exactly to FP32 -- and below that as the streaming matvec per row of X.
+static size_t part_bytes(int M, uint64_t N, int K) {
+    const int layers = gemm_q16_layers(M, (int)N, K);
+    return layers > 1 ? (size_t)layers * M * N * sizeof(float) : 0;
+}
+
+// The fp16 GEMM over the stacked weights of `a`, with scratch for its partial sums (without
+// it, where a graph is being captured and none is there yet, the spans run one after the
+// other, with the same sums).
+static emprise_status run_gemm_q16(emprise_hip* h, uint32_t type, QGemmArgs& a, uint64_t flops) {
+    const size_t bytes = part_bytes(a.M, a.N, a.K);
+    a.part = nullptr;
+    if (bytes && (gemm_q16_few(a.M) || !h->capturing || h->scratch["gemm_part"].bytes >= bytes)) {
+        void* part;
+        TRY(h->get_scratch("gemm_part", bytes, &part));
+        a.part = static_cast<float*>(part);
+    }
+    return traced(h, "gemm_q16", flops, [&] { return launch_gemm_q16(type, a, h->stream); });
+}
+
+// The activation half of `qa` for M rows of X: split into fp16 pieces in scratch, or left to
+// the GEMM itself where there are few.
+static emprise_status split_q16(emprise_hip* h, const float* X, int M, int cols, int ldx, bool sums, QGemmArgs* qa) {
+    qa->x = X;
+    qa->ldx = ldx;
+    qa->M = M;
+    qa->K = cols;
+    if (gemm_q16_few(M)) return EMPRISE_OK;
+    void* xs;
+    TRY(h->get_scratch("gemm_xs", gemm_q16_split_bytes(M, cols, sums), &xs));
+    return traced(h, "split_f16", (uint64_t)M * cols * 8,
+                  [&] { return launch_gemm_q16_split(X, M, cols, ldx, xs, sums, qa, h->stream); });
+}
+
+// Inputs of one small-batch launch over this matrix (1: not a matrix it takes).
+static int small_batch(const emprise_hip* h, const Weight* wt) {
+    if ((wt->type != kQ6K && wt->type != kQ4K) || !chunked_cols(wt->cols) || (h->q8 && wt->type == kQ6K)) return 1;
+    int per = kBatchMax;
+    while (per > 1 && matvec_batch_lds_bytes(wt->type, (int)wt->cols, per) > kBatchLdsMax) --per;
+    return per;
+}
+
+// Whether K rows of X (16-byte aligned rows) go through this weight as a GEMM. Q6_K/Q4_K:
+// once the rows no longer fit one small-batch launch, which reads the weights once as well
+// (us, one launch against the GEMM's two: Q6_K 4096 x 4096 9.3 / 14.3 at 4 rows and 15.1 /
+// 14.4 at 5, 4096 x 12288 19.6 / 26.0 at 3 and 29.0 / 26.0 at 4); widths the small-batch
+// kernel does not take from 2 rows on (2048 x 6144 at 3 rows 27.4 as three matvecs, 14.0).
+// Q6_K under --fast-q8 keeps the single-input path, which quantises its input, up to
+// kGemmMinBatch, as do the unquantised types, whose GEMM fills 128-row tiles.
+// (`rows`: of all the weights of the call. The form for few rows keeps its partial sums in
+// scratch, which cannot grow while a graph is being captured.)
+static bool on_gemm(emprise_hip* h, const Weight* wt, int K, uint64_t rows) {
+    if (wt->type != kQ6K && wt->type != kQ4K) return K >= kGemmMinBatch && wt->cols % 16 == 0;
+    if (K < kGemmMinBatch && ((h->q8 && wt->type == kQ6K) || wt->cols > kMatvecMaxCols)) return false;
+    if (K <= small_batch(h, wt)) return false;
+    return !(gemm_q16_few(K) && h->capturing && !(h->q8 && wt->type == kQ6K) && h->scratch["gemm_part"].bytes < part_bytes(K, rows, (int)wt->cols));
+}
+
+// Y[k] = [W_0; W_1; ...] X[k]: the weights' rows side by side in Y, for K rows of X. Where
+// on_gemm says so the projections run as GEMMs on the matrix cores -- Q6_K/Q4_K weights on
+// exact fp16 pieces (gemm_q.hip), consecutive weights of one type (q|k|v, the recurrent
+// in-projections) in one launch; other weights dequantised (or copied, for F32 rows)
+// exactly into FP32 blocks and multiplied in FP32 -- else as small-batch launches or the
+// streaming matvec per row of X.
 static emprise_status linear_batch_rows(emprise_hip* h, int nw, const Weight* const* ws, emprise_dev X, uint64_t ldx,
                                         emprise_dev Y, uint64_t ldy, int K) {
     const int cols = (int)ws[0]->cols;
     uint64_t rows = 0;
-    bool all_f32 = true;
-    for (int i = 0; i < nw; ++i) rows += ws[i]->rows, all_f32 = all_f32 && ws[i]->type == kF32;
+    for (int i = 0; i < nw; ++i) rows += ws[i]->rows;
     if (ldx < (uint64_t)cols || ldy < rows || ldx > (1u << 30) || ldy > (1u << 30))
         return fail(EMPRISE_EINVAL, "row strides shorter than the matrix");
-    if (K < kGemmMinBatch || cols % 16 != 0 || X % 16 != 0 || ldx % 4 != 0) {
-        uint64_t off = 0;
-        for (int i = 0; i < nw; ++i) {
-            const Weight* wt = ws[i];
-            // 2..kGemmMinBatch-1 rows through a chunked Q6_K/Q4_K matrix: up to kBatchMax rows
-            // per launch, the weights read once per launch (--fast-q8 keeps Q6_K on the
-            // single-input path, which quantises its input)
-            const bool batched = K > 1 && (wt->type == kQ6K || wt->type == kQ4K) && chunked_cols(wt->cols) &&
-                                 !(h->q8 && wt->type == kQ6K) && X % 16 == 0 && ldx % 4 == 0;
-            int per = kBatchMax;
-            while (per > 1 && matvec_batch_lds_bytes(wt->type, cols, per) > kBatchLdsMax) --per;
+    const bool aligned = X % 16 == 0 && ldx % 4 == 0;
+    const float* A = reinterpret_cast<const float*>(X);
+    float* C = reinterpret_cast<float*>(Y);
+    const uint64_t flops_per_row = 2ull * (uint64_t)K * (uint64_t)cols;
+    auto on_q16 = [&](const Weight* wt) { return aligned && (wt->type == kQ6K || wt->type == kQ4K) && on_gemm(h, wt, K, rows); };
+    bool any_q = false, sums = false;
+    for (int i = 0; i < nw; ++i)
+        if (on_q16(ws[i])) any_q = true, sums = sums || ws[i]->type == kQ4K;
+    QGemmArgs qa{};
+    if (any_q) TRY(split_q16(h, A, K, cols, (int)ldx, sums, &qa));
+    const uint64_t block = std::max<uint64_t>(128, kGemmScratchBytes / ((uint64_t)cols * 4) / 128 * 128);
+    uint64_t first = 0;  // stacked index of weight i's row 0
+    for (int i = 0; i < nw;) {
+        const Weight* wt = ws[i];
+        if (on_q16(wt)) {
+            const uint32_t type = wt->type;
+            int j = i, nr = 0;
+            qa.nseg = 0;
+            while (j < nw && ws[j]->type == type) {
+                qa.w[qa.nseg] = static_cast<const uint8_t*>(ws[j]->dev);
+                qa.row0[qa.nseg++] = nr;
+                nr += (int)ws[j]->rows;
+                ++j;
+            }
+            qa.row0[qa.nseg] = nr;
+            qa.N = nr;
+            qa.y = C + first;
+            qa.ldy = (int)ldy;
+            TRY(run_gemm_q16(h, type, qa, flops_per_row * (uint64_t)nr));
+            first += (uint64_t)nr;
+            i = j;
+            continue;
+        }
+        if (!aligned || !on_gemm(h, wt, K, rows)) {
+            const int per = aligned ? small_batch(h, wt) : 1;
             for (int k0 = 0; k0 < K;) {
-                const int n = batched ? std::min(per, K - k0) : 1;
-                float* yk = reinterpret_cast<float*>(Y) + (size_t)k0 * ldy + off;
-                const float* xk = reinterpret_cast<const float*>(X) + (size_t)k0 * ldx;
+                const int n = std::min(per, K - k0);
+                float* yk = C + (size_t)k0 * ldy + first;
+                const float* xk = A + (size_t)k0 * ldx;
                 if (n > 1) {
                     MvBatchArgs b{static_cast<const uint8_t*>(wt->dev), (int)wt->rows, cols, xk, (size_t)ldx, yk,
                                   (size_t)ldy};
@@ -616,70 +698,25 @@ static emprise_status linear_batch_rows(emprise_hip* h, int nw, const Weight* co
                 }
                 k0 += n;
             }
-            off += wt->rows;
-        }
-        return EMPRISE_OK;
-    }
-    const float* A = reinterpret_cast<const float*>(X);
-    float* C = reinterpret_cast<float*>(Y);
-    const uint64_t flops_per_row = 2ull * (uint64_t)K * (uint64_t)cols;
-    if (nw == 1 && all_f32) {
-        return traced(h, "gemm_f32", flops_per_row * rows, [&] {
-            return launch_gemm_f32(A, reinterpret_cast<const float*>(ws[0]->dev), C, K, (int)rows, cols, (int)ldx,
-                                   cols, (int)ldy, h->stream);
-        });
-    }
-    // Chunked Q6_K / Q4_K weights run on the fp16 matrix cores (gemm_q.hip: exact fp16
-    // pieces of the weights and of the activations, FP32 sums), consecutive weights of one
-    // type in one launch; the others are dequantised (or copied, for F32 rows) exactly into
-    // FP32 blocks and multiplied in FP32.
-    auto on_q16 = [](const Weight* wt) { return (wt->type == kQ6K || wt->type == kQ4K) && chunked_cols(wt->cols); };
-    bool any_q = false, sums = false;
-    for (int i = 0; i < nw; ++i)
-        if (on_q16(ws[i])) any_q = true, sums = sums || ws[i]->type == kQ4K;
-    QGemmArgs qa{};
-    if (any_q) {
-        void* xs;
-        TRY(h->get_scratch("gemm_xs", gemm_q16_split_bytes(K, cols, sums), &xs));
-        TRY(traced(h, "split_f16", (uint64_t)K * cols * 8, [&] {
-            return launch_gemm_q16_split(A, K, cols, (int)ldx, xs, sums, &qa, h->stream);
-        }));
-    }
-    const uint64_t block = std::max<uint64_t>(128, kGemmScratchBytes / ((uint64_t)cols * 4) / 128 * 128);
-    uint64_t first = 0;  // stacked index of weight i's row 0
-    for (int i = 0; i < nw;) {
-        if (on_q16(ws[i])) {
-            const uint32_t type = ws[i]->type;
-            int j = i, nr = 0;
-            qa.nseg = 0;
-            while (j < nw && on_q16(ws[j]) && ws[j]->type == type) {
-                qa.w[qa.nseg] = static_cast<const uint8_t*>(ws[j]->dev);
-                qa.row0[qa.nseg++] = nr;
-                nr += (int)ws[j]->rows;
-                ++j;
+        } else if (wt->type == kF32 && nw == 1) {
+            TRY(traced(h, "gemm_f32", flops_per_row * wt->rows, [&] {
+                return launch_gemm_f32(A, reinterpret_cast<const float*>(wt->dev), C, K, (int)wt->rows, cols, (int)ldx,
+                                       cols, (int)ldy, h->stream);
+            }));
+        } else {
+            const uint64_t nb = std::min<uint64_t>(block, wt->rows);
+            void* wf;
+            TRY(h->get_scratch("gemm_w", nb * cols * sizeof(float), &wf));
+            for (uint64_t r0 = 0; r0 < wt->rows; r0 += nb) {
+                const uint64_t n = std::min<uint64_t>(nb, wt->rows - r0);
+                TRY(traced(h, "dequant_rows", n * (wt->bytes / wt->rows + (uint64_t)cols * 4), [&] {
+                    return launch_dequant_rows(wt->dev, wt->type, cols, r0, n, static_cast<float*>(wf), h->stream);
+                }));
+                TRY(traced(h, "gemm_f32", flops_per_row * n, [&] {
+                    return launch_gemm_f32(A, static_cast<const float*>(wf), C + first + r0, K, (int)n, cols, (int)ldx,
+                                           cols, (int)ldy, h->stream);
+                }));
             }
-            qa.row0[qa.nseg] = nr;
-            qa.N = nr;
-            qa.y = C + first;
-            qa.ldy = (int)ldy;
-            TRY(traced(h, "gemm_q16", flops_per_row * (uint64_t)nr, [&] { return launch_gemm_q16(type, qa, h->stream); }));
-            first += (uint64_t)nr;
-            i = j;
-            continue;
-        }
-        const Weight* wt = ws[i];
-        const uint64_t nb = std::min<uint64_t>(block, wt->rows);
-        void* wf;
-        TRY(h->get_scratch("gemm_w", nb * cols * sizeof(float), &wf));
-        for (uint64_t r0 = 0; r0 < wt->rows; r0 += nb) {
-            const uint64_t n = std::min<uint64_t>(nb, wt->rows - r0);
-            TRY(traced(h, "dequant_rows", n * (wt->bytes / wt->rows + (uint64_t)cols * 4), [&] {
-                return launch_dequant_rows(wt->dev, wt->type, cols, r0, n, static_cast<float*>(wf), h->stream);
-            }));
-            TRY(traced(h, "gemm_f32", flops_per_row * n, [&] {
-                return launch_gemm_f32(A, static_cast<const float*>(wf), C + first + r0, K, (int)n, cols, (int)ldx, cols,
-                                       (int)ldy, h->stream);
-            }));
         }
         first += wt->rows;
         ++i;
@@ -717,17 +754,11 @@ emprise_status emprise_hip_ffn_gate_up_batch(emprise_hip* h, emprise_weight gate
     if (ldx < (uint64_t)cols || ldy < (uint64_t)F || ldx > (1u << 30) || ldy > (1u << 30) || 2ull * F > (1u << 30))
         return fail(EMPRISE_EINVAL, "row strides shorter than the matrix");
     float* y = reinterpret_cast<float*>(Y);
-    // gate and up of one chunked type: one GEMM over their interleaved rows, SwiGLU in its
+    // gate and up of one quantised type: one GEMM over their interleaved rows, SwiGLU in its
     // epilogue (gemm_q.hip, QGemmArgs::pair)
-    if ((g->type == kQ6K || g->type == kQ4K) && u->type == g->type && chunked_cols(g->cols) && K >= kGemmMinBatch &&
-        cols % 16 == 0 && X % 16 == 0 && ldx % 4 == 0) {
-        const bool sums = g->type == kQ4K;
+    if ((g->type == kQ6K || g->type == kQ4K) && u->type == g->type && on_gemm(h, g, K, 2ull * F) && X % 16 == 0 && ldx % 4 == 0) {
         QGemmArgs qa{};
-        void* xs;
-        TRY(h->get_scratch("gemm_xs", gemm_q16_split_bytes(K, cols, sums), &xs));
-        TRY(traced(h, "split_f16", (uint64_t)K * cols * 8, [&] {
-            return launch_gemm_q16_split(reinterpret_cast<const float*>(X), K, cols, (int)ldx, xs, sums, &qa, h->stream);
-        }));
+        TRY(split_q16(h, reinterpret_cast<const float*>(X), K, cols, (int)ldx, g->type == kQ4K, &qa));
         qa.nseg = 2;
         qa.w[0] = static_cast<const uint8_t*>(g->dev);
         qa.w[1] = static_cast<const uint8_t*>(u->dev);
@@ -738,7 +769,7 @@ emprise_status emprise_hip_ffn_gate_up_batch(emprise_hip* h, emprise_weight gate
         qa.y = y;
         qa.ldy = (int)ldy;
         qa.pair = 1;
-        return traced(h, "gemm_q16", 4ull * K * cols * F, [&] { return launch_gemm_q16(g->type, qa, h->stream); });
+        return run_gemm_q16(h, g->type, qa, 4ull * K * cols * F);
     }
     // otherwise the two projections (gate into Y, up into scratch), then swiglu per row
     void* ub;

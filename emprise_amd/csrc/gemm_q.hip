@@ -1,6 +1,6 @@
-// Prefill projections Y = X W^T with chunked Q6_K / Q4_K weights on the fp16 matrix cores
+// Batched projections Y = X W^T with Q6_K / Q4_K weights on the fp16 matrix cores
 // (Backend::linear_batch, reference backend.hpp:20-24 / the CUDA linear_q6_f32_batch,
-// cuda.cpp:350-413), for batches of 8 tokens and more.
+// cuda.cpp:350-413), for every width and both weight layouts (layout.hpp).
 //
 // Both operands are exact in fp16 pieces, so the products are those of the FP32 path:
 //
@@ -9,31 +9,46 @@
 //   as v = vh + vl with vh = v rounded to fp16 and vl = v - vh (|vl| <= 1): both exact
 //   fp16. A Q4_K element is (d * sc) * q - dmin * m (quant.cpp:41-61); v = sc * q is at
 //   most 63 * 15 = 945, exact in fp16 as it stands. The block scales d (and dmin) of each
-//   256 columns are applied in FP32 once per block. The staging waves decode in packed
-//   fp16 arithmetic, every step exact (below).
-// - Activations. Row m of X is scaled by a power of two 2^-e_m (exact) so that its largest
-//   magnitude lies in [1, 2) -- no fp16 overflow whatever the activations -- and split
-//   into xh = fp16(x) and xl = fp16(x - xh), which carry x to 22 significant bits.
+//   256 columns are applied in FP32 once per block.
+// - Activations. Each 256-column block of a row of X is scaled by a power of two 2^-e
+//   (exact) so that its largest magnitude lies in [2^8, 2^9) -- no fp16 overflow whatever
+//   the activations, in the values or in sums of 32 of them -- and split into xh = fp16(x)
+//   and xl = fp16(x - xh), which carry x to 22 significant bits.
 //
-// Per 256-column block the matrix cores accumulate, in FP32, sum v*xh + v*xl (+ vl*xh for
-// Q6_K; the dropped vl*xl is below 2^-21 of the term) and the block adds d times that to
-// the row's FP32 accumulator; for Q4_K the min term -dmin * sum_u m_u * (sum of x over
-// unit u) is one more product per block, with the unit sums split the same way. The
-// result is scaled back by 2^e_m. Only the rounding of the FP32 sums differs from the CPU
-// path's sequential row sum.
+// Per block the matrix cores accumulate, in FP32, sum v*xh + v*xl (+ vl*xh for Q6_K; the
+// dropped vl*xl is below 2^-21 of the term) and 2^e * d times that is added to the row's
+// FP32 accumulator; for Q4_K the min term -dmin * sum_u m_u * (sum of x over unit u) is
+// one more product per block, with the unit sums split the same way.
 //
-// Tiling: a workgroup of 8 waves computes 128 tokens x 128 rows. Waves 0..3 multiply:
-// wave c owns tokens 64*(c%2) .. +63 and rows 64*(c/2) .. +63 as 2 x 2 tiles of
-// v_mfma_f32_32x32x16_f16. Waves 4..7 stage: the K loop takes 64 columns per step (a
-// quarter of a block; in the chunked layout the 64 columns of matvec lane s of a chunk)
-// from two LDS buffers, and while the multiplying waves run step s from one, the staging
-// waves decode step s+1's codes into fp16, store them with the activation pieces into the
-// other and issue the global loads of step s+3 (two register sets in turn); one barrier
-// per step.
+// The weights never pass through LDS. The MFMA operand layout asks lane l for 8 columns of
+// row l%16, and the order of the columns inside a block is free as long as both operands
+// use the same one: lane (row, q = l/16) takes columns 64q .. 64q+63 of its row's block,
+// which is what it gets from three (Q6_K) or two (Q4_K) 16-byte loads of codes, with its
+// unit scales and the row's block scale beside them, and decodes them straight into
+// operand registers in packed fp16 arithmetic, every step exact. Slice s of a block (one
+// v_mfma_f32_16x16x32_f16 deep) is columns 64q + 8s .. +7 of each q. The activation pieces
+// are stored by the split in that order, one 1 KiB operand after the other, so a step's
+// share is a few contiguous runs and every LDS access is 16 bytes per lane in lane order.
 //
-// MFMA 32x32x16 f16 operand layout (lane l): A[i][k] with i = l % 32, k = 8*(l/32) + 0..7;
-// B[k][j] with j = l % 32, the same k; D[i][j] in accumulator r with j = l % 32 and
-// i = 8*(r/4) + 4*(l/32) + r%4.
+// Three forms, by the number of tokens M (launch_type): up to 32 the weights' bytes bound
+// the product and the waves stream them on their own (gemm_q16_few_kernel); up to 64, and
+// where whole 256-row workgroups would leave CUs idle, gemm_q16_kernel; beyond that the
+// matrix cores bound it (gemm_q16_wide_kernel). Where one workgroup per (rows, tokens) does
+// not fill the chip the columns are cut into spans (gemm_q16_spans, a function of M and K
+// alone, so that a row's sums do not depend on the rows it is stacked with), each span's
+// sums a layer of scratch that gemm_q16_reduce_kernel adds up. Measured against a kernel
+// that decoded the weights into LDS for 128 x 128 tiles (chunked layout) or dequantised
+// them to FP32 (the others), graph replays over distinct weights, us, Q6_K gate+up rows
+// 24576 x 4096 and down rows 4096 x 12288: 5 tokens 34 + 26 (58 + 34 as small-batch
+// matvecs), 99 tokens 100 + 52 (the FFN 384 before, 158 now), 2048 tokens 980 + 515 (1276 +
+// 620); Q4_K 12288 x 2048 and 2048 x 6144 at 700 tokens 148 + 85 (the FFN 1151 before, 219
+// now).
+//
+// MFMA 16x16x32 f16 operand layout (lane l): A[i][k] with i = l % 16, k = 8*(l/16) + 0..7;
+// B[k][j] with j = l % 16, the same k; D[i][j] in accumulator r with j = l % 16 and
+// i = 4*(l/16) + r.
+#include <algorithm>
+
 #include "common.hpp"
 #include "kernels.hpp"
 #include "layout.hpp"
@@ -42,530 +57,910 @@ namespace emprise {
 namespace {
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-
-constexpr int QM = 128, QN = 128, QKS = 64, QROW = QKS + 8;  // LDS rows padded to 144 bytes
-constexpr int QThreads = 512;
+typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
+// rows of the unit-major layout start at any even address
+typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t u32u __attribute__((aligned(2)));
 
 // Loads through global-address-space pointers (global_load_*, counted by vmcnt only).
 #define QGLOBAL __attribute__((address_space(1)))
-typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ uint4 gld16(const void* p) {
     const u32x4v v = *(const QGLOBAL u32x4v*)p;
     return make_uint4(v.x, v.y, v.z, v.w);
 }
-__device__ __forceinline__ uint32_t gld4(const void* p) { return *(const QGLOBAL uint32_t*)p; }
+__device__ __forceinline__ uint4 gld16u(const void* p) {
+    const u32x4u v = *(const QGLOBAL u32x4u*)p;
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
+__device__ __forceinline__ uint32_t gld4u(const void* p) { return *(const QGLOBAL u32u*)p; }
 __device__ __forceinline__ uint32_t gld2(const void* p) { return *(const QGLOBAL uint16_t*)p; }
 __device__ __forceinline__ uint32_t gld1(const void* p) { return *(const QGLOBAL uint8_t*)p; }
 
-// ---- activations: fp16 hi/lo pieces of 2^-e_m * x, and (for Q4_K) of its 32-column sums ----
+constexpr int kBlk = 256;             // columns per block
+constexpr int kTileHalves = 16 * kBlk * 2;  // a 16-token tile's pieces of one block: 16 KiB
 
-// The pieces are stored tile by tile, in the order the GEMM reads them: tile (m/128,
-// k/64) is 128 x 64 halves, row-major, so a step's activation tile is one contiguous
-// 16 KiB run per piece. Rows from M up to the next multiple of 128 are zero.
-__device__ __forceinline__ size_t tiled(int m, int k, int K) {
-    return ((size_t)(m >> 7) * (K >> 6) + (k >> 6)) * (128 * 64) + (m & 127) * 64 + (k & 63);
-}
+// ---- activations: fp16 hi/lo pieces of 2^-e * x, and (for Q4_K) of its 32-column sums ----
 
-__global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict__ X, int M, int K, int ldx,
-                                                         _Float16* __restrict__ xh, _Float16* __restrict__ xl,
-                                                         int* __restrict__ rexp, _Float16* __restrict__ sh,
-                                                         _Float16* __restrict__ sl) {
-    __shared__ float red[8];
-    const int m = blockIdx.x;
-    if (m >= M) {  // padding rows of the last tile
-        for (int i = threadIdx.x; i < K; i += blockDim.x) xh[tiled(m, i, K)] = xl[tiled(m, i, K)] = (_Float16)0.f;
-        return;
-    }
-    const float* x = X + (size_t)m * ldx;
-    float mx = 0.f;
-    for (int i = threadIdx.x; i < K; i += blockDim.x) mx = fmaxf(mx, fabsf(x[i]));
-    mx = wave_max(mx);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
-    __syncthreads();
-    mx = 0.f;
-    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) mx = fmaxf(mx, red[w]);
-    int e = 0;
-    if (mx > 0.f && mx < INFINITY) {
-        (void)frexpf(mx, &e);  // mx = f * 2^e with f in [0.5, 1)
-        e -= 1;                // mx * 2^-e in [1, 2)
-    }
-    if (threadIdx.x == 0) rexp[m] = e;
-    for (int i = threadIdx.x; i < K; i += blockDim.x) {
-        const float v = ldexpf(x[i], -e);
-        const _Float16 h = (_Float16)v;
-        xh[tiled(m, i, K)] = h;
-        xl[tiled(m, i, K)] = (_Float16)(v - (float)h);
-    }
-    if (sh) {
-        const int units = K / 32;
-        for (int u = threadIdx.x; u < units; u += blockDim.x) {
-            float s = 0.f;
-            for (int k = 0; k < 32; ++k) s += ldexpf(x[u * 32 + k], -e);
-            const _Float16 h = (_Float16)s;
-            sh[(size_t)m * units + u] = h;
-            sl[(size_t)m * units + u] = (_Float16)(s - (float)h);
-        }
-    }
-}
-
-// The same split for 16-byte aligned rows of P * 2048 columns: lane t of pass p holds
-// columns 8(256p + t) .. +7 in registers from the row maximum to the stores (two 16-byte
-// loads, one 16-byte store per piece), and a Q4_K unit's 32 columns are a DPP quad: each
-// lane sums its 8 values in column order, the quad adds the pairs (s0 + s1) + (s2 + s3).
-template <int P>
-__global__ __launch_bounds__(256) void split_rows8_kernel(const float* __restrict__ X, int M, int K, int ldx,
-                                                          _Float16* __restrict__ xh, _Float16* __restrict__ xl,
-                                                          int* __restrict__ rexp, _Float16* __restrict__ sh,
-                                                          _Float16* __restrict__ sl) {
-    typedef float f4v __attribute__((ext_vector_type(4)));
-    __shared__ float red[4];
-    const int m = blockIdx.x, t = threadIdx.x;
-    if (m >= M) {  // padding rows of the last tile
-        const half8 z = {};
-#pragma unroll
-        for (int p = 0; p < P; ++p) {
-            const size_t o = tiled(m, 8 * (256 * p + t), K);
-            *reinterpret_cast<half8*>(xh + o) = z;
-            *reinterpret_cast<half8*>(xl + o) = z;
-        }
-        return;
-    }
-    const float* x = X + (size_t)m * ldx;
-    f4v v[P][2];
+// One token's 16 columns 16c .. 16c+15 of a block, by thread c of the token's 16 threads (a
+// DPP row; all 16 call): slices 2(c%4), +1 of lane group q = c/4 into the tile's operands
+// (slice s, piece p, lane l -> halves ((2s + p)*64 + l)*8 .. +7), 2^e, and with `sums` lane
+// (i, q): the hi pieces of the sums over units 2q, 2q+1 (32 columns each), then their lo
+// pieces.
+__device__ __forceinline__ void split16(const float (&v)[16], int i, int c, _Float16* xf, float* xe, _Float16* xs,
+                                        bool sums) {
+    const int q = c >> 2;
     float mx = 0.f;
 #pragma unroll
-    for (int p = 0; p < P; ++p) {
-        const f4v* src = reinterpret_cast<const f4v*>(x + 8 * (256 * p + t));
-        v[p][0] = src[0];
-        v[p][1] = src[1];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) mx = fmaxf(mx, fmaxf(fabsf(v[p][0][i]), fabsf(v[p][1][i])));
-    }
-    mx = wave_max(mx);
-    if ((t & 63) == 0) red[t >> 6] = mx;
-    __syncthreads();
-    mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    for (int k = 0; k < 16; ++k) mx = fmaxf(mx, fabsf(v[k]));
+    mx = fmaxf(mx, dpp_f<0xb1, 0xf>(mx, mx));
+    mx = fmaxf(mx, dpp_f<0x4e, 0xf>(mx, mx));
+    mx = fmaxf(mx, dpp_f<0x141, 0xf>(mx, mx));
+    mx = fmaxf(mx, dpp_f<0x140, 0xf>(mx, mx));
     int e = 0;
     if (mx > 0.f && mx < INFINITY) {
-        (void)frexpf(mx, &e);  // mx = f * 2^e with f in [0.5, 1)
-        e -= 1;                // mx * 2^-e in [1, 2)
+        (void)frexpf(mx, &e);      // mx = f * 2^e with f in [0.5, 1)
+        e = max(e - 9, -126);      // mx * 2^-e in [2^8, 2^9)
     }
-    if (t == 0) rexp[m] = e;
-    const int units = K / 32;
+    const float up = ldexpf(1.f, -e);
+    if (c == 0) xe[i] = ldexpf(1.f, e);
+    _Float16* dst = xf + (q * 16 + i) * 8;
+    float s = 0.f;
 #pragma unroll
-    for (int p = 0; p < P; ++p) {
-        half8 h8, l8;
-        float s = 0.f;
+    for (int h = 0; h < 2; ++h) {
+        half8 hi, lo;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const float w = ldexpf(v[p][i >> 2][i & 3], -e);
-            const _Float16 h = (_Float16)w;
-            h8[i] = h;
-            l8[i] = (_Float16)(w - (float)h);
+        for (int k = 0; k < 8; ++k) {
+            const float w = v[8 * h + k] * up;
+            hi[k] = (_Float16)w;
+            lo[k] = (_Float16)(w - (float)hi[k]);
             s += w;
         }
-        const size_t o = tiled(m, 8 * (256 * p + t), K);
-        *reinterpret_cast<half8*>(xh + o) = h8;
-        *reinterpret_cast<half8*>(xl + o) = l8;
-        if (sh) {
-            s += dpp_f<0xb1, 0xf>(0.f, s);  // quad_perm [1,0,3,2]: s0 + s1, s2 + s3
-            s += dpp_f<0x4e, 0xf>(0.f, s);  // quad_perm [2,3,0,1]
-            if ((t & 3) == 0) {
-                const int u = (256 * p + t) >> 2;
-                const _Float16 h = (_Float16)s;
-                sh[(size_t)m * units + u] = h;
-                sl[(size_t)m * units + u] = (_Float16)(s - (float)h);
-            }
+        const int slice = 2 * (c & 3) + h;
+        *reinterpret_cast<half8*>(dst + (2 * slice) * 512) = hi;
+        *reinterpret_cast<half8*>(dst + (2 * slice + 1) * 512) = lo;
+    }
+    if (sums) {
+        s += dpp_f<0xb1, 0xf>(0.f, s);                // the unit's two threads
+        const float s1 = dpp_f<0x4e, 0xf>(0.f, s);    // lane group q's other unit
+        if ((c & 3) == 0) {
+            const _Float16 h0 = (_Float16)s, h1 = (_Float16)s1;
+            *reinterpret_cast<half4*>(xs + (q * 16 + i) * 4) =
+                half4{h0, h1, (_Float16)(s - (float)h0), (_Float16)(s1 - (float)h1)};
         }
     }
 }
 
-// ---- the GEMM ------------------------------------------------------------------------
+// 16 columns of token m (zero past M)
+__device__ __forceinline__ void load16(float (&v)[16], const float* X, int m, int M, size_t ldx, int col) {
+    if (m < M) {
+        const floatx4* src = reinterpret_cast<const floatx4*>(X + (size_t)m * ldx + col);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const floatx4 f = src[k];
+            v[4 * k] = f.x, v[4 * k + 1] = f.y, v[4 * k + 2] = f.z, v[4 * k + 3] = f.w;
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < 16; ++k) v[k] = 0.f;
+    }
+}
 
+// Workgroup = (16-token tile, block). xe[block][token]: 2^e; xs[block][tile][lane][4].
+__global__ __launch_bounds__(256) void split_tiles_kernel(const float* __restrict__ X, int M, int ldx, int tiles,
+                                                          _Float16* __restrict__ xf, float* __restrict__ xe,
+                                                          _Float16* __restrict__ xs) {
+    const int tile = blockIdx.x, blk = blockIdx.y, t = threadIdx.x, i = t >> 4, c = t & 15;
+    float v[16];
+    load16(v, X, tile * 16 + i, M, ldx, blk * kBlk + 16 * c);
+    const size_t at = (size_t)blk * tiles + tile;
+    split16(v, i, c, xf + at * kTileHalves, xe + at * 16, xs + at * 256, xs != nullptr);
+}
+
+// ---- weights ---------------------------------------------------------------------------
+
+// A lane's share of one block of its row: columns 64q .. 64q+63.
 template <int T> struct QRaw;
 template <> struct QRaw<kQ6K> {
-    uint2 d0, d1, d2;  // words j0, j0+1 of the three code planes (units j0, j0+1)
-    uint32_t sc;       // the two units' int8 scales (low byte: unit j0)
-    uint32_t d;        // fp16 block scale (used at a block's first step)
+    uint32_t w[3][4];  // word p of unit 4q+j in w[p][j]
+    uint32_t sc;       // the four units' int8 scales
+    uint32_t d;        // fp16 block scale
 };
 template <> struct QRaw<kQ4K> {
-    uint4 q;      // the unit's 32 nibbles
-    uint32_t s2;  // the lane's two scale bytes (low: unit 0)
-    uint32_t m4;  // the lane's min nibbles (low: unit 0)
-    uint32_t dd;  // fp16 d | fp16 dmin << 16
+    uint32_t w[2][4];  // the 32 nibbles of units 2q and 2q+1
+    uint32_t sm[3];    // chunked: scale bytes, min nibbles; unit-major: three pairs of the 12 packed bytes
+    uint32_t dd;       // fp16 d | fp16 dmin << 16
 };
 
-typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+template <bool CH> __device__ __forceinline__ void q_load(QRaw<kQ6K>& r, const uint8_t* row, int nb, int b, int q) {
+    if constexpr (CH) {
+        const uint8_t* base = row + (size_t)(b >> 4) * 3360;
+        const int l = 4 * (b & 15) + q;
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+            const uint4 v = gld16(base + p * 1024 + 16 * l);
+            r.w[p][0] = v.x, r.w[p][1] = v.y, r.w[p][2] = v.z, r.w[p][3] = v.w;
+        }
+        r.sc = gld4u(base + 3072 + 4 * l);
+        r.d = gld2(base + 3328 + 2 * (b & 15));
+    } else {
+        const uint8_t* base = row + (size_t)b * 192 + 48 * q;
+        uint32_t x[12];
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+            const uint4 v = gld16u(base + 16 * p);
+            x[4 * p] = v.x, x[4 * p + 1] = v.y, x[4 * p + 2] = v.z, x[4 * p + 3] = v.w;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int p = 0; p < 3; ++p) r.w[p][j] = x[3 * j + p];
+        r.sc = gld4u(row + (size_t)nb * 192 + 16 * b + 4 * q);
+        r.d = gld2(row + (size_t)nb * 208 + 2 * b);
+    }
+}
+
+template <bool CH> __device__ __forceinline__ void q_load(QRaw<kQ4K>& r, const uint8_t* row, int nb, int b, int q) {
+    const uint8_t *c0, *c1, *s;
+    if constexpr (CH) {
+        const uint8_t* base = row + (size_t)(b >> 4) * 2304;
+        c0 = base + 16 * (4 * (b & 15) + q);
+        c1 = c0 + 1024;
+        s = base + 2048 + 12 * (b & 15);
+        r.sm[0] = gld2(s + 2 * q);
+        r.sm[1] = gld1(s + 8 + q);
+        r.sm[2] = 0;
+        r.dd = gld4u(base + 2240 + 4 * (b & 15));
+    } else {
+        c0 = row + (size_t)b * 128 + 32 * q;
+        c1 = c0 + 16;
+        s = row + (size_t)nb * 128 + 12 * b;
+        r.sm[0] = gld2(s + 2 * q);
+        r.sm[1] = gld2(s + 2 * q + 4);
+        r.sm[2] = gld2(s + 2 * max(q - 2, 0));
+        r.dd = gld4u(row + (size_t)nb * 140 + 4 * b);
+    }
+    const uint4 v0 = gld16(c0), v1 = gld16(c1);
+    r.w[0][0] = v0.x, r.w[0][1] = v0.y, r.w[0][2] = v0.z, r.w[0][3] = v0.w;
+    r.w[1][0] = v1.x, r.w[1][1] = v1.y, r.w[1][2] = v1.z, r.w[1][3] = v1.w;
+}
+
+// The scale and min of units 2q (p = 0) and 2q+1 (p = 1) of a block (quant.cpp:48-52).
+template <bool CH> __device__ __forceinline__ void q4_sm(const QRaw<kQ4K>& r, int q, int p, uint32_t& sc, uint32_t& mn) {
+    if constexpr (CH) {
+        const uint32_t b = (r.sm[0] >> (8 * p)) & 0xffu;
+        sc = b & 63u;
+        mn = ((b >> 6) << 4) | ((r.sm[1] >> (4 * p)) & 15u);
+    } else {
+        const uint32_t a = (r.sm[0] >> (8 * p)) & 0xffu, b = (r.sm[1] >> (8 * p)) & 0xffu, c = (r.sm[2] >> (8 * p)) & 0xffu;
+        sc = q < 2 ? (a & 63u) : ((b & 15u) | ((c >> 6) << 4));
+        mn = q < 2 ? (b & 63u) : ((b >> 4) | ((a >> 6) << 4));
+    }
+}
 
 // Two code bytes (bytes 0, 1 of w, or 2, 3 with hi) as the fp16 pair 1024 + q: each byte
 // under an exponent byte 0x64 (v_perm_b32), which makes 1024 + q exact for q < 1024.
 __device__ __forceinline__ half2v codes_1024(uint32_t w, bool hi) {
     return __builtin_bit_cast(half2v, __builtin_amdgcn_perm(0x64646464u, w, hi ? 0x04030402u : 0x04010400u));
 }
-
-// Q6_K unit -> fp16 pieces: codes 0..3 in the low 6 bits of word d0, 4..7 of d1, 8..11 of
-// d2, 12..15 gathered from their top two bits. In packed fp16 arithmetic, each step exact:
-// q - 32 = (1024 + q) - 1056; vh = fp16(v), v = sc * (q - 32); vl = fma(q - 32, sc, -vh),
-// a small integer (|vl| <= 1). Two weights per instruction, about half the instructions
-// of the same split in FP32.
-__device__ __forceinline__ void q6_unit_f16(uint32_t d0, uint32_t d1, uint32_t d2, int sc, _Float16* dh,
-                                            _Float16* dl) {
-    const uint32_t w[4] = {d0 & 0x3F3F3F3Fu, d1 & 0x3F3F3F3Fu, d2 & 0x3F3F3F3Fu,
-                           ((d0 >> 6) & 0x03030303u) | ((d1 >> 4) & 0x0C0C0C0Cu) | ((d2 >> 2) & 0x30303030u)};
-    const _Float16 s16 = (_Float16)(float)sc;
-    const half2v sc2 = {s16, s16}, off = {(_Float16)-1056.f, (_Float16)-1056.f};
-    uint32_t hi[8], lo[8];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const half2v q = codes_1024(w[k], h) + off;
-            const half2v vh = q * sc2;
-            const half2v vl = __builtin_elementwise_fma(q, sc2, -vh);
-            hi[2 * k + h] = __builtin_bit_cast(uint32_t, vh);
-            lo[2 * k + h] = __builtin_bit_cast(uint32_t, vl);
-        }
-    }
-    *reinterpret_cast<uint4*>(dh) = make_uint4(hi[0], hi[1], hi[2], hi[3]);
-    *reinterpret_cast<uint4*>(dh + 8) = make_uint4(hi[4], hi[5], hi[6], hi[7]);
-    *reinterpret_cast<uint4*>(dl) = make_uint4(lo[0], lo[1], lo[2], lo[3]);
-    *reinterpret_cast<uint4*>(dl + 8) = make_uint4(lo[4], lo[5], lo[6], lo[7]);
+__device__ __forceinline__ half8 pack8(const uint32_t (&w)[4]) {
+    return __builtin_bit_cast(half8, u32x4v{w[0], w[1], w[2], w[3]});
 }
 
-// Waves 0..3 multiply, waves 4..7 stage: with two LDS buffers and one barrier per step, the
-// staging waves decode and store step s+1 (and load step s+2) while the multiplying waves
-// run step s, so the weight decode, the LDS traffic and the matrix cores overlap.
-template <int T>
-__global__ __launch_bounds__(QThreads) void gemm_q16_kernel(QGemmArgs a) {
-    constexpr int NB = T == kQ6K ? 2 : 1;   // weight pieces
-    constexpr int NQ = T == kQ4K ? QN : 1;  // Q4_K-only arrays
-    // step s is read from buffer s%2 while step s+1 is stored into the other; the block
-    // scales and Q4_K mins by block parity
-    __shared__ __align__(16) _Float16 As[2][2][QM][QROW];
-    __shared__ __align__(16) _Float16 Bs[2][NB][QN][QROW];
-    __shared__ float ds[2][QN], dms[2][NQ];
-    __shared__ __align__(16) _Float16 Ms[2][NQ][8];  // Q4_K: -m of the block's 8 units
-
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int m0 = blockIdx.y * QM, n0 = blockIdx.x * QN;
-    const int steps = a.K / QKS, cpr = a.K / kChunkCols;
-    const bool stager = wave >= 4;
-
-    if (stager) {
-        // ---- staging waves: thread pt loads and stores four 16-byte pieces of each
-        // activation tile, and weight row pr, units 2*(pt%2), +1 (Q6_K) or unit pt%2 (Q4_K,
-        // both halves)
-        const int pt = threadIdx.x - 256, pr = pt >> 1, ph = pt & 1;
-        const size_t abase = (size_t)blockIdx.y * steps * (QM * QKS);  // the tile row's first step
-        const int bn = n0 + pr;
-        const bool b_ok = bn < a.N;
-        const uint8_t* brow;  // (rows past N read row 0 and are zeroed)
-        {
-            const int r = b_ok ? bn : 0;
-            constexpr size_t kChunk = T == kQ6K ? 3360 : 2304;
-            if (a.pair) {
-                brow = a.w[r & 1] + (size_t)(r >> 1) * cpr * kChunk;
-            } else {
-                int sg = 0;
-                while (sg + 1 < a.nseg && r >= a.row0[sg + 1]) ++sg;
-                brow = a.w[sg] + (size_t)(r - a.row0[sg]) * cpr * kChunk;
-            }
+// The 16 columns of unit step j (64q + 16j .. +15) as two slices of operand registers.
+// Q6_K: codes 0..3 in the low 6 bits of word 0, 4..7 of word 1, 8..11 of word 2, 12..15
+// gathered from their top two bits; in packed fp16, each step exact: q - 32 = (1024 + q) -
+// 1056; vh = fp16(v), v = sc * (q - 32); vl = fma(q - 32, sc, -vh), a small integer.
+__device__ __forceinline__ void q6_unit(const QRaw<kQ6K>& r, int j, half8 (&hi)[2], half8 (&lo)[2]) {
+    const uint32_t d0 = r.w[0][j], d1 = r.w[1][j], d2 = r.w[2][j];
+    const uint32_t w[4] = {d0 & 0x3F3F3F3Fu, d1 & 0x3F3F3F3Fu, d2 & 0x3F3F3F3Fu,
+                           ((d0 >> 6) & 0x03030303u) | ((d1 >> 4) & 0x0C0C0C0Cu) | ((d2 >> 2) & 0x30303030u)};
+    const _Float16 s16 = (_Float16)(float)(int)(int8_t)(r.sc >> (8 * j));
+    const half2v sc2 = {s16, s16}, off = {(_Float16)-1056.f, (_Float16)-1056.f};
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        uint32_t ph[4], pl[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const half2v c = codes_1024(w[2 * h + (k >> 1)], k & 1) + off;
+            const half2v vh = c * sc2;
+            const half2v vl = __builtin_elementwise_fma(c, sc2, -vh);
+            ph[k] = __builtin_bit_cast(uint32_t, vh);
+            pl[k] = __builtin_bit_cast(uint32_t, vl);
         }
-        // two register sets in turn (step k in set k%2): the loads of step k go out two
-        // steps before it is stored; every load is issued whatever the step (past the last
-        // step it re-reads the last one), so the waits for a set never cover the other's
-        struct Regs {
-            uint4 rh[4], rl[4];
-            QRaw<T> rb;
-        } R0, R1;
-        auto load_step = [&](int s, Regs& R) {
-            uint4* rh = R.rh;
-            uint4* rl = R.rl;
-            QRaw<T>& rb = R.rb;
-            s = min(s, steps - 1);
-            const int k0 = s * QKS;
-            // the step's 128 x 64 tile of each piece: 16 KiB in a row, 16 bytes per thread
-            // and load, a wave's load 1 KiB in a row
-            const size_t at = abase + (size_t)s * (QM * QKS);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                rh[i] = gld16(a.xh + at + 8 * (i * 256 + pt));
-                rl[i] = gld16(a.xl + at + 8 * (i * 256 + pt));
-            }
-            const int c = k0 / kChunkCols, ls = (k0 % kChunkCols) / QKS;  // chunk, matvec lane
-            if constexpr (T == kQ6K) {
-                const uint8_t* base = brow + (size_t)c * 3360 + 16 * ls + 8 * ph;
-                const uint32_t x0 = gld4(base), x1 = gld4(base + 4);
-                const uint32_t y0 = gld4(base + 1024), y1 = gld4(base + 1028);
-                const uint32_t z0 = gld4(base + 2048), z1 = gld4(base + 2052);
-                rb.d0 = make_uint2(x0, x1);
-                rb.d1 = make_uint2(y0, y1);
-                rb.d2 = make_uint2(z0, z1);
-                rb.sc = gld2(brow + (size_t)c * 3360 + 3072 + 4 * ls + 2 * ph);
-                rb.d = gld2(brow + (size_t)c * 3360 + 3328 + 2 * (ls >> 2));
-                if (!b_ok) rb = {make_uint2(0, 0), make_uint2(0, 0), make_uint2(0, 0), 0u, 0u};
-            } else {
-                const uint8_t* base = brow + (size_t)c * 2304;
-                rb.q = gld16(base + 1024 * ph + 16 * ls);
-                const uint8_t* sb = base + 2048 + 12 * (ls >> 2);
-                rb.s2 = gld2(sb + 2 * (ls & 3));
-                rb.m4 = gld1(sb + 8 + (ls & 3));
-                rb.dd = gld4(base + 2240 + 4 * (ls >> 2));
-                if (!b_ok) {
-                    rb.q = make_uint4(0, 0, 0, 0);
-                    rb.s2 = rb.m4 = rb.dd = 0u;
-                }
-            }
-        };
-        // registers -> LDS buffer `buf`: the activation pieces as they are, the weights
-        // decoded to fp16
-        auto store_step = [&](int s, int buf, const Regs& R) {
-            const uint4* rh = R.rh;
-            const uint4* rl = R.rl;
-            const QRaw<T>& rb = R.rb;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int e = i * 256 + pt;  // 16-byte piece e: row e/8, columns 8*(e%8) ..
-                *reinterpret_cast<uint4*>(&As[buf][0][e >> 3][8 * (e & 7)]) = rh[i];
-                *reinterpret_cast<uint4*>(&As[buf][1][e >> 3][8 * (e & 7)]) = rl[i];
-            }
-            const bool block_start = (s & 3) == 0;
-            const int bp = (s >> 2) & 1;
-            if constexpr (T == kQ6K) {
-#pragma unroll
-                for (int u = 0; u < 2; ++u) {
-                    const int j = 2 * ph + u;
-                    q6_unit_f16(u ? rb.d0.y : rb.d0.x, u ? rb.d1.y : rb.d1.x, u ? rb.d2.y : rb.d2.x,
-                                (int)(int8_t)(rb.sc >> (8 * u)), &Bs[buf][0][pr][16 * j], &Bs[buf][NB - 1][pr][16 * j]);
-                }
-                if (block_start && ph == 0) ds[bp][pr] = half_bits_to_float((uint16_t)rb.d);
-            } else {
-                // unit p = ph of the step: codes 0..15 in the low nibbles of its four words,
-                // 16..31 in the high ones
-                const uint32_t b = (rb.s2 >> (8 * ph)) & 0xffu;
-                const float scf = (float)(b & 63u);
-                const uint32_t wv[4] = {rb.q.x, rb.q.y, rb.q.z, rb.q.w};
-                // v = (1024 + q) * sc - 1024 * sc in one fused step: exact, the product below
-                // 1039 * 63 < 65504 and the result at most 945
-                const _Float16 s16 = (_Float16)scf;
-                const half2v sc2 = {s16, s16}, base = {(_Float16)(-1024.f * scf), (_Float16)(-1024.f * scf)};
-#pragma unroll
-                for (int hf = 0; hf < 2; ++hf) {
-                    uint32_t pk[8];
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) {
-                        const uint32_t nib = (wv[k] >> (4 * hf)) & 0x0F0F0F0Fu;
-#pragma unroll
-                        for (int h = 0; h < 2; ++h)
-                            pk[2 * k + h] = __builtin_bit_cast(
-                                uint32_t, __builtin_elementwise_fma(codes_1024(nib, h), sc2, base));
-                    }
-                    _Float16* dh = &Bs[buf][0][pr][32 * ph + 16 * hf];
-                    *reinterpret_cast<uint4*>(dh) = make_uint4(pk[0], pk[1], pk[2], pk[3]);
-                    *reinterpret_cast<uint4*>(dh + 8) = make_uint4(pk[4], pk[5], pk[6], pk[7]);
-                }
-                const uint32_t mn = ((b >> 6) << 4) | ((rb.m4 >> (4 * ph)) & 15u);
-                Ms[bp][pr % NQ][2 * (s & 3) + ph] = (_Float16)(-(float)mn);
-                if (block_start && ph == 0) {
-                    ds[bp][pr] = half_bits_to_float((uint16_t)(rb.dd & 0xffffu));
-                    dms[bp][pr % NQ] = half_bits_to_float((uint16_t)(rb.dd >> 16));
-                }
-            }
-        };
-        // (steps is even: K is a multiple of 4096)
-        load_step(0, R0);
-        load_step(1, R1);
-        store_step(0, 0, R0);
-        load_step(2, R0);
-        __syncthreads();
-        for (int s = 0; s < steps; s += 2) {
-            if (s + 1 < steps) store_step(s + 1, 1, R1);
-            load_step(s + 3, R1);
-            __syncthreads();
-            if (s + 2 < steps) store_step(s + 2, 0, R0);
-            load_step(s + 4, R0);
-            __syncthreads();
-        }
-        return;
+        hi[h] = pack8(ph);
+        lo[h] = pack8(pl);
     }
+}
 
-    // ---- multiplying waves: wave c owns tokens 64*(c%2) .. +63 and rows 64*(c/2) .. +63
-    // as 2 x 2 tiles of 32 x 32
-    const int wm = (wave & 1) * 64, wn = (wave >> 1) * 64;
-    const int fr = lane & 31, fk = 8 * (lane >> 5);  // fragment row/column and k offset
-    floatx16 acc[2][2], cb[2][2];
+// Q4_K: the low (j even) or high nibbles of unit 2q + j/2; v = (1024 + q) * sc - 1024 * sc
+// in one fused step, exact: the product is below 1039 * 63 < 65504, the result at most 945.
+template <bool CH> __device__ __forceinline__ void q4_unit(const QRaw<kQ4K>& r, int q, int j, half8 (&hi)[2]) {
+    uint32_t sc, mn;
+    q4_sm<CH>(r, q, j >> 1, sc, mn);
+    const float scf = (float)sc;
+    const _Float16 s16 = (_Float16)scf, b16 = (_Float16)(-1024.f * scf);
+    const half2v sc2 = {s16, s16}, base = {b16, b16};
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int h = 0; h < 2; ++h) {
+        uint32_t ph[4];
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = cb[i][j][r] = 0.f;
-    half8 sh8[2] = {}, sl8[2] = {};  // Q4_K: the block's unit sums (lanes 0..31; 32..63 zero)
-    __syncthreads();
-    for (int s = 0; s < steps; ++s) {
-        const int buf = s & 1;
-        if (T == kQ4K && (s & 3) == 0) {
-#pragma unroll
-            for (int mb = 0; mb < 2; ++mb) {
-                const int m = m0 + wm + 32 * mb + fr, blk = s >> 2;
-                const bool ok = lane < 32 && m < a.M;
-                const size_t o = (size_t)(m < a.M ? m : 0) * (a.K / 32) + 8 * blk;
-                uint4 hv = gld16(a.sh + o), lv = gld16(a.sl + o);
-                if (!ok) hv = lv = make_uint4(0, 0, 0, 0);
-                sh8[mb] = __builtin_bit_cast(half8, hv);
-                sl8[mb] = __builtin_bit_cast(half8, lv);
-            }
+        for (int k = 0; k < 4; ++k) {
+            const uint32_t nib = (r.w[j >> 1][2 * h + (k >> 1)] >> (4 * (j & 1))) & 0x0F0F0F0Fu;
+            ph[k] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(codes_1024(nib, k & 1), sc2, base));
         }
-        // fragments of 16-column slice q, read one slice ahead of its products; the products
-        // go out piece by piece over the four tiles, so consecutive MFMAs never depend on
-        // each other
-        half8 fx[2][2][2], fw[2][2][NB];  // [slice parity][tile][piece]
-        auto frags = [&](int q, int f) {
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                fx[f][i][0] = *reinterpret_cast<const half8*>(&As[buf][0][wm + 32 * i + fr][16 * q + fk]);
-                fx[f][i][1] = *reinterpret_cast<const half8*>(&As[buf][1][wm + 32 * i + fr][16 * q + fk]);
-#pragma unroll
-                for (int pc = 0; pc < NB; ++pc)
-                    fw[f][i][pc] = *reinterpret_cast<const half8*>(&Bs[buf][pc][wn + 32 * i + fr][16 * q + fk]);
-            }
-        };
-        frags(0, 0);
-#pragma unroll
-        for (int q = 0; q < QKS / 16; ++q) {
-            const int f = q & 1;
-            if (q + 1 < QKS / 16) frags(q + 1, f ^ 1);
-#pragma unroll
-            for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-                for (int nb = 0; nb < 2; ++nb)
-                    cb[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fx[f][mb][0], fw[f][nb][0], cb[mb][nb], 0, 0, 0);
-#pragma unroll
-            for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-                for (int nb = 0; nb < 2; ++nb)
-                    cb[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fx[f][mb][1], fw[f][nb][0], cb[mb][nb], 0, 0, 0);
-            if constexpr (T == kQ6K) {
-#pragma unroll
-                for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-                    for (int nb = 0; nb < 2; ++nb)
-                        cb[mb][nb] =
-                            __builtin_amdgcn_mfma_f32_32x32x16_f16(fx[f][mb][0], fw[f][nb][NB - 1], cb[mb][nb], 0, 0, 0);
-            }
-        }
-        if ((s & 3) == 3) {
-            // block end: acc += d * (block products); Q4_K also adds -dmin * sum_u m_u * xsum_u
-            const int bp = (s >> 2) & 1;
-#pragma unroll
-            for (int nb = 0; nb < 2; ++nb) {
-                const int n = wn + 32 * nb + fr;
-                const float d = ds[bp][n];
-                half8 mv = {};
-                float dm = 0.f;
-                if constexpr (T == kQ4K) {
-                    uint4 mr = *reinterpret_cast<const uint4*>(&Ms[bp][n % NQ][0]);
-                    if (lane >= 32) mr = make_uint4(0, 0, 0, 0);
-                    mv = __builtin_bit_cast(half8, mr);
-                    dm = dms[bp][n % NQ];
-                }
-#pragma unroll
-                for (int mb = 0; mb < 2; ++mb) {
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        acc[mb][nb][r] = fmaf(d, cb[mb][nb][r], acc[mb][nb][r]);
-                        cb[mb][nb][r] = 0.f;
-                    }
-                    if constexpr (T == kQ4K) {
-                        floatx16 cm = {};
-                        cm = __builtin_amdgcn_mfma_f32_32x32x16_f16(sh8[mb], mv, cm, 0, 0, 0);
-                        cm = __builtin_amdgcn_mfma_f32_32x32x16_f16(sl8[mb], mv, cm, 0, 0, 0);
-#pragma unroll
-                        for (int r = 0; r < 16; ++r) acc[mb][nb][r] = fmaf(dm, cm[r], acc[mb][nb][r]);
-                    }
-                }
-            }
-        }
-        __syncthreads();
+        hi[h] = pack8(ph);
     }
+}
 
-    // Y[m][n] = 2^e_m * acc. SwiGLU pairs: the gate (even n) and up (odd n) of one output sit
-    // in adjacent lanes; of accumulators r, r+1 (rows m, m+1) the even lane writes row m and
-    // the odd lane row m+1, each receiving the one value it lacks through a lane swap, so
-    // every lane evaluates one silu(gate) * up (swiglu_kernel's form) per two entries.
-    const bool odd = fr & 1;
+// ---- the GEMM ------------------------------------------------------------------------
+
+// Row r of the stacked weights.
+template <int T> __device__ __forceinline__ const uint8_t* q_row(const QGemmArgs& a, int r, int nb) {
+    const size_t row_bytes = (size_t)nb * (T == kQ6K ? 210 : 144);
+    if (a.pair) return a.w[r & 1] + (size_t)(r >> 1) * row_bytes;
+    int sg = 0;
+    while (sg + 1 < a.nseg && r >= a.row0[sg + 1]) ++sg;
+    return a.w[sg] + (size_t)(r - a.row0[sg]) * row_bytes;
+}
+
+// 16-byte piece v of block b's side data for mt token tiles from t0: 2^e, then the unit sums.
+__device__ __forceinline__ uint4 q_side(const QGemmArgs& a, int tiles, int t0, int b, int v, int mt) {
+    if (v < 4 * mt) return gld16(a.xe + ((size_t)b * tiles + min(t0 + (v >> 2), tiles - 1)) * 16 + 4 * (v & 3));
+    const int u = v - 4 * mt;
+    return gld16(a.xs + ((size_t)b * tiles + min(t0 + (u >> 5), tiles - 1)) * 256 + 8 * (u & 31));
+}
+
+// The block scales, and the Q4_K mins as a packed fp16 pair, kept past the raw words.
+template <bool CH> __device__ __forceinline__ void q_block_scales(const QRaw<kQ6K>& r, int, uint32_t& d, uint32_t&) { d = r.d; }
+template <bool CH> __device__ __forceinline__ void q_block_scales(const QRaw<kQ4K>& r, int q, uint32_t& d, uint32_t& mins) {
+    uint32_t sc, m0, m1;
+    q4_sm<CH>(r, q, 0, sc, m0);
+    q4_sm<CH>(r, q, 1, sc, m1);
+    d = r.dd;
+    mins = __builtin_bit_cast(uint32_t, half2v{(_Float16)(-(float)m0), (_Float16)(-(float)m1)});
+}
+
+// Block end: acc += 2^e * (d * block products (- dmin * sum_u m_u * xsum_u)), products cleared.
+// (2^e last: d * 2^e alone could overflow.)
+template <int T, int RT, int MT>
+__device__ __forceinline__ void q_block_end(const uint4* side, int lane, const uint32_t (&dblk)[RT],
+                                            const uint32_t (&mins)[RT], floatx4 (&cb)[RT][MT], floatx4 (&acc)[RT][MT]) {
+    const float4* E = reinterpret_cast<const float4*>(side);
 #pragma unroll
-    for (int mb = 0; mb < 2; ++mb)
+    for (int m = 0; m < MT; ++m) {
+        if (MT * RT == 16 && m % 2 == 0) __builtin_amdgcn_sched_barrier(0);  // (registers: no further ahead)
+        const float4 e4 = E[4 * m + (lane >> 4)];
+        const float ev[4] = {e4.x, e4.y, e4.z, e4.w};
+        half8 xsum = {};
+        if constexpr (T == kQ4K) {
+            const half4 p = reinterpret_cast<const half4*>(side + 4 * MT)[m * 64 + lane];
+            xsum = half8{p[0], p[1], p[2], p[3], (_Float16)0.f, (_Float16)0.f, (_Float16)0.f, (_Float16)0.f};
+        }
 #pragma unroll
-        for (int nb = 0; nb < 2; ++nb) {
-            const int n = n0 + wn + 32 * nb + fr;
+        for (int i = 0; i < RT; ++i) {
+            const float d = half_bits_to_float((uint16_t)(dblk[i] & 0xffffu));
+            floatx4 cm = {0.f, 0.f, 0.f, 0.f};
+            float dm = 0.f;
+            if constexpr (T == kQ4K) {
+                const half2v mm = __builtin_bit_cast(half2v, mins[i]);
+                const half8 mv = {mm[0], mm[1], mm[0], mm[1], (_Float16)0.f, (_Float16)0.f, (_Float16)0.f, (_Float16)0.f};
+                cm = __builtin_amdgcn_mfma_f32_16x16x32_f16(xsum, mv, cm, 0, 0, 0);
+                dm = half_bits_to_float((uint16_t)(dblk[i] >> 16));
+            }
 #pragma unroll
-            for (int r = 0; r < 16; r += 2) {
-                const int m = m0 + wm + 32 * mb + 8 * (r / 4) + 4 * (lane >> 5) + (r % 4);
-                const float v0 = ldexpf(acc[mb][nb][r], a.rexp[min(m, a.M - 1)]);
-                const float v1 = ldexpf(acc[mb][nb][r + 1], a.rexp[min(m + 1, a.M - 1)]);
-                if (a.pair) {
+            for (int r = 0; r < 4; ++r) {
+                float t = d * cb[i][m][r];
+                if constexpr (T == kQ4K) t = fmaf(dm, cm[r], t);
+                acc[i][m][r] = fmaf(t, ev[r], acc[i][m][r]);
+            }
+            cb[i][m] = floatx4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+}
+
+// The products of slice h with token tiles m .. m+MP-1.
+template <int T, int RT, int MP, int MT>
+__device__ __forceinline__ void q_products(const half8 (&xh)[MP], const half8 (&xl)[MP], const half8 (&wh)[RT][2],
+                                           const half8 (&wl)[RT][2], int h, int m, floatx4 (&cb)[RT][MT]) {
+#pragma unroll
+    for (int u = 0; u < MP; ++u)
+#pragma unroll
+        for (int i = 0; i < RT; ++i)
+            cb[i][m + u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[u], wh[i][h], cb[i][m + u], 0, 0, 0);
+    if constexpr (T == kQ6K) {
+#pragma unroll
+        for (int u = 0; u < MP; ++u)
+#pragma unroll
+            for (int i = 0; i < RT; ++i)
+                cb[i][m + u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[u], wl[i][h], cb[i][m + u], 0, 0, 0);
+    }
+#pragma unroll
+    for (int u = 0; u < MP; ++u)
+#pragma unroll
+        for (int i = 0; i < RT; ++i)
+            cb[i][m + u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl[u], wh[i][h], cb[i][m + u], 0, 0, 0);
+}
+
+// A span's sums go to part[z][m][n]; with one layer, Y[m][n] directly. SwiGLU pairs: the
+// gate (even n) and up (odd n) of one output sit in adjacent lanes; of accumulators r, r+1
+// (rows m, m+1) the even lane writes row m and the odd lane row m+1, each receiving the one
+// value it lacks through a lane swap, so every lane evaluates one silu(gate) * up
+// (swiglu_kernel's form) per two entries.
+template <int RT, int MT>
+__device__ __forceinline__ void q_store(const QGemmArgs& a, int n0, int t0, int rj, int q, const floatx4 (&acc)[RT][MT]) {
+    const bool odd = rj & 1;
+    float* part = gridDim.z > 1 ? a.part + (size_t)blockIdx.z * a.M * a.N : nullptr;
+#pragma unroll
+    for (int i = 0; i < RT; ++i) {
+        const int n = n0 + 16 * i + rj;
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            const int row_m = (t0 + m) * 16 + 4 * q;
+#pragma unroll
+            for (int r = 0; r < 4; r += 2) {
+                const float v0 = acc[i][m][r], v1 = acc[i][m][r + 1];
+                const int mr = row_m + r;
+                if (part) {
+                    if (n < a.N) {
+                        if (mr < a.M) part[(size_t)mr * a.N + n] = v0;
+                        if (mr + 1 < a.M) part[(size_t)(mr + 1) * a.N + n] = v1;
+                    }
+                } else if (a.pair) {
                     const float recv = dpp_f<0xb1, 0xf>(0.f, odd ? v0 : v1);  // quad_perm [1,0,3,2]
                     const float gate = odd ? recv : v0, up = odd ? v1 : recv;
-                    const int mo = odd ? m + 1 : m;
+                    const int mo = odd ? mr + 1 : mr;
                     if (mo < a.M && n < a.N) a.y[(size_t)mo * a.ldy + (n >> 1)] = siluf_(gate) * up;
                 } else if (n < a.N) {
-                    if (m < a.M) a.y[(size_t)m * a.ldy + n] = v0;
-                    if (m + 1 < a.M) a.y[(size_t)(m + 1) * a.ldy + n] = v1;
+                    if (mr < a.M) a.y[(size_t)mr * a.ldy + n] = v0;
+                    if (mr + 1 < a.M) a.y[(size_t)(mr + 1) * a.ldy + n] = v1;
                 }
             }
         }
+    }
+}
+
+// The general form. A workgroup of WV waves covers WV*16*RT weight rows x 16*MT tokens; all
+// waves share the token operands, double-buffered in LDS UPS units (16 columns per lane) at
+// a time, one barrier per step; a wave decodes each weight once for its 16*MT tokens.
+// T: weight type; CH: chunked layout; MT: 16-token tiles and RT: 16-row tiles per wave; WV:
+// waves per workgroup; UPS: unit steps per LDS step; PF: the next block's weights are
+// loaded a whole block ahead (a second register set) instead of during the block's last
+// unit step. Grid: x = row groups, y = token groups, z = column spans. a.spans > 1 with one
+// z layer runs the spans one after the other, adding them in the order the reduction
+// would, so the results do not depend on which of the two forms ran.
+template <int T, bool CH, int MT, int RT, int WV, int UPS, bool PF, int OCC>
+__global__ __launch_bounds__(WV * 64, OCC) void gemm_q16_kernel(QGemmArgs a) {
+    constexpr int TH = WV * 64;                         // threads
+    constexpr int SPB = 4 / UPS;                        // steps per block
+    constexpr int AV = MT * UPS * 4096 / 16;            // 16-byte pieces of a step's operands
+    constexpr int AN = (AV + TH - 1) / TH;
+    constexpr int SV = MT * (T == kQ4K ? 36 : 4);       // of a block's side data: 2^e, then the unit sums
+    constexpr int SN = (SV + TH - 1) / TH;
+    constexpr int MP = MT >= 4 && RT == 1 ? 4 : MT >= 2 ? 2 : 1;
+    __shared__ __align__(16) uint4 As[2][AV];
+    __shared__ __align__(16) uint4 Ss[2][SV];
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int q = lane >> 4, rj = lane & 15;
+    const int tiles = (a.M + 15) >> 4, nb = a.K / kBlk;
+    const int t0 = blockIdx.y * MT, n0 = (blockIdx.x * WV + wave) * (16 * RT);
+    const int b0 = gridDim.z > 1 ? blockIdx.z * a.span : 0;
+    const int b1 = gridDim.z > 1 ? min(b0 + a.span, nb) : nb;
+
+    const uint8_t* row[RT];  // (rows past N read the last row; their results are not stored)
+#pragma unroll
+    for (int i = 0; i < RT; ++i) row[i] = q_row<T>(a, min(n0 + 16 * i + rj, a.N - 1), nb);
+
+    // step s (global numbering: block s / SPB, unit steps UPS * (s % SPB) ..)
+    uint4 ra[AN], rs[SN];
+    auto load_a = [&](int s) {
+        const int b = s / SPB, j = s - b * SPB;
+#pragma unroll
+        for (int k = 0; k < AN; ++k) {
+            const int v = min(k * TH + tid, AV - 1), tile = v / (UPS * 256), o = v - tile * (UPS * 256);
+            ra[k] = gld16(a.xf + ((size_t)b * tiles + min(t0 + tile, tiles - 1)) * kTileHalves + (size_t)(j * UPS * 256 + o) * 8);
+        }
+        if (j == 0) {
+#pragma unroll
+            for (int k = 0; k < SN; ++k) rs[k] = q_side(a, tiles, t0, b, min(k * TH + tid, SV - 1), MT);
+        }
+    };
+    auto store_a = [&](int s, int buf) {
+        const int b = s / SPB, j = s - b * SPB;
+#pragma unroll
+        for (int k = 0; k < AN; ++k) {
+            const int v = k * TH + tid;
+            if (AV % TH == 0 || v < AV) As[buf][v] = ra[k];
+        }
+        if (j == 0) {
+#pragma unroll
+            for (int k = 0; k < SN; ++k) {
+                const int v = k * TH + tid;
+                if (v < SV) Ss[b & 1][v] = rs[k];
+            }
+        }
+    };
+
+    floatx4 cb[RT][MT], acc[RT][MT], tot[RT][MT];
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            cb[i][m] = acc[i][m] = floatx4{0.f, 0.f, 0.f, 0.f};
+            tot[i][m] = floatx4{0.f, 0.f, 0.f, 0.f};
+        }
+
+    QRaw<T> raw[RT], nxt[PF ? RT : 1];
+    const int s0 = b0 * SPB, s1 = b1 * SPB;
+    load_a(s0);
+#pragma unroll
+    for (int i = 0; i < RT; ++i) q_load<CH>(raw[i], row[i], nb, b0, q);
+    store_a(s0, s0 & 1);
+    load_a(min(s0 + 1, s1 - 1));
+    lds_barrier();
+
+    for (int b = b0; b < b1; ++b) {
+        if constexpr (PF) {
+#pragma unroll
+            for (int i = 0; i < RT; ++i) q_load<CH>(nxt[i], row[i], nb, min(b + 1, b1 - 1), q);
+        }
+        uint32_t dblk[RT], mins[RT];
+#pragma unroll
+        for (int i = 0; i < RT; ++i) q_block_scales<CH>(raw[i], q, dblk[i], mins[i]);
+#pragma unroll
+        for (int js = 0; js < SPB; ++js) {
+            const int s = b * SPB + js, buf = s & 1;
+            // the next step's operands go into the buffer that every wave finished with
+            // before the last barrier; their loads had a whole step
+            if (s + 1 < s1) store_a(s + 1, buf ^ 1);
+            load_a(min(s + 2, s1 - 1));
+            const half8* A = reinterpret_cast<const half8*>(As[buf]);
+#pragma unroll
+            for (int ju = 0; ju < UPS; ++ju) {
+                const int j = js * UPS + ju;
+                half8 wh[RT][2], wl[RT][2];
+#pragma unroll
+                for (int i = 0; i < RT; ++i) {
+                    if constexpr (T == kQ6K) q6_unit(raw[i], j, wh[i], wl[i]);
+                    else q4_unit<CH>(raw[i], q, j, wh[i]);
+                }
+                if constexpr (!PF) {
+                    if (j == 3) {
+#pragma unroll
+                        for (int i = 0; i < RT; ++i) q_load<CH>(raw[i], row[i], nb, min(b + 1, b1 - 1), q);
+                    }
+                }
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    // MP token tiles at a time: consecutive MFMAs add to different accumulators
+#pragma unroll
+                    for (int m = 0; m < MT; m += MP) {
+                        half8 xh[MP], xl[MP];
+#pragma unroll
+                        for (int u = 0; u < MP; ++u) {
+                            xh[u] = A[(m + u) * (UPS * 256) + (ju * 4 + 2 * h) * 64 + lane];
+                            xl[u] = A[(m + u) * (UPS * 256) + (ju * 4 + 2 * h + 1) * 64 + lane];
+                        }
+                        q_products<T, RT, MP, MT>(xh, xl, wh, wl, h, m, cb);
+                    }
+                }
+            }
+            if (js == SPB - 1) {
+                q_block_end<T, RT, MT>(Ss[b & 1], lane, dblk, mins, cb, acc);
+                if (gridDim.z == 1 && a.spans > 1 && ((b + 1) % a.span == 0 || b + 1 == b1)) {
+#pragma unroll
+                    for (int i = 0; i < RT; ++i)
+#pragma unroll
+                        for (int m = 0; m < MT; ++m)
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) {
+                                tot[i][m][r] += acc[i][m][r];
+                                acc[i][m][r] = 0.f;
+                            }
+                }
+            }
+            lds_barrier();
+        }
+        if constexpr (PF) {
+#pragma unroll
+            for (int i = 0; i < RT; ++i) raw[i] = nxt[i];
+        }
+    }
+    if (gridDim.z == 1 && a.spans > 1) {
+#pragma unroll
+        for (int i = 0; i < RT; ++i)
+#pragma unroll
+            for (int m = 0; m < MT; ++m) acc[i][m] = tot[i][m];
+    }
+    q_store<RT, MT>(a, n0, t0, rj, q, acc);
+}
+
+// The form for up to 32 tokens, where the weights' bytes are the bound: a workgroup splits
+// its span of the activations itself (no pass before it), keeps all of it in LDS, and its
+// waves then walk row tiles on their own -- no barrier, two blocks' weights in flight per
+// wave -- leaving each tile's sums over the span in part[z]. Grid: x = workgroups over the
+// rows, z = spans of kFewSpan blocks.
+constexpr int kFewSpan = 4;
+template <int T, bool CH, int MT>
+__global__ __launch_bounds__(1024) void gemm_q16_few_kernel(QGemmArgs a) {
+    constexpr int AV = MT * 1024;                        // 16-byte pieces of a block's operands
+    constexpr int SV = MT * (T == kQ4K ? 36 : 4);
+    __shared__ __align__(16) uint4 As[kFewSpan * AV];
+    __shared__ __align__(16) uint4 Ss[kFewSpan * SV];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int q = lane >> 4, rj = lane & 15;
+    const int nb = a.K / kBlk, b0 = blockIdx.z * kFewSpan, nbs = min(kFewSpan, nb - b0);
+    const int waves = blockDim.x >> 6, ntiles = (a.N + 15) >> 4, stride = gridDim.x * waves;
+    const int first = blockIdx.x * waves + wave;
+    const int mine = first < ntiles ? (ntiles - first + stride - 1) / stride : 0;  // row tiles of this wave
+    const int items = mine * nbs;
+
+    struct At {
+        int tile, b;           // row tile, block within the span
+        const uint8_t* row;
+    };
+    auto seek = [&](At& p) { p.row = q_row<T>(a, min(p.tile * 16 + rj, a.N - 1), nb); };
+    auto next = [&](At& p) {
+        if (++p.b == nbs) {
+            if (p.tile + stride < ntiles) {
+                p.b = 0;
+                p.tile += stride;
+                seek(p);
+            } else {
+                p.b = nbs - 1;  // past the end: the last block again, never used
+            }
+        }
+    };
+    QRaw<T> r0, r1;
+    At ld{min(first, ntiles - 1), 0, nullptr};
+    seek(ld);
+    q_load<CH>(r0, ld.row, nb, b0 + ld.b, q);
+    next(ld);
+    q_load<CH>(r1, ld.row, nb, b0 + ld.b, q);
+
+    for (int t = tid; t < nbs * MT * 256; t += blockDim.x) {
+        const int u = t >> 8, i = (t >> 4) & 15, c = t & 15, bl = u / MT, m = u - bl * MT;
+        float v[16];
+        load16(v, a.x, m * 16 + i, a.M, a.ldx, (b0 + bl) * kBlk + 16 * c);
+        uint4* side = Ss + bl * SV;
+        split16(v, i, c, reinterpret_cast<_Float16*>(As + bl * AV + m * 1024), reinterpret_cast<float*>(side + 4 * m),
+                reinterpret_cast<_Float16*>(side + 4 * MT + 32 * m), T == kQ4K);
+    }
+    __syncthreads();
+
+    // three product sums per token tile, added at the block's end: the xh * vh of the even
+    // and of the odd slices, and the small terms -- shorter chains of FP32 additions
+    // (relative error against 64 bits at 5 tokens x 4096 columns, Q6_K / Q4_K: 1.03e-7 /
+    // 1.19e-7, with one sum and a float reduction 1.63e-7 / 1.92e-7, the FP32 matvec 1.83e-7
+    // / 1.19e-7)
+    floatx4 cb[1][MT], c1[MT], cs[MT], acc[1][MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) cb[0][m] = c1[m] = cs[m] = acc[0][m] = floatx4{0.f, 0.f, 0.f, 0.f};
+    int tile = first, bl = 0;
+    auto compute = [&](const QRaw<T>& raw) {
+        uint32_t dblk[1], mins[1];
+        q_block_scales<CH>(raw, q, dblk[0], mins[0]);
+        const half8* A = reinterpret_cast<const half8*>(As + bl * AV);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            half8 wh[1][2], wl[1][2];
+            if constexpr (T == kQ6K) q6_unit(raw, j, wh[0], wl[0]);
+            else q4_unit<CH>(raw, q, j, wh[0]);
+            half8 xh[2][MT], xl[2][MT];
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int m = 0; m < MT; ++m) {
+                    xh[h][m] = A[m * 1024 + (4 * j + 2 * h) * 64 + lane];
+                    xl[h][m] = A[m * 1024 + (4 * j + 2 * h + 1) * 64 + lane];
+                }
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                cb[0][m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[0][m], wh[0][0], cb[0][m], 0, 0, 0);
+                c1[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[1][m], wh[0][1], c1[m], 0, 0, 0);
+            }
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int m = 0; m < MT; ++m) {
+                    cs[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl[h][m], wh[0][h], cs[m], 0, 0, 0);
+                    if constexpr (T == kQ6K)
+                        cs[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[h][m], wl[0][h], cs[m], 0, 0, 0);
+                }
+        }
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) cb[0][m][r] += c1[m][r] + cs[m][r];
+            c1[m] = cs[m] = floatx4{0.f, 0.f, 0.f, 0.f};
+        }
+        q_block_end<T, 1, MT>(Ss + bl * SV, lane, dblk, mins, cb, acc);
+        if (++bl == nbs) {
+            q_store<1, MT>(a, tile * 16, 0, rj, q, acc);
+#pragma unroll
+            for (int m = 0; m < MT; ++m) acc[0][m] = floatx4{0.f, 0.f, 0.f, 0.f};
+            bl = 0;
+            tile += stride;
+        }
+    };
+    for (int t = 0; t < items; t += 2) {
+        compute(r0);
+        next(ld);
+        q_load<CH>(r0, ld.row, nb, b0 + ld.b, q);
+        if (t + 1 < items) compute(r1);
+        next(ld);
+        q_load<CH>(r1, ld.row, nb, b0 + ld.b, q);
+    }
+}
+
+// The form for more than 64 tokens: 8 waves of 32 rows x 128 tokens, one workgroup per CU.
+// A step (one unit per lane, two slices) has a decode phase -- the operands of the next
+// step to LDS, the weights of this one to registers, a finished block's scaling -- and a
+// multiply phase of 96 (Q6_K) or 64 MFMAs with their LDS reads, a barrier after each.
+// Waves 4..7 run one phase behind waves 0..3 (one of each on every SIMD), so that one
+// group's vector work always runs beside the other's matrix work. Three operand buffers:
+// both groups write step s+1 while the slower one still reads step s-1. At 2048 tokens x
+// 24576 x 4096 the matrix cores are 59% busy at the 2.0 GHz the card holds there (1.2
+// PFLOP/s of fp16 products; a chain of MFMAs on registers alone holds 1.4 to 1.9 with data
+// like these): 980 us, 1050 with all eight waves in one phase. Without the decode, the
+// staging or the block scaling it would be 9%, 7% and 6% shorter; without its LDS reads no
+// shorter.
+template <int T, bool CH>
+__global__ __launch_bounds__(512, 2) void gemm_q16_wide_kernel(QGemmArgs a) {
+    constexpr int MT = 8, RT = 2, TH = 512, XD = 2;
+    constexpr int AV = MT * 256, AN = AV / TH;
+    constexpr int SV = MT * (T == kQ4K ? 36 : 4);
+    __shared__ __align__(16) uint4 As[3][AV];
+    __shared__ __align__(16) uint4 Ss[2][SV];
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int q = lane >> 4, rj = lane & 15;
+    const int tiles = (a.M + 15) >> 4, nb = a.K / kBlk;
+    const int t0 = blockIdx.y * MT, n0 = (blockIdx.x * 8 + wave) * (16 * RT);
+    const int b0 = gridDim.z > 1 ? blockIdx.z * a.span : 0;
+    const int b1 = gridDim.z > 1 ? min(b0 + a.span, nb) : nb;
+    const uint8_t* row[RT];
+#pragma unroll
+    for (int i = 0; i < RT; ++i) row[i] = q_row<T>(a, min(n0 + 16 * i + rj, a.N - 1), nb);
+
+    uint4 ra[AN], rs;
+    uint32_t off[AN];  // of this thread's pieces of a step, in bytes
+#pragma unroll
+    for (int k = 0; k < AN; ++k) {
+        const int v = k * TH + tid;
+        off[k] = (uint32_t)min(t0 + (v >> 8), tiles - 1) * (kTileHalves * 2) + (v & 255) * 16;
+    }
+    auto load_a = [&](int s) {
+        const int b = s >> 2, j = s & 3;
+        const char* base = reinterpret_cast<const char*>(a.xf) + (size_t)b * tiles * (kTileHalves * 2) + j * 4096;
+#pragma unroll
+        for (int k = 0; k < AN; ++k) ra[k] = gld16(base + off[k]);
+        if (j == 0 && tid < SV) rs = q_side(a, tiles, t0, b, tid, MT);
+    };
+    auto store_a = [&](int s, int buf) {
+#pragma unroll
+        for (int k = 0; k < AN; ++k) As[buf][k * TH + tid] = ra[k];
+        if ((s & 3) == 0 && tid < SV) Ss[(s >> 2) & 1][tid] = rs;
+    };
+
+    floatx4 cb[RT][MT], acc[RT][MT];
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) cb[i][m] = acc[i][m] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+    QRaw<T> raw[RT];
+    uint32_t dblk[RT], mins[RT];
+    const int s0 = b0 * 4, s1 = b1 * 4;
+    load_a(s0);
+#pragma unroll
+    for (int i = 0; i < RT; ++i) q_load<CH>(raw[i], row[i], nb, b0, q);
+    store_a(s0, 0);
+    load_a(s0 + 1);
+    lds_barrier();
+    if (wave >= 4) lds_barrier();
+    int buf = 0;
+    for (int b = b0; b < b1; ++b) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int s = b * 4 + j;
+            const int nbuf = buf == 2 ? 0 : buf + 1;
+            if (s + 1 < s1) store_a(s + 1, nbuf);
+            load_a(min(s + 2, s1 - 1));
+            if (j == 0) {
+                if (b > b0) q_block_end<T, RT, MT>(Ss[(b - 1) & 1], lane, dblk, mins, cb, acc);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int i = 0; i < RT; ++i) q_block_scales<CH>(raw[i], q, dblk[i], mins[i]);
+            }
+            half8 wh[RT][2], wl[RT][2];
+#pragma unroll
+            for (int i = 0; i < RT; ++i) {
+                if constexpr (T == kQ6K) q6_unit(raw[i], j, wh[i], wl[i]);
+                else q4_unit<CH>(raw[i], q, j, wh[i]);
+            }
+            if (j == 3) {
+#pragma unroll
+                for (int i = 0; i < RT; ++i) q_load<CH>(raw[i], row[i], nb, min(b + 1, b1 - 1), q);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            lds_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_setprio(1);
+            const half8* A = reinterpret_cast<const half8*>(As[buf]);
+            // operand pairs (slice h, token tile m) in turn, each read XD pairs ahead of its
+            // products: one wave of the SIMD multiplies, so nothing else hides its LDS reads
+            half8 xh[XD + 1][1], xl[XD + 1][1];
+            auto operands = [&](int k) {
+                const int h = k / MT, m = k - h * MT;
+                xh[k % (XD + 1)][0] = A[m * 256 + (2 * h) * 64 + lane];
+                xl[k % (XD + 1)][0] = A[m * 256 + (2 * h + 1) * 64 + lane];
+            };
+#pragma unroll
+            for (int k = 0; k < XD; ++k) operands(k);
+#pragma unroll
+            for (int k = 0; k < 2 * MT; ++k) {
+                if (k + XD < 2 * MT) operands(k + XD);
+                __builtin_amdgcn_sched_barrier(0);
+                q_products<T, RT, 1, MT>(xh[k % (XD + 1)], xl[k % (XD + 1)], wh, wl, k / MT, k % MT, cb);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            __builtin_amdgcn_s_setprio(0);
+            __builtin_amdgcn_sched_barrier(0);
+            lds_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+            buf = nbuf;
+        }
+    }
+    if (wave < 4) lds_barrier();
+    q_block_end<T, RT, MT>(Ss[(b1 - 1) & 1], lane, dblk, mins, cb, acc);
+    q_store<RT, MT>(a, n0, t0, rj, q, acc);
+}
+
+// Y[m][n] = sum over the spans, in order, in S (double for the form for few tokens, whose
+// spans are short; float where the spans may also have been added in registers); SwiGLU
+// pairs as above.
+template <class S> __global__ __launch_bounds__(256) void gemm_q16_reduce_kernel(QGemmArgs a) {
+    const int m = blockIdx.y, cols = a.pair ? a.N / 2 : a.N;
+    const int n = blockIdx.x * 256 + threadIdx.x;
+    if (n >= cols) return;
+    const size_t layer = (size_t)a.M * a.N;
+    if (a.pair) {
+        const float2* p = reinterpret_cast<const float2*>(a.part + (size_t)m * a.N + 2 * n);
+        S g = 0, u = 0;
+        for (int z = 0; z < a.spans; ++z) {
+            const float2 v = p[z * (layer / 2)];
+            g += v.x;
+            u += v.y;
+        }
+        a.y[(size_t)m * a.ldy + n] = siluf_((float)g) * (float)u;
+    } else {
+        const float* p = a.part + (size_t)m * a.N + n;
+        S v = 0;
+        for (int z = 0; z < a.spans; ++z) v += p[z * layer];
+        a.y[(size_t)m * a.ldy + n] = (float)v;
+    }
+}
+
+hipError_t launch_reduce(const QGemmArgs& a, int layers, hipStream_t stream) {
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess || layers == 1) return e;
+    const dim3 grid(((a.pair ? a.N / 2 : a.N) + 255) / 256, a.M);
+    if (gemm_q16_few(a.M)) launch_kernel(gemm_q16_reduce_kernel<double>, grid, dim3(256), 0, stream, a);
+    else launch_kernel(gemm_q16_reduce_kernel<float>, grid, dim3(256), 0, stream, a);
+    return hipGetLastError();
+}
+
+constexpr int kCUs = 256;
+
+// Token tiles per workgroup for M tokens.
+int tiles_for(int M) { return M <= 16 ? 1 : M <= 32 ? 2 : M <= 64 ? 4 : 8; }
+
+// One workgroup per CU over all the spans; the waves of each share its row tiles evenly (24576
+// rows of 4096 and 16 tokens: 12 waves with two tiles each 37.9 us with the reduction, two
+// 8-wave workgroups on half of the CUs 42.7).
+template <int T, bool CH, int MT> hipError_t launch_few(const QGemmArgs& a, int layers, hipStream_t stream) {
+    const int ntiles = (a.N + 15) / 16, gx = std::min(std::max(1, kCUs / layers), ntiles);
+    const int per = (ntiles + gx - 1) / gx, rounds = (per + 15) / 16, waves = (per + rounds - 1) / rounds;
+    launch_kernel(gemm_q16_few_kernel<T, CH, MT>, dim3((ntiles + waves * rounds - 1) / (waves * rounds), 1, layers),
+                  dim3(waves * 64), 0, stream, a);
+    return launch_reduce(a, layers, stream);
+}
+
+// Workgroups of mt token tiles x `rows` weight rows.
+template <class F>
+hipError_t launch_grid(F kernel, int mt, int rows, int threads, const QGemmArgs& a, int layers, hipStream_t stream) {
+    const dim3 grid((a.N + rows - 1) / rows, ((a.M + 15) / 16 + mt - 1) / mt, layers);
+    if (grid.y > 65535) return hipErrorInvalidValue;
+    launch_kernel(kernel, grid, dim3(threads), 0, stream, a);
+    return launch_reduce(a, layers, stream);
+}
+
+template <int T, bool CH, int MT, int RT, int WV, int UPS, bool PF, int OCC>
+hipError_t launch_form(const QGemmArgs& a, int layers, hipStream_t stream) {
+    return launch_grid(gemm_q16_kernel<T, CH, MT, RT, WV, UPS, PF, OCC>, MT, WV * RT * 16, WV * 64, a, layers, stream);
+}
+
+template <int T, bool CH> hipError_t launch_type(const QGemmArgs& a, int layers, hipStream_t stream) {
+    const int mt = tiles_for(a.M);
+    if (mt == 1) return launch_few<T, CH, 1>(a, layers, stream);
+    if (mt == 2) return launch_few<T, CH, 2>(a, layers, stream);
+    if (mt == 4) return launch_form<T, CH, 4, 1, 4, 1, true, 2>(a, layers, stream);
+    // 256 rows per workgroup, or 128 where that fills the last round of workgroups better
+    // (a workgroup of half the rows takes a bit over half the time)
+    const int groups = ((a.M + 127) / 128) * layers;
+    const int wide = (groups * ((a.N + 255) / 256) + kCUs - 1) / kCUs;
+    const int half = (groups * ((a.N + 127) / 128) + kCUs - 1) / kCUs;
+    if (half * 6 < wide * 10 || (layers == 1 && a.spans > 1) || a.M > (1 << 22))
+        return launch_form<T, CH, 8, 1, 8, 1, false, 2>(a, layers, stream);
+    return launch_grid(gemm_q16_wide_kernel<T, CH>, 8, 256, 512, a, layers, stream);
 }
 
 }  // namespace
 
 size_t gemm_q16_split_bytes(int M, int K, bool sums) {
-    const size_t mp = (size_t)(M + QM - 1) / QM * QM;  // rows padded to whole tiles
-    size_t b = mp * K * 2 * sizeof(_Float16) + (size_t)M * sizeof(int);
-    if (sums) b += (size_t)M * (K / 32) * 2 * sizeof(_Float16);
-    return (b + 255) / 256 * 256;
+    const size_t tiles = (size_t)(M + 15) / 16, nb = K / kBlk;
+    return tiles * nb * (kTileHalves * sizeof(_Float16) + 16 * sizeof(float) + (sums ? 512 : 0));
 }
 
 hipError_t launch_gemm_q16_split(const float* X, int M, int K, int ldx, void* scratch, bool sums, QGemmArgs* a,
                                  hipStream_t stream) {
-    if (M < 1 || K < QKS || K % kChunkCols || ldx < K) return hipErrorInvalidValue;
-    const int mp = (M + QM - 1) / QM * QM;
-    _Float16* xh = static_cast<_Float16*>(scratch);
-    _Float16* xl = xh + (size_t)mp * K;
-    int* rexp = reinterpret_cast<int*>(xl + (size_t)mp * K);
-    _Float16* sh = sums ? reinterpret_cast<_Float16*>(rexp + M) : nullptr;
-    _Float16* sl = sums ? sh + (size_t)M * (K / 32) : nullptr;
-    const bool v16 = reinterpret_cast<uintptr_t>(X) % 16 == 0 && ldx % 4 == 0;
-    if (v16 && K == 4096)
-        launch_kernel(split_rows8_kernel<2>, dim3(mp), dim3(256), 0, stream, X, M, K, ldx, xh, xl, rexp, sh, sl);
-    else if (v16 && K == 8192)
-        launch_kernel(split_rows8_kernel<4>, dim3(mp), dim3(256), 0, stream, X, M, K, ldx, xh, xl, rexp, sh, sl);
-    else if (v16 && K == 12288)
-        launch_kernel(split_rows8_kernel<6>, dim3(mp), dim3(256), 0, stream, X, M, K, ldx, xh, xl, rexp, sh, sl);
-    else
-        launch_kernel(split_rows_kernel, dim3(mp), dim3(256), 0, stream, X, M, K, ldx, xh, xl, rexp, sh, sl);
-    a->xh = reinterpret_cast<const uint16_t*>(xh);
-    a->xl = reinterpret_cast<const uint16_t*>(xl);
-    a->rexp = rexp;
-    a->sh = reinterpret_cast<const uint16_t*>(sh);
-    a->sl = reinterpret_cast<const uint16_t*>(sl);
+    if (M < 1 || K < kBlk || K % kBlk || ldx < K || ldx % 4 || reinterpret_cast<uintptr_t>(X) % 16)
+        return hipErrorInvalidValue;
+    const int tiles = (M + 15) / 16, nb = K / kBlk;
+    if (nb > 65535) return hipErrorInvalidValue;
+    _Float16* xf = static_cast<_Float16*>(scratch);
+    float* xe = reinterpret_cast<float*>(xf + (size_t)tiles * nb * kTileHalves);
+    _Float16* xs = sums ? reinterpret_cast<_Float16*>(xe + (size_t)tiles * nb * 16) : nullptr;
+    launch_kernel(split_tiles_kernel, dim3(tiles, nb), dim3(256), 0, stream, X, M, ldx, tiles, xf, xe, xs);
+    a->xf = reinterpret_cast<const uint16_t*>(xf);
+    a->xe = xe;
+    a->xs = reinterpret_cast<const uint16_t*>(xs);
     a->M = M;
     a->K = K;
     return hipGetLastError();
 }
 
-hipError_t launch_gemm_q16(uint32_t type, const QGemmArgs& a, hipStream_t stream) {
-    if ((type != kQ6K && type != kQ4K) || a.M < 1 || a.N < 1 || a.K % kChunkCols || a.nseg < 1 || a.nseg > kMaxSeg ||
-        a.row0[0] != 0 || a.row0[a.nseg] != a.N || (type == kQ4K && !a.sh))
+bool gemm_q16_few(int M) { return M <= 32; }
+
+// Column spans of a product with M tokens and K columns.
+int gemm_q16_spans(int M, int K) {
+    const int nb = K / kBlk, groups = (M + 127) / 128;
+    int spans;
+    if (M <= 64) spans = (nb + kFewSpan - 1) / kFewSpan;
+    else if (K >= 6144) spans = std::max(1, 8 * 12288 / K / groups);
+    else spans = groups == 1 ? 4 : groups <= 4 ? 2 : 1;
+    spans = std::max(1, std::min(spans, nb / 2));
+    const int span = (nb + spans - 1) / spans;  // blocks in each but the last
+    return (nb + span - 1) / span;
+}
+
+int gemm_q16_layers(int M, int N, int K) {
+    const int spans = gemm_q16_spans(M, K), mt = tiles_for(M);
+    if (spans == 1) return 1;
+    // the spans can also run in one workgroup after the other: with enough rows for a full
+    // chip, or very many partial sums, those need not go through memory
+    if (mt >= 4 && (N >= 65536 || (size_t)spans * M * N > (size_t(64) << 20))) return 1;
+    return spans;
+}
+
+hipError_t launch_gemm_q16(uint32_t type, QGemmArgs a, hipStream_t stream) {
+    if ((type != kQ6K && type != kQ4K) || a.M < 1 || a.N < 1 || a.K % kBlk || a.nseg < 1 || a.nseg > kMaxSeg ||
+        a.row0[0] != 0 || a.row0[a.nseg] != a.N || (!gemm_q16_few(a.M) && (!a.xf || (type == kQ4K && !a.xs))))
         return hipErrorInvalidValue;
     if (a.pair ? (a.nseg != 2 || a.N % 2 || a.row0[1] * 2 != a.N || a.ldy < a.N / 2) : a.ldy < a.N)
         return hipErrorInvalidValue;
-    const dim3 grid((a.N + QN - 1) / QN, (a.M + QM - 1) / QM);
-    if (grid.y > 65535) return hipErrorInvalidValue;
-    if (type == kQ6K) launch_kernel(gemm_q16_kernel<kQ6K>, grid, dim3(QThreads), 0, stream, a);
-    else launch_kernel(gemm_q16_kernel<kQ4K>, grid, dim3(QThreads), 0, stream, a);
-    return hipGetLastError();
+    const int nb = a.K / kBlk, layers = a.part || gemm_q16_few(a.M) ? gemm_q16_layers(a.M, a.N, a.K) : 1;
+    a.spans = gemm_q16_spans(a.M, a.K);
+    a.span = (nb + a.spans - 1) / a.spans;
+    if (gemm_q16_few(a.M) && a.span > kFewSpan) return hipErrorInvalidValue;
+    if (layers > 1 && (!a.part || a.M > 65535)) return hipErrorInvalidValue;
+    const bool ch = chunked_cols(a.K);
+    if (type == kQ6K) return ch ? launch_type<kQ6K, true>(a, layers, stream) : launch_type<kQ6K, false>(a, layers, stream);
+    return ch ? launch_type<kQ4K, true>(a, layers, stream) : launch_type<kQ4K, false>(a, layers, stream);
 }
 
 }  // namespace emprise

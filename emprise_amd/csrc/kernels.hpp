@@ -110,14 +110,17 @@ hipError_t launch_gemm_f32_heads(const float* A, const float* B, float* C, int M
                                  int ldc, int batch, int bdiv, size_t sA, size_t sB, size_t sC, bool causal_keys_n,
                                  bool causal_keys_k, int first, hipStream_t stream);
 
-// Batched projection on the fp16 matrix cores over chunked Q6_K / Q4_K weights
+// Batched projection on the fp16 matrix cores over Q6_K / Q4_K weights of either layout
 // (gemm_q.hip): Y[m][n] = row n of the stacked weights . X[m], for up to kMaxSeg weights of
 // one type whose rows follow each other in Y. launch_gemm_q16_split fills the activation
-// fields from X (fp16 hi/lo pieces of 2^-e_m x, e_m per row, and with `sums` the pieces of
-// its 32-column sums) in `scratch` (gemm_q16_split_bytes); the caller fills the weights.
+// fields from X (fp16 hi/lo pieces of 2^-e x, e per row and 256 columns, and with `sums` the
+// pieces of its 32-column sums) in `scratch` (gemm_q16_split_bytes); the caller fills the
+// weights and, where gemm_q16_layers says more than one, `part` (layers * M * N floats).
 struct QGemmArgs {
-    const uint16_t *xh, *xl, *sh, *sl;  // fp16 bits: x in 128 x 64 tiles (gemm_q.hip), sums [M][K/32]
-    const int* rexp;                    // [M]
+    const float* x;
+    int ldx;
+    const uint16_t *xf, *xs;  // fp16 bits in operand order (gemm_q.hip): pieces of x, of its sums
+    const float* xe;          // 2^e
     int M, K;
     const uint8_t* w[kMaxSeg];
     int row0[kMaxSeg + 1];  // weight s holds rows [row0[s], row0[s+1])
@@ -127,11 +130,18 @@ struct QGemmArgs {
     // SwiGLU pairs: two segments of N/2 rows each (gate, up), interleaved -- GEMM row n is
     // row n/2 of segment n%2 -- and y[m][n/2] = silu(gate) * up in place of both rows
     int pair;
+    float* part;      // the spans' partial sums
+    int spans, span;  // column spans and the blocks in each (set by the launch)
 };
 size_t gemm_q16_split_bytes(int M, int K, bool sums);
 hipError_t launch_gemm_q16_split(const float* X, int M, int K, int ldx, void* scratch, bool sums, QGemmArgs* a,
                                  hipStream_t stream);
-hipError_t launch_gemm_q16(uint32_t type, const QGemmArgs& a, hipStream_t stream);
+// Whether M tokens are few enough for the form that splits x itself (x, ldx, M and K set by
+// the caller, no split before it).
+bool gemm_q16_few(int M);
+// Column spans whose partial sums pass through `part` (1: none do).
+int gemm_q16_layers(int M, int N, int K);
+hipError_t launch_gemm_q16(uint32_t type, QGemmArgs a, hipStream_t stream);
 
 // ---- Gated DeltaNet ----
 struct GdnArgs {

@@ -525,7 +525,7 @@ std::vector<std::vector<float>> Model::evaluate_block(const std::vector<int>& to
         return out;
     }
     // all positions in one batched pass: every projection reads its weights once for the
-    // block (the small-batch matvec up to 7 positions, the GEMM from 8), the recurrent
+    // block (the small-batch matvec while the block fits one launch, else the GEMM), the recurrent
     // and attention steps run position by position, then the head over every row
     const size_t n = tokens.size(), start = position_;
     backend_->dev_upload(dev_prompt_ + start * sizeof(int), tokens.data(), n * sizeof(int));

@@ -126,7 +126,7 @@ emprise_status emprise_hip_linear_batch_many(emprise_hip* h, int n, const empris
                                              uint64_t ldx, emprise_dev Y, uint64_t ldy, int K);
 /* The gate/up half of Backend::feed_forward (backend.hpp:27-28; the reference's fused FFN,
  * model.cpp:230-236, swiglu at cuda.cpp:560-566) over K inputs: Y[k] = silu(G X[k]) * (U X[k]),
- * F = rows of G = rows of U floats per row, strides in floats. Chunked Q6_K/Q4_K gate and
+ * F = rows of G = rows of U floats per row, strides in floats. Q6_K/Q4_K gate and
  * up of one type run as one GEMM whose epilogue forms the SwiGLU; the values are those of
  * linear_batch_strided for G and U followed by swiglu, bit for bit. Batched prefill
  * support, like linear_batch_strided. */

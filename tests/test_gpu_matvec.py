@@ -502,3 +502,64 @@ def test_q8_register_quantiser_matches_lds_pass(backend_q8, rows, cols):
     for t in (vd, xd, dd, xo, y_plain, y_norm, y_delta):
         be.free(t)
     be.weight_free(w)
+
+
+def _gemm_bound(W, X, cols):
+    """Per output, the FP32 sum's bound: fp16 pieces carry x and drop below 2^-21 of a
+    product, then up to three additions per 32 columns and one per block and span."""
+    terms = 3 * cols // 32 + 2 * (cols // 256) + 16
+    return (terms * 2.0**-24 + 2.0**-21) * (np.abs(X.astype(np.float64)) @ np.abs(W.astype(np.float64)).T)
+
+
+# tokens around the 16-token tiles and the forms' limits (5, 16/17, 32/33, 64/65, 128/129),
+# rows around the 16-row tiles, one block, an odd number of blocks, several spans
+@pytest.mark.parametrize("wtype", [Q6_K, Q4_K])
+@pytest.mark.parametrize("tokens,rows,cols", [(2, 1, 256), (5, 33, 768), (16, 15, 2048), (17, 300, 4096), (32, 16, 1280),
+                                              (33, 257, 2560), (64, 17, 4096), (65, 129, 512), (128, 31, 6144),
+                                              (129, 600, 1536), (300, 257, 12288), (700, 100, 256)])
+def test_linear_batch_forms(backend, wtype, tokens, rows, cols):
+    """Every form of the fp16 GEMM, in both weight layouts, against 64 bits."""
+    rng = np.random.default_rng(tokens + rows + cols + wtype)
+    w = backend.upload_weight(wtype, cols, rows, matrix(rng, wtype, rows, cols))
+    X = (rng.standard_normal((tokens, cols)) * 10.0 ** rng.uniform(-3, 3, (tokens, 1))).astype(np.float32)
+    xd, yd, wd = backend.to_device(X), backend.alloc(tokens * rows * 4), backend.alloc(rows * cols * 4)
+    backend.linear_batch(w, xd, yd, tokens)
+    Y = backend.download(yd, (tokens, rows))
+    backend.dequantize_rows(w, 0, rows, wd)
+    W = backend.download(wd, (rows, cols))
+    ref = X.astype(np.float64) @ W.astype(np.float64).T
+    # Q4_K: d*sc*q and dmin*m are summed apart, each at most |w| + dmin*m in size
+    extra = 2.0**-18 * np.abs(X).sum(1, keepdims=True) * np.abs(W).max() if wtype == Q4_K else 0.0
+    assert np.all(np.abs(Y - ref) <= _gemm_bound(W, X, cols) + extra)
+    for b in (xd, yd, wd):
+        backend.free(b)
+    backend.weight_free(w)
+
+
+@pytest.mark.parametrize("tokens", [5, 40, 200])
+def test_linear_batch_in_a_new_graph(tokens):
+    """Captured with no earlier call of its size, so with no scratch of its own: the operands'
+    scratch is there from a larger call, partial sums stay in registers (or few rows go one
+    by one), and the replays agree with the eager call."""
+    from emprise_amd import HipBackend
+
+    rng = np.random.default_rng(tokens)
+    rows, cols = 200, 4096
+    with HipBackend() as be:
+        w = be.upload_weight(Q6_K, cols, rows, matrix(rng, Q6_K, rows, cols))
+        x = be.to_device(rng.standard_normal((1024, cols)).astype(np.float32))
+        y = be.alloc(1024 * rows * 4)
+        be.linear_batch(w, x, y, 1024)
+        be.graph_begin()
+        be.linear_batch(w, x, y, tokens)
+        g = be.graph_end()
+        be.linear_batch(w, x, y, tokens)
+        eager = be.download(y, (tokens, rows))
+        for _ in range(3):
+            be.fill(y, 0.0, tokens * rows)
+            be.graph_launch(g)
+            got = be.download(y, (tokens, rows))
+            if tokens > 32:
+                assert np.array_equal(got, eager)
+            else:
+                _close(got, eager)
