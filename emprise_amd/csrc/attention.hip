@@ -421,12 +421,30 @@ __global__ __launch_bounds__(256) void rope_table_kernel(float2* t, int context,
 
 // ---- batched form: `count` consecutive prompt positions (the prefill) --------------------
 //
-// Position t (absolute p0 + t) attends over 0..p0+t. The dense parts run on the matrix
-// cores through the FP32 GEMM (S = Q K^T per head, then O = P V): attn_prep_batch_kernel
+// Position t (absolute first + t) attends over keys 0..first+t. attn_prep_batch_kernel
 // normalises and rotates the queries and new keys exactly as attention_kernel does and
-// appends k/v to the caches; attn_softmax_batch_kernel turns a row of S into the
-// reference's exp(s - peak) / total with s = dot / sqrt(head_dim) (model.cpp:143-150)
-// and zeroes the masked keys; attn_gate_batch_kernel applies the sigmoid gate.
+// appends k/v to the caches; attn_split_kv_kernel writes the keys and values of 0..first+
+// count-1 as matrix operands; attn_flash_kernel then runs the scores, an online softmax and
+// P.V tile by tile, so no score goes through memory, and applies the sigmoid gate
+// (model.cpp:129-157). With few query rows the keys are split over workgroups and
+// attn_merge_batch_kernel joins their partial results.
+//
+// The products run on the fp16 matrix cores from two fp16 pieces per FP32 operand, as the
+// quantised GEMM's activations do: x = 2^e (xh + xl), 22 significant bits, the exponent e
+// taken per query and per key (from the largest of its head_dim values) and per 32-key tile
+// of values, three products of four (xl yl is below 2^-22 of its term), FP32 sums. Each
+// product has 16 queries on the lane index: S^T = K Q^T leaves lane (query l%16, group g =
+// l/16) the scores of keys 4g .. 4g+3 of two 16-key halves, which is the operand of O^T =
+// V^T P^T if V^T lists the 32 keys in that order -- so it does, and P goes from one product
+// to the next in registers. The probabilities are carried as 2^6 p relative to a
+// reference that the row maximum may pass by 2^8, above fp16's subnormals for p down to
+// 2^-20 of it.
+//
+// Bound by the matrix cores: 2048 positions behind 4096 of the 9B shape (16 Q / 4 KV heads x
+// 256) are 172 GFLOP, three times that in fp16 products; 582 us for all the kernels here
+// (885 TFLOP/s of products), of which the split 20 and the prep 20. As two FP32 GEMMs per
+// head with the scores in memory and a softmax pass between them it took 2570 us and 805 MB
+// of scratch; its error against 64 bits was 1.4e-6, now 8.8e-7 (relative, whole output).
 
 // Workgroup = one position; wave w normalises head vectors w, w+8, ... of the group's
 // q heads (all kv heads' groups) and the kv heads' new keys.
@@ -473,139 +491,478 @@ __global__ __launch_bounds__(512) void attn_prep_batch_kernel(AttnBatchArgs a) {
     }
 }
 
-// Row (t, h) of S (keys 0..L-1, padded to lp): p = exp(s - peak) / total over keys
-// 0..first+t with s = S / sqrt(head_dim); masked and padding keys get 0.
-__global__ __launch_bounds__(256) void attn_softmax_batch_kernel(AttnBatchArgs a) {
-    __shared__ float red[8];
-    const int row = blockIdx.x;  // h * count + t
-    const int t = row % a.count;
-    const int n = a.first + t + 1;
-    float* s = a.scores + (size_t)row * a.lp;
-    const float root = sqrtf((float)a.head_dim);
-    float m = -INFINITY;
-    for (int j = threadIdx.x; j < n; j += blockDim.x) m = fmaxf(m, s[j] / root);
-    m = wave_max(m);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
-    __syncthreads();
-    m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-    __syncthreads();
-    float total = 0.f;
-    for (int j = threadIdx.x; j < n; j += blockDim.x) {
-        const float e = expf(s[j] / root - m);
-        s[j] = e;
-        total += e;
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
+
+constexpr int kKeyTile = kAttnKeyTile;
+constexpr int kFlashRows = 128;  // query rows (position x head of a KV head's group) per workgroup
+constexpr int kFlashQT = 1;      // 16-row query tiles per wave
+constexpr float kBase = 6.f;     // P is carried as 2^kBase p, p <= 2^kLag
+constexpr float kLag = 8.f;
+
+// The exponent that brings a vector of largest magnitude mx to [2^12, 2^13).
+__device__ __forceinline__ int piece_exp(float mx) {
+    int e = 0;
+    if (mx > 0.f && mx < INFINITY) {
+        (void)frexpf(mx, &e);
+        e = max(e - 13, -126);
     }
-    total = wave_sum(total);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = total;
-    __syncthreads();
-    total = (red[0] + red[1]) + (red[2] + red[3]);
-    for (int j = threadIdx.x; j < a.lp; j += blockDim.x) s[j] = j < n ? s[j] / total : 0.f;
+    return e;
+}
+__device__ __forceinline__ void split8(const float (&v)[8], float up, half8& hi, half8& lo) {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const float w = v[k] * up;
+        hi[k] = (_Float16)w;
+        lo[k] = (_Float16)(w - (float)hi[k]);
+    }
 }
 
-// The same row softmax for rows of at most 256 * KR keys, the row held in registers from
-// its one read to its one write (the same thread-to-key assignment and sums as above,
-// so the same results).
-template <int KR>
-__global__ __launch_bounds__(256) void attn_softmax_rows_kernel(AttnBatchArgs a) {
-    __shared__ float red[8];
-    const int row = blockIdx.x;  // h * count + t
-    const int t = row % a.count;
-    const int n = a.first + t + 1;
-    float* s = a.scores + (size_t)row * a.lp;
-    const float root = sqrtf((float)a.head_dim);
-    float v[KR];
-    float m = -INFINITY;
+// Maximum / sum over lanes l, l^16, l^32, l^48 (the lane groups that share a query).
+template <class F> __device__ __forceinline__ float over_groups(float x, F f) {
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = f(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return f(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+__device__ __forceinline__ float max_groups(float x) {
+    return over_groups(x, [](float a, float b) { return fmaxf(a, b); });
+}
+__device__ __forceinline__ float sum_groups(float x) {
+    return over_groups(x, [](float a, float b) { return a + b; });
+}
+
+// Operands of the keys and values of one 32-key tile of one KV head (rows past the last
+// key are zero). Keys: half kt, slice s (32 dims), piece p, lane (key l%16, dims 8(l/16) ..
+// +7) -> ((kt*HD/32 + s)*2 + p)*512 + 8l halves, 2^e per key in ke. Values: dims tile dt,
+// piece p, lane (dim l%16, g) -> (dt*2 + p)*512 + 8l: keys 4g .. 4g+3, 16+4g .. 16+4g+3;
+// the tile's e in ve.
+template <int HD>
+__global__ __launch_bounds__(256) void attn_split_kv_kernel(AttnBatchArgs a) {
+    constexpr int CK = HD / 64;            // 8-dim pieces of a key per thread
+    constexpr int CV = HD / 64;            // (dims tile, lane) items per thread
+    __shared__ float red[4];
+    const int tile = blockIdx.x, kvh = blockIdx.y, tid = threadIdx.x;
+    const int L = a.first + a.count, kvd = a.kv_heads * HD, tiles = (L + kKeyTile - 1) / kKeyTile;
+    const size_t at = (size_t)kvh * tiles + tile;
+    {
+        const int key = tid >> 3, j = tid & 7, pos = tile * kKeyTile + key;
+        float v[CK][8], mx = 0.f;
 #pragma unroll
-    for (int k = 0; k < KR; ++k) {
-        const int j = threadIdx.x + 256 * k;
-        v[k] = j < n ? s[j] / root : -INFINITY;
-        m = fmaxf(m, v[k]);
-    }
-    m = wave_max(m);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
-    __syncthreads();
-    m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-    __syncthreads();
-    float total = 0.f;
+        for (int i = 0; i < CK; ++i) {
+            const float* src = a.keys + (size_t)min(pos, L - 1) * kvd + (size_t)kvh * HD + 8 * (8 * i + j);
+            float lo4[4], hi4[4];
+            ldv<4>(lo4, src);
+            ldv<4>(hi4, src + 4);
 #pragma unroll
-    for (int k = 0; k < KR; ++k) {
-        if ((int)threadIdx.x + 256 * k < n) {
-            v[k] = expf(v[k] - m);
-            total += v[k];
+            for (int k = 0; k < 4; ++k) {
+                v[i][k] = pos < L ? lo4[k] : 0.f;
+                v[i][4 + k] = pos < L ? hi4[k] : 0.f;
+                mx = fmaxf(mx, fmaxf(fabsf(v[i][k]), fabsf(v[i][4 + k])));
+            }
+        }
+        mx = fmaxf(mx, dpp_f<0xb1, 0xf>(mx, mx));   // over the key's 8 threads
+        mx = fmaxf(mx, dpp_f<0x4e, 0xf>(mx, mx));
+        mx = fmaxf(mx, dpp_f<0x141, 0xf>(mx, mx));
+        const int e = piece_exp(mx);
+        const float up = ldexpf(1.f, -e);
+        if (j == 0) a.ke[at * kKeyTile + key] = ldexpf(1.f, e);
+        _Float16* dst = reinterpret_cast<_Float16*>(a.kf) + at * (kKeyTile * HD * 2) + (size_t)(key >> 4) * (HD / 32) * 1024;
+#pragma unroll
+        for (int i = 0; i < CK; ++i) {
+            const int c = 8 * i + j, lane = (c & 3) * 16 + (key & 15);  // dims 8c: slice c/4, group c%4
+            half8 hi, lo;
+            split8(v[i], up, hi, lo);
+            *reinterpret_cast<half8*>(dst + (c >> 2) * 1024 + lane * 8) = hi;
+            *reinterpret_cast<half8*>(dst + (c >> 2) * 1024 + 512 + lane * 8) = lo;
         }
     }
-    total = wave_sum(total);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = total;
-    __syncthreads();
-    total = (red[0] + red[1]) + (red[2] + red[3]);
+    float v[CV][8], mx = 0.f;
 #pragma unroll
-    for (int k = 0; k < KR; ++k) {
-        const int j = threadIdx.x + 256 * k;
-        if (j < a.lp) s[j] = j < n ? v[k] / total : 0.f;
+    for (int i = 0; i < CV; ++i) {
+        const int item = i * 256 + tid, dt = item >> 6, lane = item & 63, g = lane >> 4;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const int pos = tile * kKeyTile + (k >> 2) * 16 + 4 * g + (k & 3);
+            const float x = a.values[(size_t)min(pos, L - 1) * kvd + (size_t)kvh * HD + dt * 16 + (lane & 15)];
+            v[i][k] = pos < L ? x : 0.f;
+            mx = fmaxf(mx, fabsf(v[i][k]));
+        }
     }
-}
-
-// vt[kvh][d][j] = values[j][kvh][d] for keys j < L, 0 up to lp: 32 x 32 tiles via LDS.
-__global__ __launch_bounds__(256) void attn_vt_batch_kernel(AttnBatchArgs a) {
-    __shared__ float tile[32][33];
-    const int kvh = blockIdx.z, d0 = blockIdx.y * 32, j0 = blockIdx.x * 32;
-    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;  // 32 x 8
-    const int L = a.first + a.count, kvd = a.kv_heads * a.head_dim;
-    for (int r = ty; r < 32; r += 8) {
-        const int j = j0 + r;
-        tile[r][tx] = j < L ? a.values[(size_t)j * kvd + (size_t)kvh * a.head_dim + d0 + tx] : 0.f;
-    }
+    mx = wave_max(mx);
+    if ((tid & 63) == 0) red[tid >> 6] = mx;
     __syncthreads();
-    for (int r = ty; r < 32; r += 8)
-        a.vt[((size_t)kvh * a.head_dim + d0 + r) * a.lp + j0 + tx] = tile[tx][r];
+    const int e = piece_exp(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
+    const float up = ldexpf(1.f, -e);
+    if (tid == 0) a.ve[at] = e;
+    _Float16* dst = reinterpret_cast<_Float16*>(a.vf) + at * (kKeyTile * HD * 2);
+#pragma unroll
+    for (int i = 0; i < CV; ++i) {
+        const int item = i * 256 + tid, dt = item >> 6, lane = item & 63;
+        half8 hi, lo;
+        split8(v[i], up, hi, lo);
+        *reinterpret_cast<half8*>(dst + dt * 1024 + lane * 8) = hi;
+        *reinterpret_cast<half8*>(dst + dt * 1024 + 512 + lane * 8) = lo;
+    }
 }
 
-// out[t][h*hd + d] = o[t][h*hd + d] * sigmoid(gate) (model.cpp:153)
-__global__ __launch_bounds__(256) void attn_gate_batch_kernel(AttnBatchArgs a) {
-    const int hdim = a.heads * a.head_dim;
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (size_t)a.count * hdim) return;
-    const int t = (int)(i / hdim), c = (int)(i % hdim), h = c / a.head_dim, d = c % a.head_dim;
-    const float g = a.qkv[(size_t)t * a.stride + (size_t)h * a.head_dim * 2 + a.head_dim + d];
-    a.out[(size_t)t * a.out_stride + c] = a.o[i] * sigmoidf_(g);
+// Key tiles with a key of the query rows of a half-tile.
+__device__ __forceinline__ int flash_tiles(const AttnBatchArgs& a, int rows, int half) {
+    const int t_last = (min(rows, (half + 1) * (kFlashRows / 2)) - 1) / (a.heads / a.kv_heads);
+    return (a.first + t_last) / kKeyTile + 1;
+}
+
+// 128 query rows of one KV head (row r: position r / group, head kvh*group + r % group)
+// over the key tiles of one split: 8 waves of 16 rows, queries and outputs in registers, the
+// tile's key and value operands shared through LDS, double-buffered. (Four waves of 32 rows
+// with 512 registers read half as much LDS but leave one wave per SIMD, with nothing beside
+// its softmax and its waits: 843 us against 660 at that stage; reading an operand further
+// ahead of its products, or pinning vector instructions between the products, no faster.)
+template <int HD, int TH = 64 * kFlashRows / 16 / kFlashQT>
+__global__ __launch_bounds__(TH, 2) void attn_flash_kernel(AttnBatchArgs a) {
+    constexpr int NS = HD / 32, ND = HD / 16, QT = kFlashQT, PD = 2;
+    constexpr int AV = kKeyTile * HD * 4 / 16;  // 16-byte pieces of a tile's keys (and of its values)
+    constexpr int AN = AV / TH;
+    __shared__ __align__(16) u32x4v Ks[2][AV], Vs[2][AV];
+    __shared__ __align__(16) float Es[2][kKeyTile + 4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int g = lane >> 4, qj = lane & 15;
+    const int kvh = blockIdx.x, group = a.heads / a.kv_heads, rows = a.count * group;
+    const int tiles_all = (a.first + a.count + kKeyTile - 1) / kKeyTile;
+    // half-tiles p and n-1-p: waves 0..3 (one per SIMD) have the rows with few keys, waves 4..7
+    // those with many, so that every workgroup has about the same work
+    const int halves = (rows + kFlashRows / 2 - 1) / (kFlashRows / 2), far = halves - 1 - (int)blockIdx.y;
+    const bool near = wave < TH / 128;
+    const int half = near ? (int)blockIdx.y : far;
+    const int row0 = half * (kFlashRows / 2) + (near ? wave : wave - TH / 128) * 16 * QT;
+    const int tile0 = blockIdx.z * a.split_tiles;
+    const int tile1 = min(flash_tiles(a, rows, far), tile0 + a.split_tiles);
+    if (tile0 >= tile1) return;
+    const int mine = min(tile1, flash_tiles(a, rows, half));  // this wave's last tile
+    const bool active = row0 < rows && tile0 < mine && !(near && half == far);
+
+    const u32x4v* kf = reinterpret_cast<const u32x4v*>(a.kf) + (size_t)kvh * tiles_all * AV;
+    const u32x4v* vf = reinterpret_cast<const u32x4v*>(a.vf) + (size_t)kvh * tiles_all * AV;
+    u32x4v rk[AN], rv[AN];
+    float re = 0.f;
+    auto load_keys = [&](int tile) {
+#pragma unroll
+        for (int k = 0; k < AN; ++k) rk[k] = kf[(size_t)tile * AV + k * TH + tid];
+        // their 2^e and, 33rd, the exponent of the tile's values
+        const size_t at = (size_t)kvh * tiles_all + tile;
+        if (tid < kKeyTile) re = a.ke[at * kKeyTile + tid];
+        else if (tid == kKeyTile) re = (float)a.ve[at];
+    };
+    auto load_values = [&](int tile) {
+#pragma unroll
+        for (int k = 0; k < AN; ++k) rv[k] = vf[(size_t)tile * AV + k * TH + tid];
+    };
+    auto store_keys = [&](int b) {
+#pragma unroll
+        for (int k = 0; k < AN; ++k) Ks[b][k * TH + tid] = rk[k];
+        if (tid <= kKeyTile) Es[b][tid] = re;
+    };
+    auto store_values = [&](int b) {
+#pragma unroll
+        for (int k = 0; k < AN; ++k) Vs[b][k * TH + tid] = rv[k];
+    };
+    load_keys(tile0);
+    load_values(tile0);
+
+    // the wave's queries as operands: lane (query l%16, dims 32s + 8g .. +7)
+    half8 qh[QT][NS], ql[QT][NS];
+    float qs[QT];  // 2^e / sqrt(head_dim) * log2(e): scores in units of log 2
+    int last[QT];  // the query's last key
+#pragma unroll
+    for (int u = 0; u < QT; ++u) {
+        const int r = min(row0 + 16 * u + qj, rows - 1), t = r / group, h = kvh * group + (r - t * group);
+        last[u] = a.first + t;
+        const float* src = a.q + ((size_t)t * a.heads + h) * HD + 8 * g;
+        float v[NS][8], mx = 0.f;
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            float lo4[4], hi4[4];
+            ldv<4>(lo4, src + 32 * s);
+            ldv<4>(hi4, src + 32 * s + 4);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                v[s][k] = lo4[k], v[s][4 + k] = hi4[k];
+                mx = fmaxf(mx, fmaxf(fabsf(lo4[k]), fabsf(hi4[k])));
+            }
+        }
+        const int e = piece_exp(max_groups(mx));
+        const float up = ldexpf(1.f, -e);
+#pragma unroll
+        for (int s = 0; s < NS; ++s) split8(v[s], up, qh[u][s], ql[u][s]);
+        qs[u] = ldexpf(1.44269504088896340736f / sqrtf((float)HD), e);
+    }
+
+    // S^T of a tile's two key halves
+    auto scores = [&](const u32x4v* keys, floatx4 (&S)[2][QT]) {
+        const half8* K = reinterpret_cast<const half8*>(keys);
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+            for (int u = 0; u < QT; ++u) S[kt][u] = floatx4{0.f, 0.f, 0.f, 0.f};
+        half8 kh[PD + 1][2], kl[PD + 1][2];  // slices read PD ahead of their products
+        auto operands = [&](int s) {
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt) {
+                kh[s % (PD + 1)][kt] = K[((kt * NS + s) * 2) * 64 + lane];
+                kl[s % (PD + 1)][kt] = K[((kt * NS + s) * 2 + 1) * 64 + lane];
+            }
+        };
+#pragma unroll
+        for (int s = 0; s < PD && s < NS; ++s) operands(s);
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            if (s + PD < NS) operands(s + PD);
+            const int b = s % (PD + 1);
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+                for (int u = 0; u < QT; ++u) S[kt][u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kl[b][kt], qh[u][s], S[kt][u], 0, 0, 0);
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+                for (int u = 0; u < QT; ++u) S[kt][u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh[b][kt], ql[u][s], S[kt][u], 0, 0, 0);
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+                for (int u = 0; u < QT; ++u) S[kt][u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh[b][kt], qh[u][s], S[kt][u], 0, 0, 0);
+            if (s + PD < NS) __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);  // LDS reads, then
+            __builtin_amdgcn_sched_group_barrier(0x008, 6 * QT, 0);             // products
+        }
+    };
+
+    // a tile's scores in log 2 units, masked, their maximum, and the exponent of its values
+    float x[QT][8], mx[QT];
+    int ev = 0;
+    auto scaled = [&](const floatx4 (&S)[2][QT], int tile, const float* E) {
+        const float4 k0 = *reinterpret_cast<const float4*>(E + 4 * g), k1 = *reinterpret_cast<const float4*>(E + 16 + 4 * g);
+        const float ke[8] = {k0.x, k0.y, k0.z, k0.w, k1.x, k1.y, k1.z, k1.w};
+        const int key0 = tile * kKeyTile + 4 * g;
+        ev = (int)E[kKeyTile];
+#pragma unroll
+        for (int u = 0; u < QT; ++u) {
+            mx[u] = -INFINITY;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                x[u][k] = key0 + (k >> 2) * 16 + (k & 3) <= last[u] ? (S[k >> 2][u][k & 3] * ke[k]) * qs[u] : -INFINITY;
+                mx[u] = fmaxf(mx[u], x[u][k]);
+            }
+            mx[u] = max_groups(mx[u]);
+        }
+    };
+
+    floatx4 O[ND][QT], S[2][QT];
+    float m[QT], l[QT];  // the reference that scores are taken against, and the sum of 2^(score - m + kBase)
+#pragma unroll
+    for (int u = 0; u < QT; ++u) {
+        m[u] = -INFINITY;
+        l[u] = 0.f;
+#pragma unroll
+        for (int d = 0; d < ND; ++d) O[d][u] = floatx4{0.f, 0.f, 0.f, 0.f};
+    }
+    int eo = -1000;  // O holds 2^-eo times its value
+    store_keys(0);
+    store_values(0);
+    load_keys(min(tile0 + 1, tile1 - 1));
+    load_values(min(tile0 + 1, tile1 - 1));
+    lds_barrier();
+    if (active) {
+        scores(Ks[0], S);
+        scaled(S, tile0, Es[0]);
+    }
+    store_keys(1);
+    load_keys(min(tile0 + 2, tile1 - 1));
+    lds_barrier();
+    // Iteration `tile`: the keys two tiles on and the values of the next go to LDS (loaded an
+    // iteration before, into what the last one finished with); then the softmax of this tile
+    // beside the next tile's scores, and the scaling of those beside P.V, so that the vector
+    // work stands next to matrix work that does not wait for it.
+    for (int tile = tile0, buf = 0; tile < tile1; ++tile, buf ^= 1) {
+        store_keys(buf);
+        store_values(buf ^ 1);
+        load_keys(min(tile + 3, tile1 - 1));
+        load_values(min(tile + 2, tile1 - 1));
+        if (active && tile < mine) {
+            const half8* V = reinterpret_cast<const half8*>(Vs[buf]);
+            // m follows the maximum only where that passes it by kLag (P then stays within fp16),
+            // so O is seldom rescaled
+            bool up = ev > eo;
+#pragma unroll
+            for (int u = 0; u < QT; ++u) up = up || mx[u] > m[u] + kLag;
+            if (__ballot(up)) {
+                const int en = max(eo, ev);
+                const float od = ldexpf(1.f, max(eo - en, -200));
+                eo = en;
+#pragma unroll
+                for (int u = 0; u < QT; ++u) {
+                    const float mn = mx[u] > m[u] + kLag ? mx[u] : m[u];
+                    const float f = mn == m[u] ? 1.f : __builtin_amdgcn_exp2f(m[u] - mn);
+                    m[u] = mn;
+                    l[u] *= f;
+#pragma unroll
+                    for (int d = 0; d < ND; ++d) O[d][u] *= f * od;
+                }
+            }
+            const float pv = ldexpf(1.f, ev - eo);
+            half8 ph[QT], pl[QT];
+#pragma unroll
+            for (int u = 0; u < QT; ++u) {
+                const float off = m[u] == -INFINITY ? 0.f : kBase - m[u];  // (no key of the row yet: all x are -inf)
+                float sum = 0.f;
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    const float p = __builtin_amdgcn_exp2f(x[u][k] + off);
+                    sum += p;
+                    const float w = p * pv;
+                    ph[u][k] = (_Float16)w;
+                    pl[u][k] = (_Float16)(w - (float)ph[u][k]);
+                }
+                l[u] += sum;
+            }
+            scores(Ks[buf ^ 1], S);
+            scaled(S, tile + 1, Es[buf ^ 1]);
+            // two dims tiles at a time, read PD pairs ahead
+            half8 vh[PD + 1][2], vl[PD + 1][2];
+            auto operands = [&](int d) {
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    vh[d % (PD + 1)][i] = V[((2 * d + i) * 2) * 64 + lane];
+                    vl[d % (PD + 1)][i] = V[((2 * d + i) * 2 + 1) * 64 + lane];
+                }
+            };
+#pragma unroll
+            for (int d = 0; d < PD && d < ND / 2; ++d) operands(d);
+#pragma unroll
+            for (int d = 0; d < ND / 2; ++d) {
+                if (d + PD < ND / 2) operands(d + PD);
+                const int b = d % (PD + 1);
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int u = 0; u < QT; ++u) O[2 * d + i][u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl[b][i], ph[u], O[2 * d + i][u], 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int u = 0; u < QT; ++u) O[2 * d + i][u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh[b][i], pl[u], O[2 * d + i][u], 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int u = 0; u < QT; ++u) O[2 * d + i][u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh[b][i], ph[u], O[2 * d + i][u], 0, 0, 0);
+                if (d + PD < ND / 2) __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 6 * QT, 0);
+            }
+        }
+        lds_barrier();
+    }
+    if (!active) return;
+
+    // lane: query l%16, dims 16d + 4g .. +3
+    float total[QT];
+#pragma unroll
+    for (int u = 0; u < QT; ++u) total[u] = sum_groups(l[u]);
+    if (gridDim.z > 1) {
+#pragma unroll
+        for (int u = 0; u < QT; ++u) {
+            const int r = row0 + 16 * u + qj;
+            if (r >= rows) continue;
+            const size_t at = ((size_t)blockIdx.z * a.kv_heads + kvh) * rows + r;
+            float* dst = a.part + at * HD;
+#pragma unroll
+            for (int d = 0; d < ND; ++d) *reinterpret_cast<floatx4*>(dst + 16 * d + 4 * g) = O[d][u];
+            if (g == 0) *reinterpret_cast<floatx4*>(a.stat + at * 4) = floatx4{m[u], total[u], (float)eo, 0.f};
+        }
+        return;
+    }
+    // through this wave's share of LDS, row by row: consecutive lanes write consecutive dims, and
+    // the gate's code stands here once (unrolled over the outputs it was 30 KB)
+    float* tile = reinterpret_cast<float*>(Ks) + wave * (16 * HD);
+#pragma unroll
+    for (int u = 0; u < QT; ++u) {
+#pragma unroll
+        for (int d = 0; d < ND; ++d) {
+            floatx4 o;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) o[k] = ldexpf(O[d][u][k] / total[u], eo);
+            *reinterpret_cast<floatx4*>(tile + qj * HD + 16 * d + 4 * g) = o;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const int n = min(16, rows - row0 - 16 * u);
+#pragma unroll 1
+        for (int i = 0; i < n; ++i) {
+            const int r = row0 + 16 * u + i, t = r / group, h = kvh * group + (r - t * group);
+            const float* gate = a.qkv + (size_t)t * a.stride + (size_t)h * HD * 2 + HD;
+            float* dst = a.out + (size_t)t * a.out_stride + (size_t)h * HD;
+#pragma unroll
+            for (int c = lane; c < HD; c += 64) dst[c] = tile[i * HD + c] * sigmoidf_(gate[c]);
+        }
+        if (u + 1 < QT) __builtin_amdgcn_wave_barrier();
+    }
+}
+
+// Joins the splits of one query row (workgroup = KV head x row, a thread per dim): sum_s
+// 2^(m_s - M + eo_s) O_s / sum_s 2^(m_s - M) l_s, then the sigmoid gate. A split whose keys
+// all lie past those of the row's half-tile was not run.
+__global__ __launch_bounds__(256) void attn_merge_batch_kernel(AttnBatchArgs a, int splits) {
+    const int hd = a.head_dim, group = a.heads / a.kv_heads, rows = a.count * group;
+    const int kvh = blockIdx.x, r = blockIdx.y, d = threadIdx.x;
+    const int t = r / group, h = kvh * group + (r - t * group);
+    const int n = min(splits, (flash_tiles(a, rows, r / (kFlashRows / 2)) + a.split_tiles - 1) / a.split_tiles);
+    const size_t step = (size_t)a.kv_heads * rows, at = (size_t)kvh * rows + r;
+    float M = -INFINITY;
+    for (int s = 0; s < n; ++s) M = fmaxf(M, a.stat[(at + s * step) * 4]);
+    float num = 0.f, den = 0.f;
+    for (int s = 0; s < n; ++s) {
+        const floatx4 st = *reinterpret_cast<const floatx4*>(a.stat + (at + s * step) * 4);
+        const float w = __builtin_amdgcn_exp2f(st[0] - M);  // (0 for a split none of whose keys the row has)
+        den = fmaf(w, st[1], den);
+        if (w > 0.f) num += ldexpf(w * a.part[(at + s * step) * hd + d], (int)st[2]);
+    }
+    const float gate = a.qkv[(size_t)t * a.stride + (size_t)h * hd * 2 + hd + d];
+    a.out[(size_t)t * a.out_stride + (size_t)h * hd + d] = num / den * sigmoidf_(gate);
 }
 
 }  // namespace
 
-hipError_t launch_attention_batch(const AttnBatchArgs& a, hipStream_t stream) {
-    const int group = a.heads / a.kv_heads, hd = a.head_dim, L = a.first + a.count;
-    if (a.count < 1 || a.heads % a.kv_heads || a.lp % 32 || a.lp < L || hd % 32) return hipErrorInvalidValue;
+int attention_batch_splits(int heads, int kv_heads, int first, int count) {
+    const int rows = count * (heads / kv_heads), wgs = kv_heads * ((rows + kFlashRows - 1) / kFlashRows);
+    const int tiles = (first + count + kKeyTile - 1) / kKeyTile;
+    // one workgroup per CU, each with at least two tiles
+    return std::max(1, std::min(256 / wgs, tiles / 2));
+}
+
+hipError_t launch_attention_batch(const AttnBatchArgs& a0, hipStream_t stream) {
+    AttnBatchArgs a = a0;
+    const int hd = a.head_dim, L = a.first + a.count;
+    if (a.count < 1 || a.heads % a.kv_heads || (hd != 64 && hd != 128 && hd != 256)) return hipErrorInvalidValue;
     const size_t prep_lds = (size_t)(a.heads + a.kv_heads) * hd * sizeof(float);
+    const int rows = a.count * (a.heads / a.kv_heads), tiles = (L + kKeyTile - 1) / kKeyTile;
+    int splits = a.part ? attention_batch_splits(a.heads, a.kv_heads, a.first, a.count) : 1;
+    a.split_tiles = (tiles + splits - 1) / splits;
+    splits = (tiles + a.split_tiles - 1) / a.split_tiles;
+    const dim3 kv_grid(tiles, a.kv_heads), grid(a.kv_heads, (rows + kFlashRows - 1) / kFlashRows, splits);
+    if (grid.y > 65535 || rows > 0x7fffffff / 2) return hipErrorInvalidValue;
+#define EMPRISE_ATTN_CASE(HD)                                                                             \
+    case HD:                                                                                              \
+        launch_kernel(attn_prep_batch_kernel<HD / 64>, dim3(a.count), dim3(512), prep_lds, stream, a);     \
+        launch_kernel(attn_split_kv_kernel<HD>, kv_grid, dim3(256), 0, stream, a);                         \
+        launch_kernel(attn_flash_kernel<HD>, grid, dim3(64 * kFlashRows / 16 / kFlashQT), 0, stream, a);                             \
+        break;
     switch (hd) {
-    case 64: launch_kernel(attn_prep_batch_kernel<1>, dim3(a.count), dim3(512), prep_lds, stream, a); break;
-    case 128: launch_kernel(attn_prep_batch_kernel<2>, dim3(a.count), dim3(512), prep_lds, stream, a); break;
-    case 256: launch_kernel(attn_prep_batch_kernel<4>, dim3(a.count), dim3(512), prep_lds, stream, a); break;
-    default: return hipErrorInvalidValue;
+        EMPRISE_ATTN_CASE(64)
+        EMPRISE_ATTN_CASE(128)
+        EMPRISE_ATTN_CASE(256)
     }
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    const int kvd = a.kv_heads * hd;
-    // S_h = Q_h K_kvh^T for every head in one launch; tiles wholly past the causal limit
-    // are skipped (the softmax reads keys 0 .. first+t of row t only)
-    e = launch_gemm_f32_heads(a.q, a.keys, a.scores, a.count, L, hd, a.heads * hd, kvd, a.lp, a.heads, group,
-                              (size_t)hd, (size_t)hd, (size_t)a.count * a.lp, true, false, a.first, stream);
-    if (e != hipSuccess) return e;
-    if (a.lp <= 256 * 8)
-        launch_kernel(attn_softmax_rows_kernel<8>, dim3(a.heads * a.count), dim3(256), 0, stream, a);
-    else if (a.lp <= 256 * 16)
-        launch_kernel(attn_softmax_rows_kernel<16>, dim3(a.heads * a.count), dim3(256), 0, stream, a);
-    else
-        launch_kernel(attn_softmax_batch_kernel, dim3(a.heads * a.count), dim3(256), 0, stream, a);
-    launch_kernel(attn_vt_batch_kernel, dim3(a.lp / 32, hd / 32, a.kv_heads), dim3(256), 0, stream, a);
-    e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    // O_h = P_h V_kvh for every head in one launch, each tile's K loop ending at its rows'
-    // last key (P is zero past it)
-    e = launch_gemm_f32_heads(a.scores, a.vt, a.o, a.count, hd, a.lp, a.lp, a.lp, a.heads * hd, a.heads, group,
-                              (size_t)a.count * a.lp, (size_t)hd * a.lp, (size_t)hd, false, true, a.first, stream);
-    if (e != hipSuccess) return e;
-    const size_t n = (size_t)a.count * a.heads * hd;
-    launch_kernel(attn_gate_batch_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, a);
+#undef EMPRISE_ATTN_CASE
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess || splits == 1) return e;
+    launch_kernel(attn_merge_batch_kernel, dim3(a.kv_heads, rows), dim3(hd), 0, stream, a, splits);
     return hipGetLastError();
 }
 

@@ -1118,7 +1118,6 @@ emprise_status emprise_hip_attention_batch(emprise_hip* h, const emprise_hip_att
     a.rotary = p->rotary;
     a.count = count;
     a.first = first_position;
-    a.lp = (first_position + count + 31) / 32 * 32;
     a.eps = p->eps;
     a.rope_base = p->rope_base;
     a.q_norm = reinterpret_cast<const float*>(qn->dev);
@@ -1130,15 +1129,25 @@ emprise_status emprise_hip_attention_batch(emprise_hip* h, const emprise_hip_att
     a.out = reinterpret_cast<float*>(out);
     a.out_stride = out_stride;
     const size_t hq = (size_t)count * p->heads * p->head_dim;
-    void *q, *sc, *vt, *o;
+    const size_t tiles = (size_t)(first_position + count + kAttnKeyTile - 1) / kAttnKeyTile * p->kv_heads;
+    const size_t pieces = tiles * kAttnKeyTile * p->head_dim * 4;  // of the keys, and of the values
+    const int splits = attention_batch_splits(p->heads, p->kv_heads, first_position, count);
+    void *q, *kv;
     TRY(h->get_scratch("attnb_q", hq * sizeof(float), &q));
-    TRY(h->get_scratch("attnb_s", (size_t)p->heads * count * a.lp * sizeof(float), &sc));
-    TRY(h->get_scratch("attnb_vt", (size_t)p->kv_heads * p->head_dim * a.lp * sizeof(float), &vt));
-    TRY(h->get_scratch("attnb_o", hq * sizeof(float), &o));
+    TRY(h->get_scratch("attnb_kv", 2 * pieces + tiles * (kAttnKeyTile + 1) * 4, &kv));
     a.q = static_cast<float*>(q);
-    a.scores = static_cast<float*>(sc);
-    a.vt = static_cast<float*>(vt);
-    a.o = static_cast<float*>(o);
+    a.kf = static_cast<uint16_t*>(kv);
+    a.vf = a.kf + pieces / 2;
+    a.ke = reinterpret_cast<float*>(a.vf + pieces / 2);
+    a.ve = reinterpret_cast<int*>(a.ke + tiles * kAttnKeyTile);
+    const size_t part_bytes = splits * (hq + (size_t)count * p->heads * 4) * sizeof(float);
+    // (captured with none there yet: one workgroup takes all the keys of its rows)
+    if (splits > 1 && !(h->capturing && h->scratch["attnb_part"].bytes < part_bytes)) {
+        void* part;
+        TRY(h->get_scratch("attnb_part", part_bytes, &part));
+        a.part = static_cast<float*>(part);
+        a.stat = a.part + splits * hq;
+    }
     // K/V rows 0..first+count-1 read twice (scores, transpose), the new rows written
     const uint64_t bytes = 3 * (uint64_t)(first_position + count) * p->kv_heads * p->head_dim * 4 + count * qkv_w * 4;
     return traced(h, "attention_batch", bytes, [&] { return launch_attention_batch(a, h->stream); });

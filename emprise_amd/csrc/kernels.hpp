@@ -101,15 +101,6 @@ hipError_t launch_dequant_rows(const uint8_t* w, uint32_t type, int cols, uint64
 // K must be a multiple of 16; lda and ldb multiples of 4 (16-byte rows).
 hipError_t launch_gemm_f32(const float* A, const float* B, float* C, int M, int N, int K, int lda, int ldb, int ldc,
                            hipStream_t stream);
-// `batch` products in one launch (grid z): C + z*sC = (A + z*sA) (B + (z/bdiv)*sB)^T.
-// causal_keys_n: N indexes keys and row m of a chunk uses keys <= first + m, so tiles
-// past every row's last key are skipped (their C is left unwritten); causal_keys_k: the
-// same with K indexing keys, each tile's K loop ending after its rows' last key (A must
-// be zero beyond it).
-hipError_t launch_gemm_f32_heads(const float* A, const float* B, float* C, int M, int N, int K, int lda, int ldb,
-                                 int ldc, int batch, int bdiv, size_t sA, size_t sB, size_t sC, bool causal_keys_n,
-                                 bool causal_keys_k, int first, hipStream_t stream);
-
 // Batched projection on the fp16 matrix cores over Q6_K / Q4_K weights of either layout
 // (gemm_q.hip): Y[m][n] = row n of the stacked weights . X[m], for up to kMaxSeg weights of
 // one type whose rows follow each other in Y. launch_gemm_q16_split fills the activation
@@ -209,11 +200,12 @@ struct AttnArgs {
 constexpr int kAttnSub = 16;     // positions per step of attention_kernel's online softmax
 constexpr int kAttnSplit = 64;   // position ranges (workgroups) per KV head of attention_kernel
 // `count` consecutive prompt positions from absolute position `first`: qkv row t at
-// t * stride floats; q (count x heads x hd), scores (heads x count x lp), vt (kv_heads x
-// hd x lp) and o (count x heads x hd) are scratch, lp = first + count rounded up to 32;
-// out row t at t * out_stride.
+// t * stride floats; out row t at t * out_stride. Scratch: q (count x heads x hd floats);
+// per KV head and 32-key tile kf and vf (32 x hd x 2 halves each), ke (32 floats) and ve; for
+// more than one split part (splits x kv_heads x rows x hd floats, rows = count x heads per KV
+// head) and stat (4 floats for each of those rows).
 struct AttnBatchArgs {
-    int heads, kv_heads, head_dim, rotary, count, first, lp;
+    int heads, kv_heads, head_dim, rotary, count, first;
     float eps, rope_base;
     const float2* rope;  // [context][rotary / 2] (cos, sin), as AttnArgs::rope
     const float* q_norm;
@@ -223,12 +215,17 @@ struct AttnBatchArgs {
     float* keys;
     float* values;
     float* q;
-    float* scores;
-    float* vt;
-    float* o;
+    uint16_t *kf, *vf;
+    float* ke;
+    int* ve;
+    float *part, *stat;
+    int split_tiles;  // key tiles per split (set by the launch)
     float* out;
     size_t out_stride;
 };
+constexpr int kAttnKeyTile = 32;
+// Splits of the keys over workgroups (at most; 1: none).
+int attention_batch_splits(int heads, int kv_heads, int first, int count);
 hipError_t launch_attention_batch(const AttnBatchArgs& a, hipStream_t stream);
 size_t attention_partial_floats(int heads, int kv_heads, int head_dim, int context);
 hipError_t launch_attention(const AttnArgs& a, hipStream_t stream);

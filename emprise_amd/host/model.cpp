@@ -548,8 +548,7 @@ std::vector<std::vector<float>> Model::evaluate_block(const std::vector<int>& to
 // projections of one input stacked into one GEMM (q|k|v; qkv|z|alpha|beta), the RMSNorms,
 // residual adds and SwiGLU run over all rows at once, the GDN conv + state update runs
 // as one scan over the chunk's positions (emprise_hip_delta_net_batch), and attention
-// runs over the chunk at once as FP32 GEMMs with a causal softmax
-// (emprise_hip_attention_batch). Op order is that of the unfused decode step.
+// runs over the chunk at once, tile by tile (emprise_hip_attention_batch). Op order is that of the unfused decode step.
 void Model::prefill_batched(size_t start, size_t count, std::vector<float>* logits) {
     constexpr size_t kPrefillChunk = 2048;
     HipBackend& b = *backend_;

@@ -558,3 +558,90 @@ def test_quantize_q8_exact_on_ties_and_scales(backend):
     assert np.array_equal(s.view(np.uint32), s_ref.view(np.uint32))
     for b in (xd, qd, sd):
         backend.free(b)
+
+
+def _attention_rows64(heads, kv, hd, rot, base, eps, qn, kn, rows, keys, values, first):
+    """Gated causal attention of the rows in 64 bits (the rotary angle is an FP32 value);
+    also the bound's parts: per row and head the largest sum |q k| / sqrt(hd) and sum p |v|."""
+    n, f8 = len(rows), np.float64
+    i = np.arange(rot // 2, dtype=np.float32)
+
+    def norm_rope(x, w):
+        x = x / np.sqrt((x * x).mean(-1, keepdims=True) + eps) * w
+        ang = (np.arange(first, first + n, dtype=np.float32)[:, None] /
+               np.power(np.float32(base), np.float32(2) * i / np.float32(max(rot, 1)))).astype(f8)[:, None]
+        a, b = x[..., :rot // 2], x[..., rot // 2:rot]
+        return np.concatenate([a * np.cos(ang) - b * np.sin(ang), a * np.sin(ang) + b * np.cos(ang), x[..., rot:]], -1)
+    qg = rows[:, :heads * hd * 2].astype(f8).reshape(n, heads, 2, hd)
+    q = norm_rope(qg[:, :, 0], qn)
+    k = norm_rope(rows[:, heads * hd * 2:heads * hd * 2 + kv * hd].astype(f8).reshape(n, kv, hd), kn)
+    v = rows[:, heads * hd * 2 + kv * hd:heads * hd * 2 + 2 * kv * hd].astype(f8).reshape(n, kv, hd)
+    ks = np.concatenate([keys.reshape(-1, kv, hd).astype(f8), k])
+    vs = np.concatenate([values.reshape(-1, kv, hd).astype(f8), v])
+    masked = np.arange(first + n)[None] > np.arange(first, first + n)[:, None]
+    out, bound = np.zeros((n, heads, hd)), np.zeros((n, heads, hd))
+    for h in range(heads):
+        j = h // (heads // kv)
+        s = np.where(masked, -np.inf, q[:, h] @ ks[:, j].T / np.sqrt(hd))
+        p = np.exp(s - s.max(1, keepdims=True))
+        p /= p.sum(1, keepdims=True)
+        gate = 1 / (1 + np.exp(-qg[:, h, 1]))
+        size = np.where(masked, 0, np.abs(q[:, h]) @ np.abs(ks[:, j]).T / np.sqrt(hd)).max(1, keepdims=True)
+        out[:, h] = p @ vs[:, j] * gate
+        bound[:, h] = p @ np.abs(vs[:, j]) * size * gate
+    return out.reshape(n, -1), bound.reshape(n, -1)
+
+
+# query rows (count x heads per KV head) around the 64-row half-tiles, keys around the 32-key
+# tiles, one and several splits, groups that do not divide a tile, every head size
+@pytest.mark.parametrize("heads,kv,hd,rot,first,count", [(16, 4, 256, 64, 27, 5), (16, 4, 256, 64, 0, 33),
+                                                        (6, 2, 128, 32, 31, 1), (6, 2, 128, 32, 0, 22),
+                                                        (8, 2, 64, 16, 1000, 33), (4, 4, 128, 0, 95, 130),
+                                                        (16, 2, 64, 64, 500, 17), (16, 4, 256, 64, 700, 300)])
+def test_attention_batch_tiles(backend, heads, kv, hd, rot, first, count):
+    """The tiled prefill attention against 64 bits, with cached values of very different sizes.
+    Scores carry a few 2^-22 of sum |q k| / sqrt(hd) (two fp16 pieces per operand, up to 24
+    FP32 additions), which moves P by as much of itself, P.V a few 2^-22 of sum p |v|."""
+    rng = np.random.default_rng(first + count + hd)
+    kvd, qd, L = kv * hd, heads * hd * 2, first + count
+    W = qd + 2 * kvd
+    qn = (1 + 0.02 * rng.standard_normal(hd)).astype(np.float32)
+    kn = (1 + 0.02 * rng.standard_normal(hd)).astype(np.float32)
+    keys = rng.standard_normal((first, kvd)).astype(np.float32)
+    values = (rng.standard_normal((first, kvd)) * 10.0 ** rng.uniform(-4, 4, (first, 1))).astype(np.float32)
+    rows = rng.standard_normal((count, W)).astype(np.float32)
+    kc, vc = np.zeros((L, kvd), np.float32), np.zeros((L, kvd), np.float32)
+    kc[:first], vc[:first] = keys, values
+    kd, vd, rd = backend.to_device(kc), backend.to_device(vc), backend.to_device(rows)
+    od = backend.alloc(count * heads * hd * 4)
+    p = AttentionParams(heads, kv, hd, rot, L, 1e-6, 1e7, backend.vector(qn), backend.vector(kn), kd, vd, 0)
+    backend.attention_batch(p, rd, count, W, first, od, heads * hd)
+    got = backend.download(od, (count, heads * hd))
+    ref, size = _attention_rows64(heads, kv, hd, rot, 1e7, 1e-6, qn, kn, rows, keys, values, first)
+    # + the FP32 cos/sin, norms and exp2 of the device, a few 2^-23 of the score each
+    assert np.all(np.abs(got - ref) <= 2.0**-18 * size + 1e-30)
+
+
+def test_attention_batch_in_a_new_graph():
+    """Captured with no partial-result scratch yet: one workgroup takes all of a row's keys."""
+    from emprise_amd import HipBackend
+
+    heads, kv, hd, rot, context = 16, 4, 256, 64, 1100
+    rng = np.random.default_rng(1)
+    W = heads * hd * 2 + 2 * kv * hd
+    with HipBackend() as be:
+        kd, vd = be.alloc(context * kv * hd * 4), be.alloc(context * kv * hd * 4)
+        rd = be.to_device(rng.standard_normal((1040, W)).astype(np.float32))
+        od = be.alloc(1040 * heads * hd * 4)
+        one = be.vector(np.ones(hd, np.float32))
+        p = AttentionParams(heads, kv, hd, rot, context, 1e-6, 1e7, one, one, kd, vd, 0)
+        be.attention_batch(p, rd, 1040, W, 0, od, heads * hd)
+        be.graph_begin()
+        be.attention_batch(p, rd, 40, W, 60, od, heads * hd)
+        g = be.graph_end()
+        be.attention_batch(p, rd, 40, W, 60, od, heads * hd)
+        eager = be.download(od, (40, heads * hd))
+        for _ in range(3):
+            be.fill(od, 0.0, 40 * heads * hd)
+            be.graph_launch(g)
+            _close(be.download(od, (40, heads * hd)), eager, tol=1e-5)
