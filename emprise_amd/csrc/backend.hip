@@ -242,10 +242,10 @@ emprise_status run_matvec(emprise_hip* h, const Proj* p, int n, int mode, const 
         a.cols = (int)cols;
         a.mode = mode;
         int g = 0;
-        uint64_t total_rows = 0;
-        for (int s = 0; s < a.nseg; ++s)
-            if (!(mode == kMvSwiglu && s == 1)) total_rows += p[i + s].w->rows;
-        const int R = matvec_rows_per_group(type, cols, mode, total_rows);
+        const bool q8 = h->q8 && type == kQ6K;
+        const uint64_t addresses = in ? in->x | in->delta | in->x_out : reinterpret_cast<uint64_t>(x_plain);
+        a.rows_form = (type == kQ6K || type == kQ4K) && !q8 && !chunked_cols(cols) && addresses % 16 == 0;
+        const int R = matvec_rows_per_group(type, cols, mode, a.rows_form);
         a.rows_per_group = R;
         for (int s = 0; s < a.nseg; ++s) {
             const Weight* w = p[i + s].w;
@@ -284,7 +284,6 @@ emprise_status run_matvec(emprise_hip* h, const Proj* p, int n, int mode, const 
             a.conv_width = conv_width;
         }
         a.argmax = argmax_key;
-        const bool q8 = h->q8 && type == kQ6K;
         // algorithmic bytes: encoded weights + the input read (x, delta, norm) + outputs
         uint64_t bytes = cols * 4 * (1 + (a.delta ? 1 : 0) + (a.gate ? 1 : 0) + (a.x_out ? 1 : 0)) +
                          (a.norm ? (a.gate ? (uint64_t)a.head_dim : cols) * 4 : 0);

@@ -69,6 +69,7 @@ struct MvArgs {
     float* conv_state;    // [rows][conv_width]
     int conv_width;
     int rows_per_group;   // R of the launch (matvec_rows_per_group)
+    bool rows_form;       // unit-major rows through matvec_rows_kernel: x, delta and x_out 16-byte aligned, FP32
 };
 
 size_t matvec_lds_bytes(uint32_t type, int cols, bool q8);
@@ -86,9 +87,8 @@ constexpr int kBatchMax = 4;                    // inputs per batched launch
 constexpr size_t kBatchLdsMax = 160 * 1024;     // LDS of one workgroup (one per CU)
 size_t matvec_batch_lds_bytes(uint32_t type, int cols, int k);
 hipError_t launch_matvec_batch(uint32_t type, const MvBatchArgs& a, int k, hipStream_t stream);
-// rows each row-group of MvArgs covers for this weight shape, mode and the launch's
-// total output rows (small launches use one row per wave to spread their arithmetic)
-int matvec_rows_per_group(uint32_t type, uint64_t cols, int mode, uint64_t total_rows);
+// rows each row-group of MvArgs covers for this weight type and width, mode and MvArgs::rows_form
+int matvec_rows_per_group(uint32_t type, uint64_t cols, int mode, bool rows_form);
 hipError_t launch_matvec(uint32_t type, bool q8, const MvArgs& a, int grid_cap, hipStream_t stream);
 hipError_t launch_matvec_stream(uint32_t type, bool q8, const MvArgs& a, hipStream_t stream);
 // Raw GGUF Q6_K / Q4_K rows (device) -> the kernel layout of layout.hpp (device).

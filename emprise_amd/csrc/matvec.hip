@@ -4,11 +4,12 @@
 // (Backend::linear / linear_many / the gate+up half of feed_forward,
 // reference cuda.cpp:199-304, 499-532, 567-596).
 //
-// Two kernels share this structure. Rows whose width is a multiple of 4096 (every
+// Three kernels share this structure. Rows whose width is a multiple of 4096 (every
 // projection of the qwen35 shapes) run in matvec_stream_kernel: workgroups of 8 or 16
 // waves, items of one row x one 4096-column chunk, one item in flight per wave (see the
-// streaming section below). Other widths run in matvec_kernel over the unit-major
-// layout: a workgroup of 4 waves stages the input vector once in LDS (with the
+// streaming section below). Other widths run over the unit-major layout: in
+// matvec_rows_kernel (its own section below), and with int8 activations or an input that
+// is not 16-byte aligned in matvec_kernel: a workgroup of 4 waves stages the input vector once in LDS (with the
 // residual add + RMSNorm of the reference's dev_add/dev_rmsnorm fused in, and the
 // per-unit input sums the zero-point terms need), then each wave takes groups of R
 // rows. In a group, lane l handles units l, l+64, l+128, ... of every row, so one
@@ -21,12 +22,14 @@
 // (d*sc) * (sum q*x - 32*sum x) and (d*sc)*(sum q*x) - (dmin*m)*(sum x): the same
 // products as the CPU path, grouped per unit. Only the order of FP32 additions
 // differs from the reference's sequential row sum.
+#include <algorithm>
 #include <mutex>
 
 #include "common.hpp"
 #include "kernels.hpp"
 #include "decode.hpp"
 #include "layout.hpp"
+#include "qshare.hpp"
 #include "stream.hpp"
 
 namespace emprise {
@@ -871,15 +874,26 @@ template <int T, bool Q8> hipError_t launch_stream_kind(const MvArgs& a, size_t 
 
 }  // namespace
 
-// Rows per item of the streaming kernel: one row (one gate/up pair). Measured in the
+// Rows per item. Streaming kernel: one row (one gate/up pair). Measured in the
 // 9B-shape decode (per-op graph): 1 row 510.6 tok/s, 2 rows 492.0, 4 rows 426.5 -- most
 // launches give a wave only a few items, and single-row items spread them over more
 // waves and cut the registers (66-85 VGPRs: 5-7 waves per SIMD instead of 4).
-int matvec_rows_per_group(uint32_t type, uint64_t cols, int mode, uint64_t total_rows) {
-    (void)total_rows;
-    if ((type == kQ6K || type == kQ4K) && cols % kChunkCols == 0)
-        return mode == kMvSwiglu ? kMvStreamPairRows : kMvStreamRows;
-    return (type == kQ6K || type == kQ4K) ? kMvRows : 1;
+// matvec_rows_kernel (`rows_form`): 64/G, with the G lanes per row that need the fewest
+// passes over the columns times the rounds that more waves than run at once take, for a
+// square matrix; of equals the fewest lanes. Only the width counts, so that a row's sum is
+// the same bits whichever rows share its launch.
+int matvec_rows_per_group(uint32_t type, uint64_t cols, int mode, bool rows_form) {
+    if (type != kQ6K && type != kQ4K) return 1;
+    if (cols % kChunkCols == 0) return mode == kMvSwiglu ? kMvStreamPairRows : kMvStreamRows;
+    if (!rows_form) return kMvRows;
+    const uint64_t groups = cols / 64;
+    double least = 0;
+    int rows = 1;
+    for (int g = 64; g >= 8; g /= 2) {
+        const double cost = (double)((groups + g - 1) / g) * std::max(1.0, (double)(cols * g) / 64 / (16 * 256));
+        if (g == 64 || cost <= least) least = cost, rows = 64 / g;
+    }
+    return rows;
 }
 
 hipError_t launch_matvec_stream(uint32_t type, bool q8, const MvArgs& a, hipStream_t stream) {
@@ -899,6 +913,234 @@ hipError_t launch_matvec_stream(uint32_t type, bool q8, const MvArgs& a, hipStre
 
 namespace {
 
+// ---- rows in the unit-major layout (widths that are not a multiple of 4096) -------------
+//
+// G lanes share a row (64/G rows per wave and item), lane j taking the row's 64-column
+// groups j, j+G, ..: one q_load each, the next group's loads in flight while one is
+// computed. The input is staged as in the streaming kernel, in 16-byte loads all issued at
+// once and behind the first weights' loads, float4 i of group c at i * groups + c, which
+// neighbouring lanes read side by side. Bound by latency at these sizes (a 2048 x 6144 Q4_K
+// matrix is 1 us of bandwidth): an FFN of 2048 -> 6144 -> 2048 takes 16.9 us as two launches;
+// with scalar staging, unit sums by strided LDS reads and no loads ahead (matvec_kernel,
+// which stays for inputs that are not 16-byte aligned and for int8 activations) 27 us.
+constexpr int kRowWaves = 8;
+constexpr int kRowStage = 8;  // float4 of the input per thread at most: 16384 columns
+
+// Sum over the G lanes of a row, in all of them.
+template <int G> __device__ __forceinline__ float sum_lanes(float v) {
+    v += dpp_f<0xb1, 0xf>(0.f, v);   // quad_perm [1,0,3,2]
+    v += dpp_f<0x4e, 0xf>(0.f, v);   // quad_perm [2,3,0,1]
+    if constexpr (G >= 8) v += dpp_f<0x141, 0xf>(0.f, v);   // row_half_mirror
+    if constexpr (G >= 16) v += dpp_f<0x140, 0xf>(0.f, v);  // row_mirror
+    if constexpr (G >= 32) {
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    }
+    if constexpr (G >= 64) {
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    }
+    return v;
+}
+
+// xs and usum (stored_unit_sum of each unit, in order) from x + delta, normalised.
+template <int UNIT> __device__ __forceinline__ void stage_rows(const MvArgs& a, float4* xs, float* usum, float* red) {
+    constexpr int TH = kRowWaves * 64;
+    const int n4 = a.cols / 4, groups = a.cols / 64, tid = threadIdx.x;
+    const float4* x4 = reinterpret_cast<const float4*>(a.x);
+    const float4* d4 = reinterpret_cast<const float4*>(a.delta);
+    const float4* w4 = reinterpret_cast<const float4*>(a.norm);
+    const bool writer = a.x_out && blockIdx.x == 0;
+    float4 v[kRowStage];
+    float ss = 0.f;
+#pragma unroll
+    for (int k = 0; k < kRowStage; ++k)
+        if (k * TH < n4) v[k] = x4[min(k * TH + tid, n4 - 1)];
+    if (d4) {
+#pragma unroll
+        for (int k = 0; k < kRowStage; ++k)
+            if (k * TH < n4) {
+                const float4 d = d4[min(k * TH + tid, n4 - 1)];
+                v[k].x += d.x, v[k].y += d.y, v[k].z += d.z, v[k].w += d.w;
+            }
+    }
+#pragma unroll
+    for (int k = 0; k < kRowStage; ++k) {
+        const int i = k * TH + tid;
+        if (i < n4) {
+            if (writer) reinterpret_cast<float4*>(a.x_out)[i] = v[k];
+            ss += v[k].x * v[k].x + v[k].y * v[k].y + v[k].z * v[k].z + v[k].w * v[k].w;
+        }
+    }
+    float scale = 1.f;
+    if (w4) scale = 1.f / sqrtf(block_sum_lds(ss, red) / (float)a.cols + a.eps);
+#pragma unroll
+    for (int k = 0; k < kRowStage; ++k) {
+        if (k * TH >= n4) continue;
+        const int i = k * TH + tid;
+        if (w4) {
+            const float4 w = w4[min(i, n4 - 1)];
+            v[k].x *= scale * w.x, v[k].y *= scale * w.y, v[k].z *= scale * w.z, v[k].w *= scale * w.w;
+        }
+        float t = (v[k].x + v[k].y) + (v[k].z + v[k].w);  // over the unit's 4 or 8 threads
+        t += dpp_f<0xb1, 0xf>(0.f, t);
+        t += dpp_f<0x4e, 0xf>(0.f, t);
+        if constexpr (UNIT == 32) t += dpp_f<0x141, 0xf>(0.f, t);
+        if (i < n4) {
+            xs[(i & 15) * groups + (i >> 4)] = v[k];
+            if (i % (UNIT / 4) == 0) usum[i / (UNIT / 4)] = stored_unit_sum<UNIT>(t);
+        }
+    }
+}
+
+// acc += 64 columns (group c) of each row times the staged input.
+template <int NA>
+__device__ __forceinline__ void dot_group(const QRaw<kQ6K> (&r)[NA], const float4* xs, const float* usum, int groups, int c,
+                                          float (&acc)[NA]) {
+    const float4 off4 = reinterpret_cast<const float4*>(usum)[c];
+    const float off[4] = {off4.x, off4.y, off4.z, off4.w};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        float4 x[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[i] = xs[(4 * j + i) * groups + c];
+#pragma unroll
+        for (int k = 0; k < NA; ++k) {
+            const float d = half_bits_to_float((uint16_t)r[k].d) * (float)(int)(int8_t)(r[k].sc >> (8 * j));
+            acc[k] = fmaf(d, q6_unit(r[k].w[0][j], r[k].w[1][j], r[k].w[2][j], x, off[j]), acc[k]);
+        }
+    }
+}
+template <int NA>
+__device__ __forceinline__ void dot_group(const QRaw<kQ4K> (&r)[NA], const float4* xs, const float* usum, int groups, int c,
+                                          float (&acc)[NA]) {
+    const float2 sum = reinterpret_cast<const float2*>(usum)[c];
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+        float s[NA][2] = {};
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {  // the low, then the high nibbles
+            float4 x[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) x[i] = xs[(8 * p + 4 * h + i) * groups + c];
+#pragma unroll
+            for (int k = 0; k < NA; ++k)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    s[k][i & 1] = dot4(opaque((r[k].w[p][i] >> (4 * h)) & 0x0F0F0F0Fu), x[i], s[k][i & 1]);
+            __builtin_amdgcn_sched_barrier(0);  // (registers: no reads further ahead)
+        }
+#pragma unroll
+        for (int k = 0; k < NA; ++k) {
+            const float dd = half_bits_to_float((uint16_t)(r[k].dd & 0xffffu)), dm = half_bits_to_float((uint16_t)(r[k].dd >> 16));
+            uint32_t sc, mn;
+            q4_sm<false>(r[k], c & 3, p, sc, mn);
+            acc[k] += (dd * (float)sc) * (s[k][0] + s[k][1]) - (dm * (float)mn) * (p ? sum.y : sum.x);
+        }
+    }
+}
+
+template <int T, bool PAIR, int G>
+__global__ __launch_bounds__(kRowWaves * 64) void matvec_rows_kernel(MvArgs a) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ float red[kRowWaves];
+    __shared__ unsigned long long block_best;
+    constexpr int R = 64 / G, NA = PAIR ? 2 : 1, UW = Fmt<T>::unit;
+    float4* xs = reinterpret_cast<float4*>(smem);
+    float* usum = reinterpret_cast<float*>(xs + a.cols / 4);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), j = lane % G;
+    const int nb = a.cols / 256, groups = a.cols / 64, passes = (groups + G - 1) / G, stride = gridDim.x * kRowWaves;
+    const size_t row_bytes = (size_t)nb * Fmt<T>::block;
+
+    struct Item {
+        int g, p, seg, row;       // item, pass; segment, this lane's row
+        const uint8_t* rp[NA];
+    };
+    auto seek = [&](Item& it) {
+        it.seg = 0;
+        while (it.seg + 1 < a.nseg && it.g >= a.seg[it.seg + 1].g0) ++it.seg;
+        it.row = (it.g - a.seg[it.seg].g0) * R + lane / G;
+        const size_t o = (size_t)min(it.row, a.seg[it.seg].rows - 1) * row_bytes;
+        it.rp[0] = a.seg[it.seg].w + o;
+        if constexpr (PAIR) it.rp[NA - 1] = a.seg[1].w + o;
+    };
+    auto load = [&](const Item& it, QRaw<T> (&raw)[NA]) {
+        const int c = min(it.p * G + j, groups - 1);  // (past the row's end: its last group, not added)
+#pragma unroll
+        for (int r = 0; r < NA; ++r) q_load<false>(raw[r], it.rp[r], nb, c >> 2, c & 3);
+    };
+    Item cur{min(blockIdx.x * kRowWaves + wave, (unsigned)a.groups - 1u) == blockIdx.x * kRowWaves + wave
+                 ? (int)(blockIdx.x * kRowWaves + wave)
+                 : a.groups,
+             0, 0, 0, {}};
+    QRaw<T> raw[NA], ahead[NA];
+    if (cur.g < a.groups) {
+        seek(cur);
+        load(cur, raw);
+    }
+    stage_rows<UW>(a, xs, usum, red);
+    if (a.mode == kMvArgmax && threadIdx.x == 0) block_best = 0ull;
+    lds_barrier();
+
+    unsigned long long best = 0ull;
+    float acc[NA] = {};
+    while (cur.g < a.groups) {
+        Item nxt = cur;
+        if (++nxt.p == passes) {
+            nxt.p = 0;
+            nxt.g += stride;
+            if (nxt.g < a.groups) seek(nxt);
+        }
+        if (nxt.g < a.groups) load(nxt, ahead);
+        const int c = cur.p * G + j, cc = min(c, groups - 1);
+        float part[NA] = {};
+        dot_group<NA>(raw, xs, usum, groups, cc, part);
+#pragma unroll
+        for (int r = 0; r < NA; ++r) acc[r] += c < groups ? part[r] : 0.f;
+        if (cur.p == passes - 1) {
+#pragma unroll
+            for (int r = 0; r < NA; ++r) acc[r] = sum_lanes<G>(acc[r]);
+            if (j == 0 && cur.row < a.seg[cur.seg].rows) {
+                float* y = a.seg[cur.seg].y + cur.row;
+                if constexpr (PAIR) {
+                    *y = siluf_(acc[0]) * acc[NA - 1];
+                } else if (a.conv_w && cur.seg == 0) {
+                    *y = conv_step(a.conv_w, a.conv_state, a.conv_width, cur.row, acc[0]);
+                } else {
+                    *y = (a.silu_mask >> cur.seg) & 1 ? siluf_(acc[0]) : acc[0];
+                    if (a.mode == kMvArgmax) {
+                        const unsigned long long k = argmax_key(acc[0], cur.row);
+                        best = k > best ? k : best;
+                    }
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < NA; ++r) acc[r] = 0.f;
+        }
+        cur = nxt;
+#pragma unroll
+        for (int r = 0; r < NA; ++r) raw[r] = ahead[r];
+    }
+    if (a.mode == kMvArgmax) {
+        if (best) atomicMax(&block_best, best);
+        __syncthreads();
+        if (threadIdx.x == 0 && block_best) atomicMax(a.argmax, block_best);
+    }
+}
+
+template <int T, bool PAIR> hipError_t launch_rows(const MvArgs& a, hipStream_t stream) {
+    const size_t lds = matvec_lds_bytes(T, a.cols, false);
+    const int grid = std::max(1, std::min((a.groups + kRowWaves - 1) / kRowWaves, 512));  // 16 waves per CU
+    const dim3 block(kRowWaves * 64);
+    switch (64 / a.rows_per_group) {
+    case 8: launch_kernel(matvec_rows_kernel<T, PAIR, 8>, dim3(grid), block, lds, stream, a); break;
+    case 16: launch_kernel(matvec_rows_kernel<T, PAIR, 16>, dim3(grid), block, lds, stream, a); break;
+    case 32: launch_kernel(matvec_rows_kernel<T, PAIR, 32>, dim3(grid), block, lds, stream, a); break;
+    case 64: launch_kernel(matvec_rows_kernel<T, PAIR, 64>, dim3(grid), block, lds, stream, a); break;
+    default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
 
 // Plain-layout (F32 / F16 / BF16) matvec: one wave per row, lanes stride the columns.
 template <int T>
@@ -1272,6 +1514,12 @@ hipError_t launch_matvec(uint32_t type, bool q8, const MvArgs& a, int grid_cap, 
     const bool pair = a.mode == kMvSwiglu;
     if ((type == kQ6K || type == kQ4K) && a.cols % kChunkCols == 0) return launch_matvec_stream(type, q8, a, stream);
     if (a.gate) return hipErrorInvalidValue;  // the per-head input transform is a streaming-kernel feature
+    if (a.rows_form) {
+        if (q8 || a.cols > kRowStage * kRowWaves * 256) return hipErrorInvalidValue;
+        if (type == kQ6K) return pair ? launch_rows<kQ6K, true>(a, stream) : launch_rows<kQ6K, false>(a, stream);
+        if (type == kQ4K) return pair ? launch_rows<kQ4K, true>(a, stream) : launch_rows<kQ4K, false>(a, stream);
+        return hipErrorInvalidValue;
+    }
     switch (type) {
     case kQ6K:
         if (q8) {

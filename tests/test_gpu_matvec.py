@@ -563,3 +563,68 @@ def test_linear_batch_in_a_new_graph(tokens):
                 assert np.array_equal(got, eager)
             else:
                 _close(got, eager)
+
+
+def _matvec_bound(W, x, rows_abs=0.0):
+    """Per output: FP32 sums of at most cols terms in short chains (64 per lane and group of
+    columns, then the lanes), with 2^-24 per addition and per product."""
+    terms = 160 + W.shape[1] // 64
+    return terms * 2.0**-24 * (np.abs(W.astype(np.float64)) @ np.abs(x.astype(np.float64)) + rows_abs)
+
+
+# widths of 1 to 64 groups per pass and with a last pass that is not full, row counts around
+# the rows of a wave and a workgroup
+@pytest.mark.parametrize("wtype", [Q6_K, Q4_K])
+@pytest.mark.parametrize("rows,cols", [(1, 256), (67, 512), (9, 768), (130, 1536), (33, 2048), (65, 2560), (17, 6144),
+                                       (3, 16128), (5001, 512), (4500, 2304)])
+def test_linear_unit_major_rows(backend, wtype, rows, cols):
+    """Rows whose width is no multiple of 4096: plain, two segments in one launch (the same
+    bits), normalised with a residual, SwiGLU pairs and the output head, against 64 bits;
+    an input 4 bytes off a 16-byte boundary takes the general kernel."""
+    rng = np.random.default_rng(rows + cols + wtype)
+    be, eps = backend, 1e-6
+    w = be.upload_weight(wtype, cols, rows, matrix(rng, wtype, rows, cols))
+    w2 = be.upload_weight(wtype, cols, rows, matrix(rng, wtype, rows, cols))
+    wide = be.alloc(rows * cols * 4)
+    be.dequantize_rows(w, 0, rows, wide)
+    W = be.download(wide, (rows, cols)).astype(np.float64)
+    be.dequantize_rows(w2, 0, rows, wide)
+    W2 = be.download(wide, (rows, cols)).astype(np.float64)
+    x, delta = (rng.standard_normal(cols).astype(np.float32) for _ in range(2))
+    nw = (1 + 0.02 * rng.standard_normal(cols)).astype(np.float32)
+    buf = be.to_device(np.concatenate([x, np.zeros(1, np.float32), x]))
+    dd, xo, nwd = be.to_device(delta), be.alloc(cols * 4), be.vector(nw)
+    y, y2, idx = be.alloc(rows * 4), be.alloc(rows * 4), be.alloc(4)
+    # Q4_K: d*sc*q and dmin*m are summed apart, each at most |w| + dmin*m in size
+    mins = np.abs(x).sum() * np.abs(W).max() if wtype == Q4_K else 0.0
+    bound = _matvec_bound(W, x, mins)
+
+    be.linear(w, buf, y)
+    one = be.download(y, rows)
+    assert np.all(np.abs(one - W @ x) <= bound)
+    be.linear_many([w2, w], buf, [y2, y])
+    assert np.array_equal(be.download(y, rows), one)
+    be.linear(w, buf + (cols + 1) * 4, y)
+    assert np.all(np.abs(be.download(y, rows) - one) <= 2 * bound)
+
+    v = x + delta
+    n = oracle.rms(v, nw, eps)
+    nb = _matvec_bound(W, n, mins * np.abs(n).sum() / np.abs(x).sum())
+    be.linear_norm(Input(buf, dd, xo, nwd, eps), [w], [y])
+    assert np.array_equal(be.download(xo, cols), v)
+    assert np.all(np.abs(be.download(y, rows) - W @ n) <= 2 * nb)  # (the norm's own rounding)
+    be.lm_head(Input(buf, dd, xo, nwd, eps), w, y2, idx)
+    assert np.array_equal(be.download(y2, rows), be.download(y, rows))
+    assert int(be.download(idx, 1, np.int32)[0]) == int(np.argmax(be.download(y, rows)))
+
+    dw = be.upload_weight(F32, rows, 1, np.ones(rows, np.float32))
+    be.feed_forward(w, w2, dw, buf, y)  # down projection: the sum of the hidden values
+    g, u = W @ x, W2 @ x
+    h = g / (1 + np.exp(-g)) * u
+    ub = _matvec_bound(W2, x, np.abs(x).sum() * np.abs(W2).max() if wtype == Q4_K else 0.0)
+    hb = 1.2 * bound * np.abs(u) + ub * np.abs(g) + 1.2 * bound * ub + 2.0**-20 * np.abs(h)
+    assert abs(be.download(y, 1)[0] - h.sum()) <= hb.sum() + (rows // 64 + 16) * 2.0**-24 * np.abs(h).sum()
+    for b in (wide, buf, dd, xo, y, y2, idx):
+        be.free(b)
+    for q in (w, w2, nwd, dw):
+        be.weight_free(q)
