@@ -154,7 +154,8 @@ struct emprise_hip {
             s.ptr = nullptr;
             s.bytes = 0;
             HIP_TRY(hipMalloc(&s.ptr, bytes));
-            if (zero) HIP_TRY(hipMemset(s.ptr, 0, bytes));
+            // on this stream: one of the null stream's may still be running when the next kernel reads it
+            if (zero) HIP_TRY(hipMemsetAsync(s.ptr, 0, bytes, stream));
             s.bytes = bytes;
         }
         *out = s.ptr;
