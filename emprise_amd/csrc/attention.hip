@@ -1,12 +1,12 @@
 // Gated GQA attention decode on gfx950 (Model::Impl::attention_preout, reference
 // model.cpp:129-157, which the reference runs on the host even on its device path).
 //
-// Split-KV ("flash decoding") over a fixed grid: workgroup (kv head, range j of
-// kAttnSplit) serves the `group` = heads/kv_heads query heads that share the KV head, so
+// Split-KV ("flash decoding") over a fixed grid: workgroup (range j of kAttnSplit, kv head;
+// the ranges that short contexts leave empty are dispatched last: 4 KV heads at 200 positions
+// 9.5 us, head-major 10.7) serves the `group` = heads/kv_heads query heads that share the KV head, so
 // each K/V row is read once for all of them, over range j of the positions 0..pos. The
 // ranges are whole sub-chunks of kAttnSub positions, as many per range as it takes to
-// cover the context with kAttnSplit ranges: one sub-chunk each up to 1024 positions,
-// four at 4096. Every workgroup recomputes the RMSNorm + RoPE of its query heads and of
+// cover the context with the ranges in use (attn_per). Every workgroup recomputes the RMSNorm + RoPE of its query heads and of
 // the new key (a few KiB of work); the workgroup whose range holds the current position
 // also appends the new k/v to the caches and uses them straight from LDS. Each
 // workgroup writes an unnormalised partial (o, running max, sum of exponentials); a
@@ -50,6 +50,7 @@ namespace {
 
 constexpr int kAttnWaves = 8;
 constexpr int kMaxGroup = 8;
+constexpr int kAttnLong = 512;  // sub-chunks (8192 positions) past which kAttnSplit ranges are faster
 
 // E consecutive floats (lane l of a wave owns dims E*l .. E*l+E-1 of a head): one
 // 16-, 8- or 4-byte access.
@@ -70,13 +71,20 @@ template <int E> __device__ __forceinline__ void stv(float* p, const float (&v)[
     else *p = v[0];
 }
 
-// Positions [first_sub * CH, end_sub * CH) of the workgroup's range: the `len`
-// positions are cut into nsub = ceil(len / CH) sub-chunks, and range j of kAttnSplit
-// takes `per` = ceil(nsub / kAttnSplit) consecutive sub-chunks (ranges past the end are
-// empty). The combine kernel recomputes the same split to know how many partials exist.
-__device__ __forceinline__ int attn_per(int len) {
+// The `len` positions are cut into nsub = ceil(len / CH) sub-chunks, and range j takes
+// `per` = ceil(nsub / ranges) consecutive ones (ranges past the end are empty). The combine
+// kernel recomputes the same split to know how many partials exist.
+//
+// ranges: kAttnFew while they give every CU a workgroup and the range is short, else
+// kAttnSplit, two workgroups per CU, so that 16 waves' rows are in flight. The second 64
+// partials cost the merge a round trip behind the position read (4 KV heads x 256, us with
+// 128 and 64 ranges: 19.0 / 16.7 at 4000 positions, 27.6 / 22.3 at 8000, 32.3 / 36.2 at
+// 16000, 53.3 / 63.3 at 30000). Two KV heads fill the chip only with 128 (10.9 / 12.1 at
+// 4000, 28.8 / 48.5 at 30000).
+__device__ __forceinline__ int attn_per(int len, int kv_heads) {
     const int nsub = (len + kAttnSub - 1) / kAttnSub;
-    return (nsub + kAttnSplit - 1) / kAttnSplit;
+    const int ranges = kv_heads * kAttnFew < 256 || nsub > kAttnLong ? kAttnSplit : kAttnFew;
+    return (nsub + ranges - 1) / ranges;
 }
 
 // Eight wave-wide sums at once: halving exchanges across lanes l^32 and l^16
@@ -106,22 +114,25 @@ __device__ __forceinline__ void wave_sum8(const float (&x)[8], float (&out)[8]) 
     for (int j = 0; j < 8; ++j) out[j] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), 8 * j));
 }
 
-template <int E>  // head_dim = 64 * E
-__global__ __launch_bounds__(kAttnWaves * 64) void attention_kernel(AttnArgs a) {
+// Bound by the K/V rows in flight: with registers and LDS for up to 4 query heads per KV head
+// (97 and 39 KiB at head_dim 256, instead of 149 and 76 KiB for 8) two workgroups share a CU.
+// 30000 positions of 4 KV heads x 256: 66.6 -> 52.7 us (3.7 -> 4.7 TB/s); 2 x 64: 49.2 -> 28.8.
+template <int E, int MG>  // head_dim = 64 * E, at most MG query heads per KV head
+__global__ __launch_bounds__(kAttnWaves * 64, MG <= 4 ? 4 : 2) void attention_kernel(AttnArgs a) {
     constexpr int HD = 64 * E, CH = kAttnSub, PW = CH / kAttnWaves;  // rows per wave and sub-chunk
-    __shared__ __align__(16) float qs[kMaxGroup][HD];
+    __shared__ __align__(16) float qs[MG][HD];
     __shared__ __align__(16) float knew[HD], vnew[HD];
-    __shared__ float wstat[kAttnWaves][kMaxGroup][2];  // per wave and head: max, sum
-    __shared__ __align__(16) float acc_lds[kAttnWaves][kMaxGroup][HD];
+    __shared__ float wstat[kAttnWaves][MG][2];  // per wave and head: max, sum
+    __shared__ __align__(16) float acc_lds[kAttnWaves][MG][HD];
 
     const int group = a.heads / a.kv_heads;
-    const int kvh = blockIdx.x / kAttnSplit, range = blockIdx.x % kAttnSplit;
+    const int range = blockIdx.x / a.kv_heads, kvh = blockIdx.x - range * a.kv_heads;
     const int pos = *a.position;
     if (pos < 0 || pos >= a.context) return;  // the host keeps positions inside the caches
     const int rpos = a.rope_position ? *a.rope_position : pos;
     if (rpos < 0 || rpos >= a.context) return;  // the RoPE table has `context` rows
     const int len = pos + 1;
-    const int nsub = (len + CH - 1) / CH, per = attn_per(len);
+    const int nsub = (len + CH - 1) / CH, per = attn_per(len, a.kv_heads);
     const int sub0 = range * per, sub1 = min(nsub, sub0 + per);
     if (sub0 >= sub1) return;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -150,7 +161,7 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attention_kernel(AttnArgs a) 
     // K and V rows of the first sub-chunk. The norm inputs are loaded unconditionally
     // (clamped heads) so waiting for them never waits for the K/V rows, whose latency
     // overlaps the norms and RoPE.
-    constexpr int NJ = (kMaxGroup + kAttnWaves) / kAttnWaves;  // heads per wave, incl. the key
+    constexpr int NJ = (MG + kAttnWaves) / kAttnWaves;  // heads per wave, incl. the key
     float xin[NJ][E], qn[E], kn[E];
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
@@ -211,14 +222,14 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attention_kernel(AttnArgs a) 
     // softmax over its rows of the range's sub-chunks (running maximum, sum and P.V),
     // with the next sub-chunk's rows loading while the current one is used; the four
     // waves are merged (max-rescaled) through LDS at the end.
-    float qv[kMaxGroup][E];
+    float qv[MG][E];
 #pragma unroll
-    for (int g = 0; g < kMaxGroup; ++g)
+    for (int g = 0; g < MG; ++g)
         if (g < group) ldv<E>(qv[g], qs[g] + E * lane);
     const float inv_root = 1.f / sqrtf((float)HD);
-    float mw[kMaxGroup], lw[kMaxGroup], acc[kMaxGroup][E];
+    float mw[MG], lw[MG], acc[MG][E];
 #pragma unroll
-    for (int g = 0; g < kMaxGroup; ++g) {
+    for (int g = 0; g < MG; ++g) {
         mw[g] = -INFINITY;
         lw[g] = 0.f;
 #pragma unroll
@@ -228,7 +239,7 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attention_kernel(AttnArgs a) 
         const int t0 = sub * CH, tn = min(CH, len - t0);
         float kn2[PW][E], vn2[PW][E];
         if (sub + 1 < sub1) load_rows(kn2, vn2, sub + 1);
-        float sc[PW][kMaxGroup];
+        float sc[PW][MG];
 #pragma unroll
         for (int i = 0; i < PW; ++i) {
             const int tt = wave + kAttnWaves * i;
@@ -237,7 +248,7 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attention_kernel(AttnArgs a) 
                 ldv<E>(vr[i], vnew + E * lane);
             }
         }
-        if (PW * 4 == 8 && group == 4) {
+        if (PW * 4 == 8 && MG == 4 && group == 4) {
             // the wave's eight scores (PW rows x 4 heads) reduced together
             float d[8], s8[8];
 #pragma unroll
@@ -258,7 +269,7 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attention_kernel(AttnArgs a) 
 #pragma unroll
             for (int i = 0; i < PW; ++i)
 #pragma unroll
-                for (int g = 0; g < kMaxGroup; ++g) {
+                for (int g = 0; g < MG; ++g) {
                     if (g < group) {
                         float p = 0.f;
 #pragma unroll
@@ -268,7 +279,7 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attention_kernel(AttnArgs a) 
                 }
         }
 #pragma unroll
-        for (int g = 0; g < kMaxGroup; ++g) {
+        for (int g = 0; g < MG; ++g) {
             if (g < group) {
                 float m = mw[g];
 #pragma unroll
@@ -305,7 +316,7 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attention_kernel(AttnArgs a) 
         }
     }
 #pragma unroll
-    for (int g = 0; g < kMaxGroup; ++g) {
+    for (int g = 0; g < MG; ++g) {
         if (g < group) {
             stv<E>(acc_lds[wave][g] + E * lane, acc[g]);
             if (lane == 0) {
@@ -320,8 +331,8 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attention_kernel(AttnArgs a) 
     // uniform per wave: head_dim is a multiple of 64, so a wave's 64 consecutive items
     // share one head, and __shfl never reads an inactive lane.)
     float wgt = 0.f, mg = -INFINITY;
-    if (lane < kAttnWaves * kMaxGroup) {
-        const int w = lane >> 3, g = lane & 7;
+    if (lane < kAttnWaves * MG) {
+        const int w = lane / MG, g = lane % MG;
         if (g < group) {
 #pragma unroll
             for (int v = 0; v < kAttnWaves; ++v) mg = fmaxf(mg, wstat[v][g][0]);
@@ -335,14 +346,14 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attention_kernel(AttnArgs a) 
         const int g = idx / HD, d = idx % HD;
         float o = 0.f;
 #pragma unroll
-        for (int w = 0; w < kAttnWaves; ++w) o = fmaf(__shfl(wgt, w * 8 + g, 64), acc_lds[w][g][d], o);
+        for (int w = 0; w < kAttnWaves; ++w) o = fmaf(__shfl(wgt, w * MG + g, 64), acc_lds[w][g][d], o);
         part[g * stride + d] = o;
     }
     if (wave == 0) {
-        const int g = lane < kMaxGroup ? lane : 0;
+        const int g = lane < MG ? lane : 0;
         float l = 0.f;
 #pragma unroll
-        for (int w = 0; w < kAttnWaves; ++w) l = fmaf(__shfl(wgt, w * 8 + g, 64), wstat[w][g][1], l);
+        for (int w = 0; w < kAttnWaves; ++w) l = fmaf(__shfl(wgt, w * MG + g, 64), wstat[w][g][1], l);
         const float m = __shfl(mg, g, 64);
         if (lane < group) {
             part[lane * stride + HD] = m;
@@ -353,14 +364,16 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attention_kernel(AttnArgs a) 
 
 // Merges the range partials of one query head and 64 of its output dims:
 // o = sum_c e^(m_c - M) o_c / sum_c e^(m_c - M) l_c, then the sigmoid output gate
-// (model.cpp:153). There are at most kAttnSplit partials, so every load -- the gate,
-// each wave's share of the o values (ranges w, w+4, ...), the statistics -- goes out
+// (model.cpp:153). The loads of the first kAttnFew partials -- the gate, each wave's share
+// of the o values (ranges w, w+4, ...), the statistics -- go out
 // together with the position's, before it is known which ranges hold positions (the
 // slots of the others are loaded but never used); the four waves' sums are added
 // through LDS. Loading only the ranges that hold positions makes those loads wait for
 // the position read: measured 1.2 us slower per call at 512 positions and 2.3 us at
 // 1024-4096 (graph replay), for half the merge's fetched bytes at 512.
-constexpr int kCombineBatch = kAttnSplit / 4;  // ranges per wave
+// Partials past kAttnFew exist only where they pay for that wait (attn_per).
+constexpr int kCombineBatch = kAttnFew / 4;  // ranges per wave
+static_assert(kAttnSplit == 2 * kAttnFew, "two batches");
 __global__ __launch_bounds__(256) void attention_combine_kernel(AttnArgs a) {
     __shared__ float wts[kAttnSplit];
     __shared__ float red[8];
@@ -377,12 +390,24 @@ __global__ __launch_bounds__(256) void attention_combine_kernel(AttnArgs a) {
     float ov[kCombineBatch];
 #pragma unroll
     for (int i = 0; i < kCombineBatch; ++i) ov[i] = base[(size_t)(wave + 4 * i) * cstride + d];
-    const int cs = min((int)threadIdx.x, kAttnSplit - 1);
-    const float m_c = base[(size_t)cs * cstride + hd], l_c = base[(size_t)cs * cstride + hd + 1];
+    const int cs = min((int)threadIdx.x, kAttnFew - 1);
+    float m_c = base[(size_t)cs * cstride + hd], l_c = base[(size_t)cs * cstride + hd + 1];
     if (pos < 0 || pos >= a.context) return;
-    const int nsub = pos / kAttnSub + 1, per = attn_per(pos + 1);
+    const int nsub = pos / kAttnSub + 1, per = attn_per(pos + 1, a.kv_heads);
     const int nchunks = (nsub + per - 1) / per;  // ranges holding positions
     const bool own = (int)threadIdx.x < nchunks;
+    float more[kCombineBatch];
+    if (nchunks > kAttnFew) {
+#pragma unroll
+        for (int i = 0; i < kCombineBatch; ++i) {
+            const int c = min(kAttnFew + wave + 4 * i, nchunks - 1);
+            more[i] = base[(size_t)c * cstride + d];
+        }
+        if (own && (int)threadIdx.x >= kAttnFew) {
+            m_c = base[(size_t)threadIdx.x * cstride + hd];
+            l_c = base[(size_t)threadIdx.x * cstride + hd + 1];
+        }
+    }
     const float mloc = wave_max(own ? m_c : -INFINITY);
     if (lane == 0) red[wave] = mloc;
     lds_barrier();
@@ -397,6 +422,13 @@ __global__ __launch_bounds__(256) void attention_combine_kernel(AttnArgs a) {
     for (int i = 0; i < kCombineBatch; ++i) {
         const int c = wave + 4 * i;
         if (c < nchunks) num = fmaf(wts[c], ov[i], num);
+    }
+    if (nchunks > kAttnFew) {
+#pragma unroll
+        for (int i = 0; i < kCombineBatch; ++i) {
+            const int c = kAttnFew + wave + 4 * i;
+            if (c < nchunks) num = fmaf(wts[c], more[i], num);
+        }
     }
     part[wave][lane] = num;
     lds_barrier();
@@ -975,18 +1007,21 @@ hipError_t launch_rope_table(float2* table, int context, int rotary, float base,
 }
 
 size_t attention_partial_floats(int heads, int kv_heads, int head_dim, int context) {
-    (void)context;  // the grid has kAttnSplit ranges at every context length
+    (void)context;  // (the combine kernel reads kAttnFew slots at every context length)
     return (size_t)kv_heads * kAttnSplit * (heads / kv_heads) * (head_dim + 2);
 }
 
 hipError_t launch_attention(const AttnArgs& a, hipStream_t stream) {
     if (a.heads % a.kv_heads || a.heads / a.kv_heads > kMaxGroup || a.rotary > a.head_dim || a.rotary % 2)
         return hipErrorInvalidValue;
-    const dim3 grid(a.kv_heads * kAttnSplit), block(kAttnWaves * 64);
+    // no more ranges than the caches have sub-chunks (2 KV heads x 64, 1024-position caches: 7.9 us
+    // at 16 positions, 8.5 with the empty ranges)
+    const dim3 grid(a.kv_heads * std::min(kAttnSplit, (a.context + kAttnSub - 1) / kAttnSub)), block(kAttnWaves * 64);
+    const bool few = a.heads / a.kv_heads <= 4;
     switch (a.head_dim) {
-    case 64: launch_kernel(attention_kernel<1>, grid, block, 0, stream, a); break;
-    case 128: launch_kernel(attention_kernel<2>, grid, block, 0, stream, a); break;
-    case 256: launch_kernel(attention_kernel<4>, grid, block, 0, stream, a); break;
+    case 64: launch_kernel(few ? attention_kernel<1, 4> : attention_kernel<1, 8>, grid, block, 0, stream, a); break;
+    case 128: launch_kernel(few ? attention_kernel<2, 4> : attention_kernel<2, 8>, grid, block, 0, stream, a); break;
+    case 256: launch_kernel(few ? attention_kernel<4, 4> : attention_kernel<4, 8>, grid, block, 0, stream, a); break;
     default: return hipErrorInvalidValue;
     }
     const hipError_t e = hipGetLastError();

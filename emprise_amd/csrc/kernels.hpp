@@ -198,7 +198,8 @@ struct AttnArgs {
     const float2* rope;  // [context][rotary / 2]: (cos, sin) of pos / base^(2i / rotary)
 };
 constexpr int kAttnSub = 16;     // positions per step of attention_kernel's online softmax
-constexpr int kAttnSplit = 64;   // position ranges (workgroups) per KV head of attention_kernel
+constexpr int kAttnSplit = 128;  // position ranges (workgroups) per KV head of attention_kernel, at most
+constexpr int kAttnFew = 64;     // those that a short context uses (attn_per)
 // `count` consecutive prompt positions from absolute position `first`: qkv row t at
 // t * stride floats; out row t at t * out_stride. Scratch: q (count x heads x hd floats);
 // per KV head and 32-key tile kf and vf (32 x hd x 2 halves each), ke (32 floats) and ve; for

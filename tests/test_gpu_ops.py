@@ -404,6 +404,19 @@ def test_attention_tiny(backend, L):
     _attention_case(backend, 8, 2, 64, 16, L, 512, seed=100 + L)
 
 
+# where the number of ranges changes (past 8192 positions; caches of at most 64 and 128
+# sub-chunks; fewer than 4 KV heads), with up to 4 and up to 8 query heads per KV head. One
+# rotated pair past 4096 positions: its angle is the position itself, where the others' differ
+# by L * 2^-23 (1e-3 at 8192) between two powf of one ulp
+@pytest.mark.parametrize("heads,kv,hd,rot,L,context", [(16, 4, 256, 2, 8192, 9000), (16, 4, 256, 2, 8193, 9000),
+                                                       (12, 4, 128, 32, 1100, 1101), (8, 2, 64, 16, 1024, 1024),
+                                                       (8, 2, 64, 16, 1025, 1040), (8, 2, 64, 16, 2049, 4096),
+                                                       (10, 2, 256, 64, 2500, 2500), (8, 1, 128, 2, 9000, 9001),
+                                                       (3, 1, 64, 2, 17, 20)])
+def test_attention_ranges(backend, heads, kv, hd, rot, L, context):
+    _attention_case(backend, heads, kv, hd, rot, L, context, seed=L)
+
+
 @pytest.mark.parametrize("heads,kv,hd,rot,first,count,context", [(16, 4, 256, 64, 0, 40, 4096),
                                                                 (16, 4, 256, 64, 100, 37, 4096),
                                                                 (8, 2, 64, 16, 0, 130, 512), (8, 2, 64, 16, 5, 1, 512)])
