@@ -130,7 +130,7 @@ __global__ __launch_bounds__(kGdnWaves * 64) void gdn_rows_kernel(GdnArgs a) {
 // (the ones before the prompt from the history), so the positions are independent:
 // thread = (channel, kConvSpan consecutive positions), channels across the threads of a
 // workgroup for coalesced rows. The sum runs in delta_conv_kernel's order, so the outputs
-// are its outputs bit for bit; the history moves on in delta_conv_history_kernel, once
+// are its outputs bit for bit; the history moves on in gdn_prep_batch_kernel, once
 // every read of the old one is done.
 constexpr int kConvSpan = 8;
 
@@ -160,21 +160,6 @@ __global__ __launch_bounds__(256) void delta_conv_batch_kernel(GdnBatchArgs a) {
             sum += y[u + CW - 1] * k[CW - 1];
             a.conv_out[(size_t)(t0 + u) * ch + c] = siluf_(sum);
         }
-    }
-}
-
-// The history after the prompt: the last CW inputs of (old history, prompt). One thread
-// per channel, ascending, so each old entry is read before its slot is overwritten.
-template <int CW>
-__global__ __launch_bounds__(256) void delta_conv_history_kernel(GdnBatchArgs a) {
-    const int c = blockIdx.x * 256 + threadIdx.x;
-    const int ch = 2 * a.key_heads * a.state_dim + a.value_heads * a.state_dim;
-    if (c >= ch) return;
-    float* hist = a.conv_state + (size_t)c * CW;
-#pragma unroll
-    for (int i = 0; i < CW; ++i) {
-        const int m = a.count - CW + i;
-        hist[i] = m >= 0 ? a.qkv[(size_t)m * a.stride + c] : hist[CW + m];
     }
 }
 
@@ -230,6 +215,16 @@ __global__ __launch_bounds__(256) void gdn_prep_batch_kernel(GdnBatchArgs a) {
         const int t = i / a.value_heads, h = i - t * a.value_heads;
         a.gates[2 * (size_t)i] = expf(a.ssm_a[h] * softplusf_(a.alpha[(size_t)t * a.stride + h] + a.dt[h]));
         a.gates[2 * (size_t)i + 1] = sigmoidf_(a.beta[(size_t)t * a.stride + h]);
+    }
+    // The conv history after the prompt: the last conv_width inputs of (old history, prompt).
+    // Ascending, so each old entry is read before its slot is overwritten.
+    const int c = blockIdx.x * 256 + threadIdx.x, cw = a.conv_width;
+    if (c < ch) {
+        float* hist = a.conv_state + (size_t)c * cw;
+        for (int n = 0; n < cw; ++n) {
+            const int m = a.count - cw + n;
+            hist[n] = m >= 0 ? a.qkv[(size_t)m * a.stride + c] : hist[cw + m];
+        }
     }
 }
 
@@ -349,11 +344,17 @@ __global__ __launch_bounds__(kScanWaves * 64) void gdn_scan_kernel(GdnBatchArgs 
 }
 
 // Per-head RMSNorm with ssm_norm, then SiLU(gate) (backend.cpp:57-58), as gdn_kernel's
-// epilogue; workgroup (position, head), one wave.
+// epilogue; one wave per (position, head), four to a workgroup. With this and the history's
+// move in the prep kernel instead of a launch of its own the 9B heads take 19.0 / 20.7 / 43.2 /
+// 132.3 us over 2 / 20 / 150 / 777 positions (21.1 / 22.3 / 44.8 / 133.4 before), 8 heads of 64
+// 14.7 / 16.6 / 27.3 / 79.9 (16.7 / 18.1 / 28.7 / 81.9).
+constexpr int kNormWaves = 4;
 template <int E>
-__global__ __launch_bounds__(64) void gdn_norm_gate_batch_kernel(GdnBatchArgs a) {
+__global__ __launch_bounds__(kNormWaves * 64) void gdn_norm_gate_batch_kernel(GdnBatchArgs a) {
     constexpr int SD = 64 * E;
-    const int t = blockIdx.x / a.value_heads, h = blockIdx.x - t * a.value_heads, lane = threadIdx.x;
+    const int pair = blockIdx.x * kNormWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (pair >= a.count * a.value_heads) return;
+    const int t = pair / a.value_heads, h = pair - t * a.value_heads, lane = threadIdx.x & 63;
     const float* o = a.o + (size_t)t * a.value_heads * SD + (size_t)h * SD;
     const float* gate = a.gate + (size_t)t * a.stride + (size_t)h * SD;
     float ov[E], ss = 0.f;
@@ -377,11 +378,10 @@ hipError_t launch_gdn_batch(const GdnBatchArgs& a, hipStream_t stream) {
     if (a.count < 1 || a.count > 65535 * kConvSpan || (a.state_dim != 64 && a.state_dim != 128))
         return hipErrorInvalidValue;
     const int ch = 2 * a.key_heads * a.state_dim + a.value_heads * a.state_dim;
-    const dim3 cgrid((ch + 255) / 256, (a.count + kConvSpan - 1) / kConvSpan), hgrid((ch + 255) / 256), cblock(256);
+    const dim3 cgrid((ch + 255) / 256, (a.count + kConvSpan - 1) / kConvSpan), cblock(256);
 #define EMPRISE_CONV_CASE(W)                                                              \
     case W:                                                                               \
         launch_kernel(delta_conv_batch_kernel<W>, cgrid, cblock, 0, stream, a);           \
-        launch_kernel(delta_conv_history_kernel<W>, hgrid, cblock, 0, stream, a);         \
         break;
     switch (a.conv_width) {
         EMPRISE_CONV_CASE(1)
@@ -397,7 +397,8 @@ hipError_t launch_gdn_batch(const GdnBatchArgs& a, hipStream_t stream) {
 #undef EMPRISE_CONV_CASE
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    const int pgrid = std::max((a.count * a.key_heads + 15) / 16, (a.count * a.value_heads + 255) / 256);
+    const int pgrid = std::max({(a.count * a.key_heads + 15) / 16, (a.count * a.value_heads + 255) / 256, (ch + 255) / 256});
+    const dim3 ngrid((a.count * a.value_heads + kNormWaves - 1) / kNormWaves), nblock(kNormWaves * 64);
     if (a.state_dim == 64) {
         launch_kernel(gdn_prep_batch_kernel<1>, dim3(pgrid), dim3(256), 0, stream, a);
         e = hipGetLastError();
@@ -406,7 +407,7 @@ hipError_t launch_gdn_batch(const GdnBatchArgs& a, hipStream_t stream) {
                       stream, a);
         e = hipGetLastError();
         if (e != hipSuccess) return e;
-        launch_kernel(gdn_norm_gate_batch_kernel<1>, dim3(a.count * a.value_heads), dim3(64), 0, stream, a);
+        launch_kernel(gdn_norm_gate_batch_kernel<1>, ngrid, nblock, 0, stream, a);
     } else {
         launch_kernel(gdn_prep_batch_kernel<2>, dim3(pgrid), dim3(256), 0, stream, a);
         e = hipGetLastError();
@@ -415,7 +416,7 @@ hipError_t launch_gdn_batch(const GdnBatchArgs& a, hipStream_t stream) {
                       stream, a);
         e = hipGetLastError();
         if (e != hipSuccess) return e;
-        launch_kernel(gdn_norm_gate_batch_kernel<2>, dim3(a.count * a.value_heads), dim3(64), 0, stream, a);
+        launch_kernel(gdn_norm_gate_batch_kernel<2>, ngrid, nblock, 0, stream, a);
     }
     return hipGetLastError();
 }
