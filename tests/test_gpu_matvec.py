@@ -628,3 +628,18 @@ def test_linear_unit_major_rows(backend, wtype, rows, cols):
         be.free(b)
     for q in (w, w2, nwd, dw):
         be.weight_free(q)
+
+
+def test_lm_head_is_right_on_a_new_backend():
+    """The argmax key is scratch that a backend's first call allocates and clears."""
+    from emprise_amd import HipBackend
+
+    rng = np.random.default_rng(4)
+    rows, cols = 5, 256
+    data, x = matrix(rng, Q6_K, rows, cols), rng.standard_normal(cols).astype(np.float32)
+    for _ in range(4):
+        with HipBackend() as be:
+            w = be.upload_weight(Q6_K, cols, rows, data)
+            xd, y, idx = be.to_device(x), be.alloc(rows * 4), be.alloc(4)
+            be.lm_head(Input(xd, 0, 0, be.vector(np.ones(cols, np.float32)), 1e-6), w, y, idx)
+            assert int(be.download(idx, 1, np.int32)[0]) == int(np.argmax(be.download(y, rows)))
