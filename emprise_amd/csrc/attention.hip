@@ -656,7 +656,11 @@ __global__ __launch_bounds__(TH, 2) void attn_flash_kernel(AttnBatchArgs a) {
     constexpr int NS = HD / 32, ND = HD / 16, QT = kFlashQT, PD = 2;
     constexpr int AV = kKeyTile * HD * 4 / 16;  // 16-byte pieces of a tile's keys (and of its values)
     constexpr int AN = AV / TH;
-    __shared__ __align__(16) u32x4v Ks[2][AV], Vs[2][AV];
+    // keys of two tiles, values of two tiles; at the end one array for the outputs of all waves
+    __shared__ __align__(16) u32x4v KV[4][AV];
+    static_assert(sizeof(KV) >= (size_t)kFlashRows * HD * sizeof(float), "outputs in KV");
+    u32x4v(*const Ks)[AV] = KV;
+    u32x4v(*const Vs)[AV] = KV + 2;
     __shared__ __align__(16) float Es[2][kKeyTile + 4];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = lane >> 4, qj = lane & 15;
@@ -912,7 +916,7 @@ __global__ __launch_bounds__(TH, 2) void attn_flash_kernel(AttnBatchArgs a) {
     }
     // through this wave's share of LDS, row by row: consecutive lanes write consecutive dims, and
     // the gate's code stands here once (unrolled over the outputs it was 30 KB)
-    float* tile = reinterpret_cast<float*>(Ks) + wave * (16 * HD);
+    float* tile = reinterpret_cast<float*>(KV) + wave * (16 * HD);
 #pragma unroll
     for (int u = 0; u < QT; ++u) {
 #pragma unroll
