@@ -461,22 +461,22 @@ __global__ __launch_bounds__(256) void rope_table_kernel(float2* t, int context,
 // (model.cpp:129-157). With few query rows the keys are split over workgroups and
 // attn_merge_batch_kernel joins their partial results.
 //
-// The products run on the fp16 matrix cores from two fp16 pieces per FP32 operand, as the
-// quantised GEMM's activations do: x = 2^e (xh + xl), 22 significant bits, the exponent e
-// taken per query and per key (from the largest of its head_dim values) and per 32-key tile
-// of values, three products of four (xl yl is below 2^-22 of its term), FP32 sums. Each
-// product has 16 queries on the lane index: S^T = K Q^T leaves lane (query l%16, group g =
-// l/16) the scores of keys 4g .. 4g+3 of two 16-key halves, which is the operand of O^T =
-// V^T P^T if V^T lists the 32 keys in that order -- so it does, and P goes from one product
-// to the next in registers. The probabilities are carried as 2^6 p relative to a
-// reference that the row maximum may pass by 2^8, above fp16's subnormals for p down to
-// 2^-20 of it.
+// Scores run on the fp16 matrix cores from two fp16 pieces per FP32 operand: x = 2^e (xh +
+// xl), 22 significant bits, e taken per query and per key (from the largest of its head_dim
+// values), three products of four (xl yl is below 2^-22 of its term), FP32 sums. P.V carries P
+// and V whole, as three bf16 pieces of 8 bits each (with FP32's range, so it does not matter how the values' sizes differ), in the six products above 2^-24 of their
+// term, a tile's summed apart from O. Each product has 16 queries on the lane index: S^T = K Q^T
+// leaves lane (query l%16, group g = l/16) the scores of keys 4g .. 4g+3 of two 16-key halves,
+// which is the operand of O^T = V^T P^T if V^T lists the 32 keys in that order -- so it does, and
+// P goes from one product to the next in registers.
 //
-// Bound by the matrix cores: 2048 positions behind 4096 of the 9B shape (16 Q / 4 KV heads x
-// 256) are 172 GFLOP, three times that in fp16 products; 582 us for all the kernels here
-// (885 TFLOP/s of products), of which the split 20 and the prep 20. As two FP32 GEMMs per
-// head with the scores in memory and a softmax pass between them it took 2570 us and 805 MB
-// of scratch; its error against 64 bits was 1.4e-6, now 8.8e-7 (relative, whole output).
+// Bound by the matrix cores and, about as much, by LDS reads (80 KiB per wave and tile): 2048
+// positions behind 4096 of the 9B shape (16 Q / 4 KV heads x 256) are 172 GFLOP, four and a half
+// times that in 16-bit products; 733 us for all the kernels here, of which the split 21 and the
+// prep 24. As two FP32 GEMMs per head with the scores in memory and a softmax pass between them it
+// took 2570 us and 805 MB of scratch, with 1.4e-6 of error against 64 bits, now 4e-7 (relative,
+// whole output). P.V from two fp16 pieces with an exponent per tile of values took 579 us, with
+// 8.8e-7, but lost all digits of values much smaller than others in their tile or before it.
 
 // Workgroup = one position; wave w normalises head vectors w, w+8, ... of the group's
 // q heads (all kv heads' groups) and the kv heads' new keys.
@@ -524,14 +524,14 @@ __global__ __launch_bounds__(512) void attn_prep_batch_kernel(AttnBatchArgs a) {
 }
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
 
 constexpr int kKeyTile = kAttnKeyTile;
 constexpr int kFlashRows = 128;  // query rows (position x head of a KV head's group) per workgroup
-constexpr int kFlashQT = 1;      // 16-row query tiles per wave
-constexpr float kBase = 6.f;     // P is carried as 2^kBase p, p <= 2^kLag
-constexpr float kLag = 8.f;
+constexpr int kFlashThreads = 64 * kFlashRows / 16;
+constexpr float kLag = 8.f;      // a row's maximum may pass its reference by this (powers of two)
 
 // The exponent that brings a vector of largest magnitude mx to [2^12, 2^13).
 __device__ __forceinline__ int piece_exp(float mx) {
@@ -549,6 +549,27 @@ __device__ __forceinline__ void split8(const float (&v)[8], float up, half8& hi,
         hi[k] = (_Float16)w;
         lo[k] = (_Float16)(w - (float)hi[k]);
     }
+}
+// x = p0 + p1 + p2, each the next 8 significant bits of it as bf16 (a NaN stays one; an
+// infinity becomes one).
+__device__ __forceinline__ void split3(const float (&v)[8], bf16x8 (&p)[3]) {
+    uint32_t w[3][4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        uint32_t b[3][2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const float x = v[2 * k + i];
+            b[0][i] = __float_as_uint(x);
+            const float r = x - __uint_as_float(b[0][i] & 0xffff0000u);
+            b[1][i] = __float_as_uint(r);
+            b[2][i] = __float_as_uint(r - __uint_as_float(b[1][i] & 0xffff0000u));
+        }
+#pragma unroll
+        for (int n = 0; n < 3; ++n) w[n][k] = __builtin_amdgcn_perm(b[n][1], b[n][0], 0x07060302u);  // the upper halves
+    }
+#pragma unroll
+    for (int n = 0; n < 3; ++n) p[n] = __builtin_bit_cast(bf16x8, u32x4v{w[n][0], w[n][1], w[n][2], w[n][3]});
 }
 
 // Maximum / sum over lanes l, l^16, l^32, l^48 (the lane groups that share a query).
@@ -568,13 +589,11 @@ __device__ __forceinline__ float sum_groups(float x) {
 // Operands of the keys and values of one 32-key tile of one KV head (rows past the last
 // key are zero). Keys: half kt, slice s (32 dims), piece p, lane (key l%16, dims 8(l/16) ..
 // +7) -> ((kt*HD/32 + s)*2 + p)*512 + 8l halves, 2^e per key in ke. Values: dims tile dt,
-// piece p, lane (dim l%16, g) -> (dt*2 + p)*512 + 8l: keys 4g .. 4g+3, 16+4g .. 16+4g+3;
-// the tile's e in ve.
+// piece p, lane (dim l%16, g) -> (dt*3 + p)*512 + 8l: keys 4g .. 4g+3, 16+4g .. 16+4g+3.
 template <int HD>
 __global__ __launch_bounds__(256) void attn_split_kv_kernel(AttnBatchArgs a) {
     constexpr int CK = HD / 64;            // 8-dim pieces of a key per thread
     constexpr int CV = HD / 64;            // (dims tile, lane) items per thread
-    __shared__ float red[4];
     const int tile = blockIdx.x, kvh = blockIdx.y, tid = threadIdx.x;
     const int L = a.first + a.count, kvd = a.kv_heads * HD, tiles = (L + kKeyTile - 1) / kKeyTile;
     const size_t at = (size_t)kvh * tiles + tile;
@@ -610,32 +629,21 @@ __global__ __launch_bounds__(256) void attn_split_kv_kernel(AttnBatchArgs a) {
             *reinterpret_cast<half8*>(dst + (c >> 2) * 1024 + 512 + lane * 8) = lo;
         }
     }
-    float v[CV][8], mx = 0.f;
+    uint16_t* dst = a.vf + at * (kKeyTile * HD * 3);
 #pragma unroll
     for (int i = 0; i < CV; ++i) {
         const int item = i * 256 + tid, dt = item >> 6, lane = item & 63, g = lane >> 4;
+        float v[8];
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
             const int pos = tile * kKeyTile + (k >> 2) * 16 + 4 * g + (k & 3);
             const float x = a.values[(size_t)min(pos, L - 1) * kvd + (size_t)kvh * HD + dt * 16 + (lane & 15)];
-            v[i][k] = pos < L ? x : 0.f;
-            mx = fmaxf(mx, fabsf(v[i][k]));
+            v[k] = pos < L ? x : 0.f;
         }
-    }
-    mx = wave_max(mx);
-    if ((tid & 63) == 0) red[tid >> 6] = mx;
-    __syncthreads();
-    const int e = piece_exp(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
-    const float up = ldexpf(1.f, -e);
-    if (tid == 0) a.ve[at] = e;
-    _Float16* dst = reinterpret_cast<_Float16*>(a.vf) + at * (kKeyTile * HD * 2);
+        bf16x8 p[3];
+        split3(v, p);
 #pragma unroll
-    for (int i = 0; i < CV; ++i) {
-        const int item = i * 256 + tid, dt = item >> 6, lane = item & 63;
-        half8 hi, lo;
-        split8(v[i], up, hi, lo);
-        *reinterpret_cast<half8*>(dst + dt * 1024 + lane * 8) = hi;
-        *reinterpret_cast<half8*>(dst + dt * 1024 + 512 + lane * 8) = lo;
+        for (int n = 0; n < 3; ++n) *reinterpret_cast<bf16x8*>(dst + (dt * 3 + n) * 512 + lane * 8) = p[n];
     }
 }
 
@@ -649,19 +657,16 @@ __device__ __forceinline__ int flash_tiles(const AttnBatchArgs& a, int rows, int
 // over the key tiles of one split: 8 waves of 16 rows, queries and outputs in registers, the
 // tile's key and value operands shared through LDS, double-buffered. (Four waves of 32 rows
 // with 512 registers read half as much LDS but leave one wave per SIMD, with nothing beside
-// its softmax and its waits: 843 us against 660 at that stage; reading an operand further
-// ahead of its products, or pinning vector instructions between the products, no faster.)
-template <int HD, int TH = 64 * kFlashRows / 16 / kFlashQT>
-__global__ __launch_bounds__(TH, 2) void attn_flash_kernel(AttnBatchArgs a) {
-    constexpr int NS = HD / 32, ND = HD / 16, QT = kFlashQT, PD = 2;
-    constexpr int AV = kKeyTile * HD * 4 / 16;  // 16-byte pieces of a tile's keys (and of its values)
-    constexpr int AN = AV / TH;
+// its softmax and its waits: 843 us against 660 at that stage.)
+template <int HD>
+__global__ __launch_bounds__(kFlashThreads, 2) void attn_flash_kernel(AttnBatchArgs a) {
+    constexpr int TH = kFlashThreads, NS = HD / 32, ND = HD / 16;
+    constexpr int KN = kKeyTile * HD * 4 / 16, VN = kKeyTile * HD * 6 / 16;  // 16-byte pieces of a tile's keys, values
+    constexpr int KL = KN / TH, VL = (VN + TH - 1) / TH;
+    constexpr int KD = 1, VD = 3;  // operands are read this many steps ahead of their products
     // keys of two tiles, values of two tiles; at the end one array for the outputs of all waves
-    __shared__ __align__(16) u32x4v KV[4][AV];
+    __shared__ __align__(16) u32x4v KV[2 * KN + 2 * VN];
     static_assert(sizeof(KV) >= (size_t)kFlashRows * HD * sizeof(float), "outputs in KV");
-    u32x4v(*const Ks)[AV] = KV;
-    u32x4v(*const Vs)[AV] = KV + 2;
-    __shared__ __align__(16) float Es[2][kKeyTile + 4];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = lane >> 4, qj = lane & 15;
     const int kvh = blockIdx.x, group = a.heads / a.kv_heads, rows = a.count * group;
@@ -671,49 +676,42 @@ __global__ __launch_bounds__(TH, 2) void attn_flash_kernel(AttnBatchArgs a) {
     const int halves = (rows + kFlashRows / 2 - 1) / (kFlashRows / 2), far = halves - 1 - (int)blockIdx.y;
     const bool near = wave < TH / 128;
     const int half = near ? (int)blockIdx.y : far;
-    const int row0 = half * (kFlashRows / 2) + (near ? wave : wave - TH / 128) * 16 * QT;
+    const int row0 = half * (kFlashRows / 2) + (near ? wave : wave - TH / 128) * 16;
     const int tile0 = blockIdx.z * a.split_tiles;
     const int tile1 = min(flash_tiles(a, rows, far), tile0 + a.split_tiles);
     if (tile0 >= tile1) return;
     const int mine = min(tile1, flash_tiles(a, rows, half));  // this wave's last tile
     const bool active = row0 < rows && tile0 < mine && !(near && half == far);
 
-    const u32x4v* kf = reinterpret_cast<const u32x4v*>(a.kf) + (size_t)kvh * tiles_all * AV;
-    const u32x4v* vf = reinterpret_cast<const u32x4v*>(a.vf) + (size_t)kvh * tiles_all * AV;
-    u32x4v rk[AN], rv[AN];
-    float re = 0.f;
+    const u32x4v* kf = reinterpret_cast<const u32x4v*>(a.kf) + (size_t)kvh * tiles_all * KN;
+    const u32x4v* vf = reinterpret_cast<const u32x4v*>(a.vf) + (size_t)kvh * tiles_all * VN;
+    u32x4v rk[KL], rv[VL];
     auto load_keys = [&](int tile) {
 #pragma unroll
-        for (int k = 0; k < AN; ++k) rk[k] = kf[(size_t)tile * AV + k * TH + tid];
-        // their 2^e and, 33rd, the exponent of the tile's values
-        const size_t at = (size_t)kvh * tiles_all + tile;
-        if (tid < kKeyTile) re = a.ke[at * kKeyTile + tid];
-        else if (tid == kKeyTile) re = (float)a.ve[at];
+        for (int k = 0; k < KL; ++k) rk[k] = kf[(size_t)tile * KN + k * TH + tid];
     };
     auto load_values = [&](int tile) {
 #pragma unroll
-        for (int k = 0; k < AN; ++k) rv[k] = vf[(size_t)tile * AV + k * TH + tid];
+        for (int k = 0; k < VL; ++k) rv[k] = vf[(size_t)tile * VN + min(k * TH + tid, VN - 1)];
     };
     auto store_keys = [&](int b) {
 #pragma unroll
-        for (int k = 0; k < AN; ++k) Ks[b][k * TH + tid] = rk[k];
-        if (tid <= kKeyTile) Es[b][tid] = re;
+        for (int k = 0; k < KL; ++k) KV[b * KN + k * TH + tid] = rk[k];
     };
     auto store_values = [&](int b) {
 #pragma unroll
-        for (int k = 0; k < AN; ++k) Vs[b][k * TH + tid] = rv[k];
+        for (int k = 0; k < VL; ++k)
+            if (VN % TH == 0 || k * TH + tid < VN) KV[2 * KN + b * VN + k * TH + tid] = rv[k];
     };
     load_keys(tile0);
     load_values(tile0);
 
     // the wave's queries as operands: lane (query l%16, dims 32s + 8g .. +7)
-    half8 qh[QT][NS], ql[QT][NS];
-    float qs[QT];  // 2^e / sqrt(head_dim) * log2(e): scores in units of log 2
-    int last[QT];  // the query's last key
-#pragma unroll
-    for (int u = 0; u < QT; ++u) {
-        const int r = min(row0 + 16 * u + qj, rows - 1), t = r / group, h = kvh * group + (r - t * group);
-        last[u] = a.first + t;
+    half8 qh[NS], ql[NS];
+    float qs;                                      // 2^e / sqrt(head_dim) * log2(e): scores in units of log 2
+    const int row = min(row0 + qj, rows - 1), last = a.first + row / group;  // the query's last key
+    {
+        const int t = row / group, h = kvh * group + (row - t * group);
         const float* src = a.q + ((size_t)t * a.heads + h) * HD + 8 * g;
         float v[NS][8], mx = 0.f;
 #pragma unroll
@@ -730,86 +728,71 @@ __global__ __launch_bounds__(TH, 2) void attn_flash_kernel(AttnBatchArgs a) {
         const int e = piece_exp(max_groups(mx));
         const float up = ldexpf(1.f, -e);
 #pragma unroll
-        for (int s = 0; s < NS; ++s) split8(v[s], up, qh[u][s], ql[u][s]);
-        qs[u] = ldexpf(1.44269504088896340736f / sqrtf((float)HD), e);
+        for (int s = 0; s < NS; ++s) split8(v[s], up, qh[s], ql[s]);
+        qs = ldexpf(1.44269504088896340736f / sqrtf((float)HD), e);
     }
 
-    // S^T of a tile's two key halves
-    auto scores = [&](const u32x4v* keys, floatx4 (&S)[2][QT]) {
-        const half8* K = reinterpret_cast<const half8*>(keys);
+    // a tile's scores in log 2 units (S^T of its two key halves), masked, and their maximum
+    float x[8], mx;
+    float4 ke[2];  // the tile's 2^e
+    auto load_scales = [&](int tile) {
+        const float* e = a.ke + ((size_t)kvh * tiles_all + tile) * kKeyTile + 4 * g;
+        ke[0] = *reinterpret_cast<const float4*>(e);
+        ke[1] = *reinterpret_cast<const float4*>(e + 16);
+    };
+    auto scores = [&](int b, floatx4 (&S)[2]) {
+        const half8* K = reinterpret_cast<const half8*>(KV + b * KN);
 #pragma unroll
-        for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-            for (int u = 0; u < QT; ++u) S[kt][u] = floatx4{0.f, 0.f, 0.f, 0.f};
-        half8 kh[PD + 1][2], kl[PD + 1][2];  // slices read PD ahead of their products
+        for (int kt = 0; kt < 2; ++kt) S[kt] = floatx4{0.f, 0.f, 0.f, 0.f};
+        half8 kh[KD + 1][2], kl[KD + 1][2];
         auto operands = [&](int s) {
 #pragma unroll
             for (int kt = 0; kt < 2; ++kt) {
-                kh[s % (PD + 1)][kt] = K[((kt * NS + s) * 2) * 64 + lane];
-                kl[s % (PD + 1)][kt] = K[((kt * NS + s) * 2 + 1) * 64 + lane];
+                kh[s % (KD + 1)][kt] = K[((kt * NS + s) * 2) * 64 + lane];
+                kl[s % (KD + 1)][kt] = K[((kt * NS + s) * 2 + 1) * 64 + lane];
             }
         };
 #pragma unroll
-        for (int s = 0; s < PD && s < NS; ++s) operands(s);
+        for (int s = 0; s < KD && s < NS; ++s) operands(s);
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
-            if (s + PD < NS) operands(s + PD);
-            const int b = s % (PD + 1);
+            if (s + KD < NS) operands(s + KD);
+            const int r = s % (KD + 1);
 #pragma unroll
-            for (int kt = 0; kt < 2; ++kt)
+            for (int kt = 0; kt < 2; ++kt) S[kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kl[r][kt], qh[s], S[kt], 0, 0, 0);
 #pragma unroll
-                for (int u = 0; u < QT; ++u) S[kt][u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kl[b][kt], qh[u][s], S[kt][u], 0, 0, 0);
+            for (int kt = 0; kt < 2; ++kt) S[kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh[r][kt], ql[s], S[kt], 0, 0, 0);
 #pragma unroll
-            for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-                for (int u = 0; u < QT; ++u) S[kt][u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh[b][kt], ql[u][s], S[kt][u], 0, 0, 0);
-#pragma unroll
-            for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-                for (int u = 0; u < QT; ++u) S[kt][u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh[b][kt], qh[u][s], S[kt][u], 0, 0, 0);
-            if (s + PD < NS) __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);  // LDS reads, then
-            __builtin_amdgcn_sched_group_barrier(0x008, 6 * QT, 0);             // products
+            for (int kt = 0; kt < 2; ++kt) S[kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh[r][kt], qh[s], S[kt], 0, 0, 0);
+            if (s + KD < NS) __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);  // LDS reads, then
+            __builtin_amdgcn_sched_group_barrier(0x008, 6, 0);                  // products
         }
     };
-
-    // a tile's scores in log 2 units, masked, their maximum, and the exponent of its values
-    float x[QT][8], mx[QT];
-    int ev = 0;
-    auto scaled = [&](const floatx4 (&S)[2][QT], int tile, const float* E) {
-        const float4 k0 = *reinterpret_cast<const float4*>(E + 4 * g), k1 = *reinterpret_cast<const float4*>(E + 16 + 4 * g);
-        const float ke[8] = {k0.x, k0.y, k0.z, k0.w, k1.x, k1.y, k1.z, k1.w};
+    auto scaled = [&](const floatx4 (&S)[2], int tile) {
+        const float e[8] = {ke[0].x, ke[0].y, ke[0].z, ke[0].w, ke[1].x, ke[1].y, ke[1].z, ke[1].w};
         const int key0 = tile * kKeyTile + 4 * g;
-        ev = (int)E[kKeyTile];
+        mx = -INFINITY;
 #pragma unroll
-        for (int u = 0; u < QT; ++u) {
-            mx[u] = -INFINITY;
-#pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                x[u][k] = key0 + (k >> 2) * 16 + (k & 3) <= last[u] ? (S[k >> 2][u][k & 3] * ke[k]) * qs[u] : -INFINITY;
-                mx[u] = fmaxf(mx[u], x[u][k]);
-            }
-            mx[u] = max_groups(mx[u]);
+        for (int k = 0; k < 8; ++k) {
+            x[k] = key0 + (k >> 2) * 16 + (k & 3) <= last ? (S[k >> 2][k & 3] * e[k]) * qs : -INFINITY;
+            mx = fmaxf(mx, x[k]);
         }
+        mx = max_groups(mx);
     };
 
-    floatx4 O[ND][QT], S[2][QT];
-    float m[QT], l[QT];  // the reference that scores are taken against, and the sum of 2^(score - m + kBase)
+    floatx4 O[ND], S[2];
+    float m = -INFINITY, l = 0.f;  // the reference of the scores, a whole number; the sum of 2^(score - m - kLag)
 #pragma unroll
-    for (int u = 0; u < QT; ++u) {
-        m[u] = -INFINITY;
-        l[u] = 0.f;
-#pragma unroll
-        for (int d = 0; d < ND; ++d) O[d][u] = floatx4{0.f, 0.f, 0.f, 0.f};
-    }
-    int eo = -1000;  // O holds 2^-eo times its value
+    for (int d = 0; d < ND; ++d) O[d] = floatx4{0.f, 0.f, 0.f, 0.f};
+    load_scales(tile0);
     store_keys(0);
     store_values(0);
     load_keys(min(tile0 + 1, tile1 - 1));
     load_values(min(tile0 + 1, tile1 - 1));
     lds_barrier();
     if (active) {
-        scores(Ks[0], S);
-        scaled(S, tile0, Es[0]);
+        scores(0, S);
+        scaled(S, tile0);
     }
     store_keys(1);
     load_keys(min(tile0 + 2, tile1 - 1));
@@ -824,73 +807,57 @@ __global__ __launch_bounds__(TH, 2) void attn_flash_kernel(AttnBatchArgs a) {
         load_keys(min(tile + 3, tile1 - 1));
         load_values(min(tile + 2, tile1 - 1));
         if (active && tile < mine) {
-            const half8* V = reinterpret_cast<const half8*>(Vs[buf]);
-            // m follows the maximum only where that passes it by kLag (P then stays within fp16),
-            // so O is seldom rescaled
-            bool up = ev > eo;
+            load_scales(min(tile + 1, tile1 - 1));
+            const bf16x8* V = reinterpret_cast<const bf16x8*>(KV + 2 * KN + buf * VN);
+            // m follows the maximum only where that passes it by kLag, so O is seldom rescaled;
+            // as a whole number it makes the rescaling exact
+            if (__ballot(mx > m + kLag)) {
+                const float mn = mx > m + kLag ? ceilf(mx) : m;
+                const float f = mn == m ? 1.f : __builtin_amdgcn_exp2f(m - mn);
+                m = mn;
+                l *= f;
 #pragma unroll
-            for (int u = 0; u < QT; ++u) up = up || mx[u] > m[u] + kLag;
-            if (__ballot(up)) {
-                const int en = max(eo, ev);
-                const float od = ldexpf(1.f, max(eo - en, -200));
-                eo = en;
-#pragma unroll
-                for (int u = 0; u < QT; ++u) {
-                    const float mn = mx[u] > m[u] + kLag ? mx[u] : m[u];
-                    const float f = mn == m[u] ? 1.f : __builtin_amdgcn_exp2f(m[u] - mn);
-                    m[u] = mn;
-                    l[u] *= f;
-#pragma unroll
-                    for (int d = 0; d < ND; ++d) O[d][u] *= f * od;
-                }
+                for (int d = 0; d < ND; ++d) O[d] *= f;
             }
-            const float pv = ldexpf(1.f, ev - eo);
-            half8 ph[QT], pl[QT];
+            const float off = m == -INFINITY ? 0.f : -kLag - m;  // (no key of the row yet: all x are -inf)
+            bf16x8 P[3];
+            {
+                float p[8], sum = 0.f;
 #pragma unroll
-            for (int u = 0; u < QT; ++u) {
-                const float off = m[u] == -INFINITY ? 0.f : kBase - m[u];  // (no key of the row yet: all x are -inf)
-                float sum = 0.f;
-#pragma unroll
-                for (int k = 0; k < 8; ++k) {
-                    const float p = __builtin_amdgcn_exp2f(x[u][k] + off);
-                    sum += p;
-                    const float w = p * pv;
-                    ph[u][k] = (_Float16)w;
-                    pl[u][k] = (_Float16)(w - (float)ph[u][k]);
-                }
-                l[u] += sum;
+                for (int k = 0; k < 8; ++k) sum += p[k] = __builtin_amdgcn_exp2f(x[k] + off);
+                l += sum;
+                split3(p, P);
             }
-            scores(Ks[buf ^ 1], S);
-            scaled(S, tile + 1, Es[buf ^ 1]);
-            // two dims tiles at a time, read PD pairs ahead
-            half8 vh[PD + 1][2], vl[PD + 1][2];
-            auto operands = [&](int d) {
+            scores(buf ^ 1, S);
+            scaled(S, tile + 1);
+            // P.V of two dims tiles at a time: the products of pieces i and j for i + j <= 2, the
+            // smallest first, in a sum of their own, so that O is rounded once per tile; step
+            // (d, n) uses piece 2 - n of the values
+            floatx4 T[2];
+            bf16x8 v[VD + 1][2];
+            auto operands = [&](int i) {
 #pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    vh[d % (PD + 1)][i] = V[((2 * d + i) * 2) * 64 + lane];
-                    vl[d % (PD + 1)][i] = V[((2 * d + i) * 2 + 1) * 64 + lane];
-                }
+                for (int u = 0; u < 2; ++u) v[i % (VD + 1)][u] = V[((2 * (i / 3) + u) * 3 + 2 - i % 3) * 64 + lane];
             };
+            constexpr int N = 3 * (ND / 2);
 #pragma unroll
-            for (int d = 0; d < PD && d < ND / 2; ++d) operands(d);
+            for (int i = 0; i < VD && i < N; ++i) operands(i);
 #pragma unroll
-            for (int d = 0; d < ND / 2; ++d) {
-                if (d + PD < ND / 2) operands(d + PD);
-                const int b = d % (PD + 1);
+            for (int i = 0; i < N; ++i) {
+                if (i + VD < N) operands(i + VD);
 #pragma unroll
-                for (int i = 0; i < 2; ++i)
+                for (int n = i % 3; n >= 0; --n)
 #pragma unroll
-                    for (int u = 0; u < QT; ++u) O[2 * d + i][u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl[b][i], ph[u], O[2 * d + i][u], 0, 0, 0);
+                    for (int u = 0; u < 2; ++u)
+                        T[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v[i % (VD + 1)][u], P[n], i % 3 ? T[u] : floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                if (i % 3 == 2) {
 #pragma unroll
-                for (int i = 0; i < 2; ++i)
-#pragma unroll
-                    for (int u = 0; u < QT; ++u) O[2 * d + i][u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh[b][i], pl[u], O[2 * d + i][u], 0, 0, 0);
-#pragma unroll
-                for (int i = 0; i < 2; ++i)
-#pragma unroll
-                    for (int u = 0; u < QT; ++u) O[2 * d + i][u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh[b][i], ph[u], O[2 * d + i][u], 0, 0, 0);
-                if (d + PD < ND / 2) __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
-                __builtin_amdgcn_sched_group_barrier(0x008, 6 * QT, 0);
+                    for (int u = 0; u < 2; ++u) O[2 * (i / 3) + u] += T[u];
+                }
+                if (i + VD < N) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+                if (i % 3 == 0) __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+                else if (i % 3 == 1) __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+                else __builtin_amdgcn_sched_group_barrier(0x008, 6, 0);
             }
         }
         lds_barrier();
@@ -898,52 +865,42 @@ __global__ __launch_bounds__(TH, 2) void attn_flash_kernel(AttnBatchArgs a) {
     if (!active) return;
 
     // lane: query l%16, dims 16d + 4g .. +3
-    float total[QT];
-#pragma unroll
-    for (int u = 0; u < QT; ++u) total[u] = sum_groups(l[u]);
+    const float total = sum_groups(l);
     if (gridDim.z > 1) {
+        if (row0 + qj >= rows) return;
+        const size_t at = ((size_t)blockIdx.z * a.kv_heads + kvh) * rows + row;
+        float* dst = a.part + at * HD;
 #pragma unroll
-        for (int u = 0; u < QT; ++u) {
-            const int r = row0 + 16 * u + qj;
-            if (r >= rows) continue;
-            const size_t at = ((size_t)blockIdx.z * a.kv_heads + kvh) * rows + r;
-            float* dst = a.part + at * HD;
-#pragma unroll
-            for (int d = 0; d < ND; ++d) *reinterpret_cast<floatx4*>(dst + 16 * d + 4 * g) = O[d][u];
-            if (g == 0) *reinterpret_cast<floatx4*>(a.stat + at * 4) = floatx4{m[u], total[u], (float)eo, 0.f};
-        }
+        for (int d = 0; d < ND; ++d) *reinterpret_cast<floatx4*>(dst + 16 * d + 4 * g) = O[d];
+        if (g == 0) *reinterpret_cast<float2*>(a.stat + at * 2) = make_float2(m, total);
         return;
     }
     // through this wave's share of LDS, row by row: consecutive lanes write consecutive dims, and
     // the gate's code stands here once (unrolled over the outputs it was 30 KB)
     float* tile = reinterpret_cast<float*>(KV) + wave * (16 * HD);
 #pragma unroll
-    for (int u = 0; u < QT; ++u) {
+    for (int d = 0; d < ND; ++d) {
+        floatx4 o;
 #pragma unroll
-        for (int d = 0; d < ND; ++d) {
-            floatx4 o;
-#pragma unroll
-            for (int k = 0; k < 4; ++k) o[k] = ldexpf(O[d][u][k] / total[u], eo);
-            *reinterpret_cast<floatx4*>(tile + qj * HD + 16 * d + 4 * g) = o;
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        const int n = min(16, rows - row0 - 16 * u);
+        for (int k = 0; k < 4; ++k) o[k] = O[d][k] / total;
+        *reinterpret_cast<floatx4*>(tile + qj * HD + 16 * d + 4 * g) = o;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const int n = min(16, rows - row0);
 #pragma unroll 1
-        for (int i = 0; i < n; ++i) {
-            const int r = row0 + 16 * u + i, t = r / group, h = kvh * group + (r - t * group);
-            const float* gate = a.qkv + (size_t)t * a.stride + (size_t)h * HD * 2 + HD;
-            float* dst = a.out + (size_t)t * a.out_stride + (size_t)h * HD;
+    for (int i = 0; i < n; ++i) {
+        const int r = row0 + i, t = r / group, h = kvh * group + (r - t * group);
+        const float* gate = a.qkv + (size_t)t * a.stride + (size_t)h * HD * 2 + HD;
+        float* dst = a.out + (size_t)t * a.out_stride + (size_t)h * HD;
 #pragma unroll
-            for (int c = lane; c < HD; c += 64) dst[c] = tile[i * HD + c] * sigmoidf_(gate[c]);
-        }
-        if (u + 1 < QT) __builtin_amdgcn_wave_barrier();
+        for (int c = lane; c < HD; c += 64) dst[c] = tile[i * HD + c] * sigmoidf_(gate[c]);
     }
 }
 
 // Joins the splits of one query row (workgroup = KV head x row, a thread per dim): sum_s
-// 2^(m_s - M + eo_s) O_s / sum_s 2^(m_s - M) l_s, then the sigmoid gate. A split whose keys
+// 2^(m_s - M) O_s / sum_s 2^(m_s - M) l_s, then the sigmoid gate. A split whose keys
 // all lie past those of the row's half-tile was not run.
 __global__ __launch_bounds__(256) void attn_merge_batch_kernel(AttnBatchArgs a, int splits) {
     const int hd = a.head_dim, group = a.heads / a.kv_heads, rows = a.count * group;
@@ -952,13 +909,13 @@ __global__ __launch_bounds__(256) void attn_merge_batch_kernel(AttnBatchArgs a, 
     const int n = min(splits, (flash_tiles(a, rows, r / (kFlashRows / 2)) + a.split_tiles - 1) / a.split_tiles);
     const size_t step = (size_t)a.kv_heads * rows, at = (size_t)kvh * rows + r;
     float M = -INFINITY;
-    for (int s = 0; s < n; ++s) M = fmaxf(M, a.stat[(at + s * step) * 4]);
+    for (int s = 0; s < n; ++s) M = fmaxf(M, a.stat[(at + s * step) * 2]);
     float num = 0.f, den = 0.f;
     for (int s = 0; s < n; ++s) {
-        const floatx4 st = *reinterpret_cast<const floatx4*>(a.stat + (at + s * step) * 4);
-        const float w = __builtin_amdgcn_exp2f(st[0] - M);  // (0 for a split none of whose keys the row has)
-        den = fmaf(w, st[1], den);
-        if (w > 0.f) num += ldexpf(w * a.part[(at + s * step) * hd + d], (int)st[2]);
+        const float2 st = *reinterpret_cast<const float2*>(a.stat + (at + s * step) * 2);
+        const float w = __builtin_amdgcn_exp2f(st.x - M);  // (0 for a split none of whose keys the row has)
+        den = fmaf(w, st.y, den);
+        num = fmaf(w, a.part[(at + s * step) * hd + d], num);
     }
     const float gate = a.qkv[(size_t)t * a.stride + (size_t)h * hd * 2 + hd + d];
     a.out[(size_t)t * a.out_stride + (size_t)h * hd + d] = num / den * sigmoidf_(gate);
@@ -988,7 +945,7 @@ hipError_t launch_attention_batch(const AttnBatchArgs& a0, hipStream_t stream) {
     case HD:                                                                                              \
         launch_kernel(attn_prep_batch_kernel<HD / 64>, dim3(a.count), dim3(512), prep_lds, stream, a);     \
         launch_kernel(attn_split_kv_kernel<HD>, kv_grid, dim3(256), 0, stream, a);                         \
-        launch_kernel(attn_flash_kernel<HD>, grid, dim3(64 * kFlashRows / 16 / kFlashQT), 0, stream, a);                             \
+        launch_kernel(attn_flash_kernel<HD>, grid, dim3(kFlashThreads), 0, stream, a);                         \
         break;
     switch (hd) {
         EMPRISE_ATTN_CASE(64)

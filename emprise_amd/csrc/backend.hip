@@ -1130,17 +1130,16 @@ emprise_status emprise_hip_attention_batch(emprise_hip* h, const emprise_hip_att
     a.out_stride = out_stride;
     const size_t hq = (size_t)count * p->heads * p->head_dim;
     const size_t tiles = (size_t)(first_position + count + kAttnKeyTile - 1) / kAttnKeyTile * p->kv_heads;
-    const size_t pieces = tiles * kAttnKeyTile * p->head_dim * 4;  // of the keys, and of the values
+    const size_t elems = tiles * kAttnKeyTile * p->head_dim;  // of the keys, and of the values
     const int splits = attention_batch_splits(p->heads, p->kv_heads, first_position, count);
     void *q, *kv;
     TRY(h->get_scratch("attnb_q", hq * sizeof(float), &q));
-    TRY(h->get_scratch("attnb_kv", 2 * pieces + tiles * (kAttnKeyTile + 1) * 4, &kv));
+    TRY(h->get_scratch("attnb_kv", elems * 10 + tiles * kAttnKeyTile * 4, &kv));
     a.q = static_cast<float*>(q);
     a.kf = static_cast<uint16_t*>(kv);
-    a.vf = a.kf + pieces / 2;
-    a.ke = reinterpret_cast<float*>(a.vf + pieces / 2);
-    a.ve = reinterpret_cast<int*>(a.ke + tiles * kAttnKeyTile);
-    const size_t part_bytes = splits * (hq + (size_t)count * p->heads * 4) * sizeof(float);
+    a.vf = a.kf + elems * 2;
+    a.ke = reinterpret_cast<float*>(a.vf + elems * 3);
+    const size_t part_bytes = splits * (hq + (size_t)count * p->heads * 2) * sizeof(float);
     // (captured with none there yet: one workgroup takes all the keys of its rows)
     if (splits > 1 && !(h->capturing && h->scratch["attnb_part"].bytes < part_bytes)) {
         void* part;

@@ -202,9 +202,9 @@ constexpr int kAttnSplit = 128;  // position ranges (workgroups) per KV head of 
 constexpr int kAttnFew = 64;     // those that a short context uses (attn_per)
 // `count` consecutive prompt positions from absolute position `first`: qkv row t at
 // t * stride floats; out row t at t * out_stride. Scratch: q (count x heads x hd floats);
-// per KV head and 32-key tile kf and vf (32 x hd x 2 halves each), ke (32 floats) and ve; for
+// per KV head and 32-key tile kf (32 x hd x 2 fp16), vf (32 x hd x 3 bf16) and ke (32 floats); for
 // more than one split part (splits x kv_heads x rows x hd floats, rows = count x heads per KV
-// head) and stat (4 floats for each of those rows).
+// head) and stat (2 floats for each of those rows).
 struct AttnBatchArgs {
     int heads, kv_heads, head_dim, rotary, count, first;
     float eps, rope_base;
@@ -218,7 +218,6 @@ struct AttnBatchArgs {
     float* q;
     uint16_t *kf, *vf;
     float* ke;
-    int* ve;
     float *part, *stat;
     int split_tiles;  // key tiles per split (set by the launch)
     float* out;

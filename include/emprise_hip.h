@@ -267,9 +267,10 @@ emprise_status emprise_hip_attention(emprise_hip* h, const emprise_hip_attention
  * model.cpp:355-366): qkv is the row of the first position, the rows of later positions
  * `stride` floats further; their k/v are appended to the caches at their positions and
  * position t attends over 0..first_position+t; out receives `count` rows `out_stride`
- * floats apart. p->position is not used. The dot products and P.V run on the matrix cores
- * (exact fp16 pieces to 22 bits, FP32 sums), so the outputs equal those of `count`
- * emprise_hip_attention calls up to summation order. */
+ * floats apart. p->position is not used. The products run on the matrix cores: queries and
+ * keys in two fp16 pieces (22 bits), probabilities and values whole in three bf16 pieces, FP32
+ * sums; so the outputs equal those of `count` emprise_hip_attention calls up to summation order
+ * and the scores' 2^-22. (An infinite cached value gives NaN.) */
 emprise_status emprise_hip_attention_batch(emprise_hip* h, const emprise_hip_attention_params* p, emprise_dev qkv,
                                            int count, uint64_t stride, int first_position, emprise_dev out,
                                            uint64_t out_stride);

@@ -573,9 +573,10 @@ def test_quantize_q8_exact_on_ties_and_scales(backend):
         backend.free(b)
 
 
-def _attention_rows64(heads, kv, hd, rot, base, eps, qn, kn, rows, keys, values, first):
+def _attention_rows64(heads, kv, hd, rot, base, eps, qn, kn, rows, keys, values, first, per_key=False):
     """Gated causal attention of the rows in 64 bits (the rotary angle is an FP32 value);
-    also the bound's parts: per row and head the largest sum |q k| / sqrt(hd) and sum p |v|."""
+    also the bound's parts: per row and head the largest sum |q k| / sqrt(hd) and sum p |v|
+    (per_key: each key's own sum with its p |v|, and their mean with sum p |v|)."""
     n, f8 = len(rows), np.float64
     i = np.arange(rot // 2, dtype=np.float32)
 
@@ -599,9 +600,13 @@ def _attention_rows64(heads, kv, hd, rot, base, eps, qn, kn, rows, keys, values,
         p = np.exp(s - s.max(1, keepdims=True))
         p /= p.sum(1, keepdims=True)
         gate = 1 / (1 + np.exp(-qg[:, h, 1]))
-        size = np.where(masked, 0, np.abs(q[:, h]) @ np.abs(ks[:, j]).T / np.sqrt(hd)).max(1, keepdims=True)
+        size = np.where(masked, 0, np.abs(q[:, h]) @ np.abs(ks[:, j]).T / np.sqrt(hd))
         out[:, h] = p @ vs[:, j] * gate
-        bound[:, h] = p @ np.abs(vs[:, j]) * size * gate
+        if per_key:
+            pv = p @ np.abs(vs[:, j])
+            bound[:, h] = ((p * size) @ np.abs(vs[:, j]) + (1 + (p * size).sum(1, keepdims=True)) * pv) * gate
+        else:
+            bound[:, h] = p @ np.abs(vs[:, j]) * size.max(1, keepdims=True) * gate
     return out.reshape(n, -1), bound.reshape(n, -1)
 
 
@@ -633,6 +638,60 @@ def test_attention_batch_tiles(backend, heads, kv, hd, rot, first, count):
     ref, size = _attention_rows64(heads, kv, hd, rot, 1e7, 1e-6, qn, kn, rows, keys, values, first)
     # + the FP32 cos/sin, norms and exp2 of the device, a few 2^-23 of the score each
     assert np.all(np.abs(got - ref) <= 2.0**-18 * size + 1e-30)
+
+
+# what the values of one 32-key tile, key or dim are beside the others must not matter
+@pytest.mark.parametrize("heads,kv,hd,first,count", [(4, 1, 256, 1000, 24), (8, 2, 64, 500, 70), (2, 2, 128, 2100, 3)])
+@pytest.mark.parametrize("sizes", ["tiles", "zero tile", "weightless key", "later key", "dims", "checkered"])
+def test_attention_batch_values_of_any_size(backend, heads, kv, hd, first, count, sizes):
+    """The tiled prefill attention where large values have next to no weight, against 64 bits.
+    The bound: a score is a few 2^-22 of sum |q k| / sqrt(hd) off, which moves its key's share
+    p |v| and, through the sum of the weights, all of the output by as much; P.V, the norms and
+    exp2 a few 2^-23 of sum p |v|. Per output value: no other dim's or key's size enters."""
+    rng = np.random.default_rng(first + count + hd)
+    kvd, qd, L, group = kv * hd, heads * hd * 2, first + count, heads // kv
+    W, one = qd + 2 * kvd, np.ones(hd, np.float32)
+    keys = rng.standard_normal((first, kv, hd)).astype(np.float32)
+    values = rng.standard_normal((first, kv, hd)).astype(np.float32)
+    rows = rng.standard_normal((count, W)).astype(np.float32)
+    new_v = rows[:, qd + kvd:].reshape(count, kv, hd)
+    if sizes == "tiles":
+        values *= np.repeat(10.0 ** rng.uniform(-8, 8, (L // 32 + 1, kv)), 32, 0)[:first, :, None].astype(np.float32)
+    elif sizes == "zero tile":
+        values *= np.float32(1e-3)
+        values[:64] = 0
+        new_v *= np.float32(1e-3)
+    elif sizes == "weightless key":  # against all the queries (equal up to a little), with a weight near 2^-90
+        for j in range(kv):
+            base = np.sign(rng.standard_normal(hd)).astype(np.float32)
+            q = rows[:, :qd].reshape(count, kv, group, 2, hd)
+            q[:, j, :, 0] = base * rng.uniform(0.9, 1.1, (count, group, hd)).astype(np.float32)
+            keys[3, j], keys[200, j] = -base * 60 / np.sqrt(hd), -base * 64 / np.sqrt(hd)
+            values[3, j] *= np.float32(1e8)
+            values[200, j] *= np.float32(1e12)
+    elif sizes == "later key":  # which the rows before it may not see
+        new_v[count // 2] *= np.float32(1e10)
+    elif sizes == "dims":
+        scale = (10.0 ** rng.uniform(-12, 12, (kv, hd))).astype(np.float32)
+        values *= scale
+        new_v *= scale
+    else:  # every other value, in rows and dims alike
+        odd = (np.arange(first)[:, None, None] + np.arange(hd)) % 2 == 1
+        values *= np.where(odd, 1e-10, 1.0).astype(np.float32)
+    kc, vc = np.zeros((L, kvd), np.float32), np.zeros((L, kvd), np.float32)
+    kc[:first], vc[:first] = keys.reshape(first, kvd), values.reshape(first, kvd)
+    kd, vd, rd = backend.to_device(kc), backend.to_device(vc), backend.to_device(rows)
+    od = backend.alloc(count * heads * hd * 4)
+    w = backend.vector(one)
+    backend.attention_batch(AttentionParams(heads, kv, hd, 0, L, 1e-6, 1e7, w, w, kd, vd, 0), rd, count, W, first, od,
+                            heads * hd)
+    got = backend.download(od, (count, heads * hd))
+    ref, size = _attention_rows64(heads, kv, hd, 0, 1e7, 1e-6, one, one, rows, keys, values, first, per_key=True)
+    off = np.abs(got - ref) / (size + 1e-30)
+    assert off.max() <= 2.0**-19, np.unravel_index(off.argmax(), off.shape)
+    for b in (kd, vd, rd, od):
+        backend.free(b)
+    backend.weight_free(w)
 
 
 def test_attention_batch_in_a_new_graph():
