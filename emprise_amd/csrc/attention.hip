@@ -462,9 +462,10 @@ __global__ __launch_bounds__(256) void rope_table_kernel(float2* t, int context,
 // attn_merge_batch_kernel joins their partial results.
 //
 // Scores run on the fp16 matrix cores from two fp16 pieces per FP32 operand: x = 2^e (xh +
-// xl), 22 significant bits, e taken per query and per key (from the largest of its head_dim
-// values), three products of four (xl yl is below 2^-22 of its term), FP32 sums. P.V carries P
-// and V whole, as three bf16 pieces of 8 bits each (with FP32's range, so it does not matter how the values' sizes differ), in the six products above 2^-24 of their
+// 2^-11 xl), 22 significant bits of every value down to 2^-28 of its vector's largest, e taken
+// per query and per key, three products of four (xl yl is below 2^-22 of its term), those with a
+// low piece in a sum of their own, FP32 sums. P.V carries P and V whole, as three bf16 pieces of 8
+// bits each (with FP32's range, so it does not matter how the values' sizes differ), in the six products above 2^-24 of their
 // term, a tile's summed apart from O. Each product has 16 queries on the lane index: S^T = K Q^T
 // leaves lane (query l%16, group g = l/16) the scores of keys 4g .. 4g+3 of two 16-key halves,
 // which is the operand of O^T = V^T P^T if V^T lists the 32 keys in that order -- so it does, and
@@ -532,13 +533,14 @@ constexpr int kKeyTile = kAttnKeyTile;
 constexpr int kFlashRows = 128;  // query rows (position x head of a KV head's group) per workgroup
 constexpr int kFlashThreads = 64 * kFlashRows / 16;
 constexpr float kLag = 8.f;      // a row's maximum may pass its reference by this (powers of two)
+constexpr float kLow = 2048.f;   // the low fp16 pieces of queries and keys are carried 2^11 times as large
 
-// The exponent that brings a vector of largest magnitude mx to [2^12, 2^13).
+// The exponent that brings a vector of largest magnitude mx to [2^14, 2^15).
 __device__ __forceinline__ int piece_exp(float mx) {
     int e = 0;
     if (mx > 0.f && mx < INFINITY) {
         (void)frexpf(mx, &e);
-        e = max(e - 13, -126);
+        e = max(e - 15, -126);
     }
     return e;
 }
@@ -547,7 +549,7 @@ __device__ __forceinline__ void split8(const float (&v)[8], float up, half8& hi,
     for (int k = 0; k < 8; ++k) {
         const float w = v[k] * up;
         hi[k] = (_Float16)w;
-        lo[k] = (_Float16)(w - (float)hi[k]);
+        lo[k] = (_Float16)((w - (float)hi[k]) * kLow);
     }
 }
 // x = p0 + p1 + p2, each the next 8 significant bits of it as bf16 (a NaN stays one; an
@@ -740,10 +742,10 @@ __global__ __launch_bounds__(kFlashThreads, 2) void attn_flash_kernel(AttnBatchA
         ke[0] = *reinterpret_cast<const float4*>(e);
         ke[1] = *reinterpret_cast<const float4*>(e + 16);
     };
-    auto scores = [&](int b, floatx4 (&S)[2]) {
+    auto scores = [&](int b, floatx4 (&S)[2], floatx4 (&R)[2]) {
         const half8* K = reinterpret_cast<const half8*>(KV + b * KN);
 #pragma unroll
-        for (int kt = 0; kt < 2; ++kt) S[kt] = floatx4{0.f, 0.f, 0.f, 0.f};
+        for (int kt = 0; kt < 2; ++kt) S[kt] = R[kt] = floatx4{0.f, 0.f, 0.f, 0.f};
         half8 kh[KD + 1][2], kl[KD + 1][2];
         auto operands = [&](int s) {
 #pragma unroll
@@ -759,28 +761,29 @@ __global__ __launch_bounds__(kFlashThreads, 2) void attn_flash_kernel(AttnBatchA
             if (s + KD < NS) operands(s + KD);
             const int r = s % (KD + 1);
 #pragma unroll
-            for (int kt = 0; kt < 2; ++kt) S[kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kl[r][kt], qh[s], S[kt], 0, 0, 0);
-#pragma unroll
-            for (int kt = 0; kt < 2; ++kt) S[kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh[r][kt], ql[s], S[kt], 0, 0, 0);
+            for (int kt = 0; kt < 2; ++kt) R[kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kl[r][kt], qh[s], R[kt], 0, 0, 0);
 #pragma unroll
             for (int kt = 0; kt < 2; ++kt) S[kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh[r][kt], qh[s], S[kt], 0, 0, 0);
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt) R[kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh[r][kt], ql[s], R[kt], 0, 0, 0);
             if (s + KD < NS) __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);  // LDS reads, then
             __builtin_amdgcn_sched_group_barrier(0x008, 6, 0);                  // products
         }
     };
-    auto scaled = [&](const floatx4 (&S)[2], int tile) {
+    auto scaled = [&](const floatx4 (&S)[2], const floatx4 (&R)[2], int tile) {
         const float e[8] = {ke[0].x, ke[0].y, ke[0].z, ke[0].w, ke[1].x, ke[1].y, ke[1].z, ke[1].w};
         const int key0 = tile * kKeyTile + 4 * g;
         mx = -INFINITY;
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
-            x[k] = key0 + (k >> 2) * 16 + (k & 3) <= last ? (S[k >> 2][k & 3] * e[k]) * qs : -INFINITY;
+            const float s = fmaf(R[k >> 2][k & 3], 1.f / kLow, S[k >> 2][k & 3]);
+            x[k] = key0 + (k >> 2) * 16 + (k & 3) <= last ? (s * e[k]) * qs : -INFINITY;
             mx = fmaxf(mx, x[k]);
         }
         mx = max_groups(mx);
     };
 
-    floatx4 O[ND], S[2];
+    floatx4 O[ND], S[2], R[2];
     float m = -INFINITY, l = 0.f;  // the reference of the scores, a whole number; the sum of 2^(score - m - kLag)
 #pragma unroll
     for (int d = 0; d < ND; ++d) O[d] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -791,8 +794,8 @@ __global__ __launch_bounds__(kFlashThreads, 2) void attn_flash_kernel(AttnBatchA
     load_values(min(tile0 + 1, tile1 - 1));
     lds_barrier();
     if (active) {
-        scores(0, S);
-        scaled(S, tile0);
+        scores(0, S, R);
+        scaled(S, R, tile0);
     }
     store_keys(1);
     load_keys(min(tile0 + 2, tile1 - 1));
@@ -828,8 +831,8 @@ __global__ __launch_bounds__(kFlashThreads, 2) void attn_flash_kernel(AttnBatchA
                 l += sum;
                 split3(p, P);
             }
-            scores(buf ^ 1, S);
-            scaled(S, tile + 1);
+            scores(buf ^ 1, S, R);
+            scaled(S, R, tile + 1);
             // P.V of two dims tiles at a time: the products of pieces i and j for i + j <= 2, the
             // smallest first, in a sum of their own, so that O is rounded once per tile; step
             // (d, n) uses piece 2 - n of the values

@@ -268,9 +268,10 @@ emprise_status emprise_hip_attention(emprise_hip* h, const emprise_hip_attention
  * `stride` floats further; their k/v are appended to the caches at their positions and
  * position t attends over 0..first_position+t; out receives `count` rows `out_stride`
  * floats apart. p->position is not used. The products run on the matrix cores: queries and
- * keys in two fp16 pieces (22 bits), probabilities and values whole in three bf16 pieces, FP32
- * sums; so the outputs equal those of `count` emprise_hip_attention calls up to summation order
- * and the scores' 2^-22. (An infinite cached value gives NaN.) */
+ * keys in two fp16 pieces (22 bits of every value down to 2^-28 of its vector's largest),
+ * probabilities and values whole in three bf16 pieces, FP32 sums; so the outputs equal those
+ * of `count` emprise_hip_attention calls up to summation order and the scores' 2^-22. (An
+ * infinite cached value gives NaN.) */
 emprise_status emprise_hip_attention_batch(emprise_hip* h, const emprise_hip_attention_params* p, emprise_dev qkv,
                                            int count, uint64_t stride, int first_position, emprise_dev out,
                                            uint64_t out_stride);

@@ -694,6 +694,33 @@ def test_attention_batch_values_of_any_size(backend, heads, kv, hd, first, count
     backend.weight_free(w)
 
 
+@pytest.mark.parametrize("heads,kv,hd,first,count", [(4, 1, 256, 300, 24), (8, 2, 64, 500, 70)])
+def test_attention_batch_keys_with_large_dims(backend, heads, kv, hd, first, count):
+    """Keys that are large in one dim where the queries are small (by the norms' weights), so
+    that all dims count alike in the scores; the bound of the test above."""
+    rng = np.random.default_rng(first + hd)
+    kvd, qd, L = kv * hd, heads * hd * 2, first + count
+    W, qn, kn = qd + 2 * kvd, np.ones(hd, np.float32), np.ones(hd, np.float32)
+    qn[5], kn[5] = 2.0**-24, 2.0**24
+    keys = rng.standard_normal((first, kv, hd)).astype(np.float32)
+    keys[:, :, 5] *= np.float32(2.0**24)
+    values = rng.standard_normal((first, kv, hd)).astype(np.float32)
+    rows = rng.standard_normal((count, W)).astype(np.float32)
+    kc, vc = np.zeros((L, kvd), np.float32), np.zeros((L, kvd), np.float32)
+    kc[:first], vc[:first] = keys.reshape(first, kvd), values.reshape(first, kvd)
+    kd, vd, rd = backend.to_device(kc), backend.to_device(vc), backend.to_device(rows)
+    od, qw, kw = backend.alloc(count * heads * hd * 4), backend.vector(qn), backend.vector(kn)
+    backend.attention_batch(AttentionParams(heads, kv, hd, 0, L, 1e-6, 1e7, qw, kw, kd, vd, 0), rd, count, W, first, od,
+                            heads * hd)
+    got = backend.download(od, (count, heads * hd))
+    ref, size = _attention_rows64(heads, kv, hd, 0, 1e7, 1e-6, qn, kn, rows, keys, values, first, per_key=True)
+    assert np.max(np.abs(got - ref) / size) <= 2.0**-19
+    for b in (kd, vd, rd, od):
+        backend.free(b)
+    for w in (qw, kw):
+        backend.weight_free(w)
+
+
 def test_attention_batch_in_a_new_graph():
     """Captured with no partial-result scratch yet: one workgroup takes all of a row's keys."""
     from emprise_amd import HipBackend
