@@ -10,6 +10,7 @@
 #include <cstdio>
 #include <cstring>
 #include <map>
+#include <memory>
 #include <set>
 #include <string>
 #include <thread>
@@ -112,14 +113,21 @@ struct emprise_hip {
     std::string name;
     std::unordered_map<uint64_t, Weight> weights;
     uint64_t next_weight = 1;
-    std::unordered_map<uint64_t, hipGraphExec_t> graphs;
-    uint64_t next_graph = 1;
-    std::vector<hipEvent_t> events;
-    // scratch buffers, grown outside graph capture only
+    // scratch buffers, grown outside graph capture only; a graph keeps those it was captured
+    // with, so that a replay after a larger call has grown one still finds it
+    using Buffer = std::shared_ptr<void>;
     struct Scratch {
-        void* ptr = nullptr;
+        Buffer ptr;
         size_t bytes = 0;
     };
+    struct Graph {
+        hipGraphExec_t exec = nullptr;
+        std::vector<Buffer> buffers;
+    };
+    std::vector<Buffer> captured;  // of the graph being captured
+    std::unordered_map<uint64_t, Graph> graphs;
+    uint64_t next_graph = 1;
+    std::vector<hipEvent_t> events;
     std::unordered_map<std::string, Scratch> scratch;
     std::set<std::string> rope_ready;  // RoPE tables (scratch keys) already filled
     // kernel trace (emprise_hip_trace_begin/end)
@@ -150,15 +158,17 @@ struct emprise_hip {
         Scratch& s = scratch[key];
         if (s.bytes < bytes) {
             if (capturing) return fail(EMPRISE_ESTATE, "scratch '%s' must be sized before graph capture", key);
-            if (s.ptr) HIP_TRY(hipFree(s.ptr));
-            s.ptr = nullptr;
+            s.ptr.reset();
             s.bytes = 0;
-            HIP_TRY(hipMalloc(&s.ptr, bytes));
+            void* p = nullptr;
+            HIP_TRY(hipMalloc(&p, bytes));
+            s.ptr = Buffer(p, [](void* q) { (void)hipFree(q); });
             // on this stream: one of the null stream's may still be running when the next kernel reads it
-            if (zero) HIP_TRY(hipMemsetAsync(s.ptr, 0, bytes, stream));
+            if (zero) HIP_TRY(hipMemsetAsync(p, 0, bytes, stream));
             s.bytes = bytes;
         }
-        *out = s.ptr;
+        if (capturing) captured.push_back(s.ptr);
+        *out = s.ptr.get();
         return EMPRISE_OK;
     }
 };
@@ -351,9 +361,11 @@ void emprise_hip_destroy(emprise_hip* h) {
     if (!h) return;
     (void)hipSetDevice(h->device);
     (void)hipStreamSynchronize(h->stream);
-    for (auto& kv : h->graphs) (void)hipGraphExecDestroy(kv.second);
+    for (auto& kv : h->graphs) (void)hipGraphExecDestroy(kv.second.exec);
+    h->graphs.clear();
+    h->captured.clear();
     for (auto& kv : h->weights) (void)hipFree(kv.second.dev);
-    for (auto& kv : h->scratch) (void)hipFree(kv.second.ptr);
+    h->scratch.clear();
     for (int k = 0; k < 2; ++k) {
         if (h->upload.host[k]) (void)hipHostFree(h->upload.host[k]);
         if (h->upload.dev[k]) (void)hipFree(h->upload.dev[k]);
@@ -1229,14 +1241,15 @@ emprise_status emprise_hip_graph_end(emprise_hip* h, emprise_graph* out) {
     if (!h || !out) return fail(EMPRISE_EINVAL, "null argument");
     if (!h->capturing) return fail(EMPRISE_ESTATE, "not capturing");
     h->capturing = false;
+    emprise_hip::Graph g;
+    g.buffers.swap(h->captured);
     hipGraph_t graph = nullptr;
     HIP_TRY(hipStreamEndCapture(h->stream, &graph));
-    hipGraphExec_t exec = nullptr;
-    hipError_t e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
+    hipError_t e = hipGraphInstantiate(&g.exec, graph, nullptr, nullptr, 0);
     (void)hipGraphDestroy(graph);
     if (e != hipSuccess) return fail(EMPRISE_EDEVICE, "graph instantiate: %s", hipGetErrorString(e));
     const uint64_t id = h->next_graph++;
-    h->graphs.emplace(id, exec);
+    h->graphs.emplace(id, std::move(g));
     *out = id;
     return EMPRISE_OK;
 }
@@ -1245,7 +1258,7 @@ emprise_status emprise_hip_graph_launch(emprise_hip* h, emprise_graph g) {
     if (!h) return fail(EMPRISE_EINVAL, "null backend");
     auto it = h->graphs.find(g);
     if (it == h->graphs.end()) return fail(EMPRISE_EINVAL, "unknown graph");
-    HIP_TRY(hipGraphLaunch(it->second, h->stream));
+    HIP_TRY(hipGraphLaunch(it->second.exec, h->stream));
     return EMPRISE_OK;
 }
 
@@ -1254,7 +1267,7 @@ emprise_status emprise_hip_graph_destroy(emprise_hip* h, emprise_graph g) {
     auto it = h->graphs.find(g);
     if (it == h->graphs.end()) return fail(EMPRISE_EINVAL, "unknown graph");
     HIP_TRY(hipStreamSynchronize(h->stream));
-    HIP_TRY(hipGraphExecDestroy(it->second));
+    HIP_TRY(hipGraphExecDestroy(it->second.exec));
     h->graphs.erase(it);
     return EMPRISE_OK;
 }

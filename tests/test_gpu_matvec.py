@@ -565,6 +565,42 @@ def test_linear_batch_in_a_new_graph(tokens):
                 _close(got, eager)
 
 
+@pytest.mark.parametrize("tokens,cols", [(5, 4096), (3, 1536), (40, 4096)])
+def test_graph_keeps_the_scratch_it_was_captured_with(tokens, cols):
+    """Partial sums' and operands' scratch that a later, larger call outgrows: replays of a graph
+    captured before it neither lose their memory nor write into what took its place."""
+    from emprise_amd import HipBackend
+
+    rng = np.random.default_rng(tokens + cols)
+    rows, big = 200, 3000
+    with HipBackend() as be:
+        w = be.upload_weight(Q6_K, cols, rows, matrix(rng, Q6_K, rows, cols))
+        wide = be.upload_weight(Q6_K, cols, big, matrix(rng, Q6_K, big, cols))
+        x = be.to_device(rng.standard_normal((600, cols)).astype(np.float32))
+        y, z = be.alloc(tokens * rows * 4), be.alloc(600 * big * 4)
+        be.linear_batch(w, x, y, tokens)
+        eager = be.download(y, (tokens, rows))
+        be.graph_begin()
+        be.linear_batch(w, x, y, tokens)
+        g = be.graph_end()
+        for more in (32, 64, 600):  # each outgrows one of the buffers
+            be.linear_batch(wide, x, z, more)
+        be.sync()
+        n = 1 << 16
+        others = [be.alloc(n * 4) for _ in range(64)]
+        for b in others:
+            be.fill(b, 7.0, n)
+        for _ in range(3):
+            be.fill(y, 0.0, tokens * rows)
+            be.graph_launch(g)
+            assert np.array_equal(be.download(y, (tokens, rows)), eager)
+        for b in others:
+            assert np.all(be.download(b, n) == 7.0)
+        be.graph_destroy(g)
+        be.linear_batch(w, x, y, tokens)
+        assert np.array_equal(be.download(y, (tokens, rows)), eager)
+
+
 def _matvec_bound(W, x, rows_abs=0.0):
     """Per output: FP32 sums of at most cols terms in short chains (64 per lane and group of
     columns, then the lanes), with 2^-24 per addition and per product."""
