@@ -601,7 +601,7 @@ static size_t part_bytes(int M, uint64_t N, int K) {
 static emprise_status run_gemm_q16(emprise_hip* h, uint32_t type, QGemmArgs& a, uint64_t flops) {
     const size_t bytes = part_bytes(a.M, a.N, a.K);
     a.part = nullptr;
-    if (bytes && (gemm_q16_few(a.M) || !h->capturing || h->scratch["gemm_part"].bytes >= bytes)) {
+    if (bytes && (!h->capturing || h->scratch["gemm_part"].bytes >= bytes)) {
         void* part;
         TRY(h->get_scratch("gemm_part", bytes, &part));
         a.part = static_cast<float*>(part);
@@ -638,13 +638,10 @@ static int small_batch(const emprise_hip* h, const Weight* wt) {
 // kernel does not take from 2 rows on (2048 x 6144 at 3 rows 27.4 as three matvecs, 14.0).
 // Q6_K under --fast-q8 keeps the single-input path, which quantises its input, up to
 // kGemmMinBatch, as do the unquantised types, whose GEMM fills 128-row tiles.
-// (`rows`: of all the weights of the call. The form for few rows keeps its partial sums in
-// scratch, which cannot grow while a graph is being captured.)
-static bool on_gemm(emprise_hip* h, const Weight* wt, int K, uint64_t rows) {
+static bool on_gemm(const emprise_hip* h, const Weight* wt, int K) {
     if (wt->type != kQ6K && wt->type != kQ4K) return K >= kGemmMinBatch && wt->cols % 16 == 0;
     if (K < kGemmMinBatch && ((h->q8 && wt->type == kQ6K) || wt->cols > kMatvecMaxCols)) return false;
-    if (K <= small_batch(h, wt)) return false;
-    return !(gemm_q16_few(K) && h->capturing && !(h->q8 && wt->type == kQ6K) && h->scratch["gemm_part"].bytes < part_bytes(K, rows, (int)wt->cols));
+    return K > small_batch(h, wt);
 }
 
 // Y[k] = [W_0; W_1; ...] X[k]: the weights' rows side by side in Y, for K rows of X. Where
@@ -664,7 +661,7 @@ static emprise_status linear_batch_rows(emprise_hip* h, int nw, const Weight* co
     const float* A = reinterpret_cast<const float*>(X);
     float* C = reinterpret_cast<float*>(Y);
     const uint64_t flops_per_row = 2ull * (uint64_t)K * (uint64_t)cols;
-    auto on_q16 = [&](const Weight* wt) { return aligned && (wt->type == kQ6K || wt->type == kQ4K) && on_gemm(h, wt, K, rows); };
+    auto on_q16 = [&](const Weight* wt) { return aligned && (wt->type == kQ6K || wt->type == kQ4K) && on_gemm(h, wt, K); };
     bool any_q = false, sums = false;
     for (int i = 0; i < nw; ++i)
         if (on_q16(ws[i])) any_q = true, sums = sums || ws[i]->type == kQ4K;
@@ -693,7 +690,7 @@ static emprise_status linear_batch_rows(emprise_hip* h, int nw, const Weight* co
             i = j;
             continue;
         }
-        if (!aligned || !on_gemm(h, wt, K, rows)) {
+        if (!aligned || !on_gemm(h, wt, K)) {
             const int per = aligned ? small_batch(h, wt) : 1;
             for (int k0 = 0; k0 < K;) {
                 const int n = std::min(per, K - k0);
@@ -768,7 +765,7 @@ emprise_status emprise_hip_ffn_gate_up_batch(emprise_hip* h, emprise_weight gate
     float* y = reinterpret_cast<float*>(Y);
     // gate and up of one quantised type: one GEMM over their interleaved rows, SwiGLU in its
     // epilogue (gemm_q.hip, QGemmArgs::pair)
-    if ((g->type == kQ6K || g->type == kQ4K) && u->type == g->type && on_gemm(h, g, K, 2ull * F) && X % 16 == 0 && ldx % 4 == 0) {
+    if ((g->type == kQ6K || g->type == kQ4K) && u->type == g->type && on_gemm(h, g, K) && X % 16 == 0 && ldx % 4 == 0) {
         QGemmArgs qa{};
         TRY(split_q16(h, reinterpret_cast<const float*>(X), K, cols, (int)ldx, g->type == kQ4K, &qa));
         qa.nseg = 2;

@@ -481,18 +481,85 @@ __global__ __launch_bounds__(WV * 64, OCC) void gemm_q16_kernel(QGemmArgs a) {
     q_store<RT, MT>(a, n0, t0, rj, q, acc);
 }
 
-// The form for up to 32 tokens, where the weights' bytes are the bound: a workgroup splits
+// The forms for up to 32 tokens, where the weights' bytes are the bound: a workgroup splits
 // its span of the activations itself (no pass before it), keeps all of it in LDS, and its
-// waves then walk row tiles on their own -- no barrier, two blocks' weights in flight per
-// wave -- leaving each tile's sums over the span in part[z]. Grid: x = workgroups over the
-// rows, z = spans of kFewSpan blocks.
+// waves then walk row tiles on their own.
 constexpr int kFewSpan = 4;
+template <int T, int MT> struct Few {
+    static constexpr int AV = MT * 1024;                        // 16-byte pieces of a block's operands
+    static constexpr int SV = MT * (T == kQ4K ? 36 : 4);        // of its side data
+    uint4 x[kFewSpan * AV], side[kFewSpan * SV];
+};
+
+// Blocks b0 .. b0+nbs-1 of the activations.
+template <int T, int MT> __device__ __forceinline__ void few_stage(const QGemmArgs& a, int b0, int nbs, Few<T, MT>& lds) {
+    using F = Few<T, MT>;
+    for (int t = threadIdx.x; t < nbs * MT * 256; t += blockDim.x) {
+        const int u = t >> 8, i = (t >> 4) & 15, c = t & 15, bl = u / MT, m = u - bl * MT;
+        float v[16];
+        load16(v, a.x, m * 16 + i, a.M, a.ldx, (b0 + bl) * kBlk + 16 * c);
+        uint4* side = lds.side + bl * F::SV;
+        split16(v, i, c, reinterpret_cast<_Float16*>(lds.x + bl * F::AV + m * 1024), reinterpret_cast<float*>(side + 4 * m),
+                reinterpret_cast<_Float16*>(side + 4 * MT + 32 * m), T == kQ4K);
+    }
+}
+
+// acc += the products of staged block bl.
+//
+// Three product sums per token tile, added at the block's end: the xh * vh of the even
+// and of the odd slices, and the small terms -- shorter chains of FP32 additions
+// (relative error against 64 bits at 5 tokens x 4096 columns, Q6_K / Q4_K: 1.03e-7 /
+// 1.19e-7, with one sum and a float reduction 1.63e-7 / 1.92e-7, the FP32 matvec 1.83e-7
+// / 1.19e-7)
+template <int T, bool CH, int MT>
+__device__ __forceinline__ void few_block(const QRaw<T>& raw, const Few<T, MT>& lds, int bl, int lane, floatx4 (&acc)[1][MT]) {
+    using F = Few<T, MT>;
+    const int q = lane >> 4;
+    floatx4 cb[1][MT], c1[MT], cs[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) cb[0][m] = c1[m] = cs[m] = floatx4{0.f, 0.f, 0.f, 0.f};
+    uint32_t dblk[1], mins[1];
+    q_block_scales<CH>(raw, q, dblk[0], mins[0]);
+    const half8* A = reinterpret_cast<const half8*>(lds.x + bl * F::AV);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        half8 wh[1][2], wl[1][2];
+        if constexpr (T == kQ6K) q6_unit(raw, j, wh[0], wl[0]);
+        else q4_unit<CH>(raw, q, j, wh[0]);
+        half8 xh[2][MT], xl[2][MT];
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                xh[h][m] = A[m * 1024 + (4 * j + 2 * h) * 64 + lane];
+                xl[h][m] = A[m * 1024 + (4 * j + 2 * h + 1) * 64 + lane];
+            }
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            cb[0][m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[0][m], wh[0][0], cb[0][m], 0, 0, 0);
+            c1[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[1][m], wh[0][1], c1[m], 0, 0, 0);
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                cs[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl[h][m], wh[0][h], cs[m], 0, 0, 0);
+                if constexpr (T == kQ6K)
+                    cs[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[h][m], wl[0][h], cs[m], 0, 0, 0);
+            }
+    }
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) cb[0][m][r] += c1[m][r] + cs[m][r];
+    q_block_end<T, 1, MT>(lds.side + bl * F::SV, lane, dblk, mins, cb, acc);
+}
+
+// No barrier after the staging, two blocks' weights in flight per wave; each tile's sums over
+// the span go to part[z]. Grid: x = workgroups over the rows, z = spans of kFewSpan blocks.
 template <int T, bool CH, int MT>
 __global__ __launch_bounds__(1024) void gemm_q16_few_kernel(QGemmArgs a) {
-    constexpr int AV = MT * 1024;                        // 16-byte pieces of a block's operands
-    constexpr int SV = MT * (T == kQ4K ? 36 : 4);
-    __shared__ __align__(16) uint4 As[kFewSpan * AV];
-    __shared__ __align__(16) uint4 Ss[kFewSpan * SV];
+    __shared__ __align__(16) Few<T, MT> lds;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int q = lane >> 4, rj = lane & 15;
     const int nb = a.K / kBlk, b0 = blockIdx.z * kFewSpan, nbs = min(kFewSpan, nb - b0);
@@ -524,63 +591,15 @@ __global__ __launch_bounds__(1024) void gemm_q16_few_kernel(QGemmArgs a) {
     next(ld);
     q_load<CH>(r1, ld.row, nb, b0 + ld.b, q);
 
-    for (int t = tid; t < nbs * MT * 256; t += blockDim.x) {
-        const int u = t >> 8, i = (t >> 4) & 15, c = t & 15, bl = u / MT, m = u - bl * MT;
-        float v[16];
-        load16(v, a.x, m * 16 + i, a.M, a.ldx, (b0 + bl) * kBlk + 16 * c);
-        uint4* side = Ss + bl * SV;
-        split16(v, i, c, reinterpret_cast<_Float16*>(As + bl * AV + m * 1024), reinterpret_cast<float*>(side + 4 * m),
-                reinterpret_cast<_Float16*>(side + 4 * MT + 32 * m), T == kQ4K);
-    }
+    few_stage(a, b0, nbs, lds);
     __syncthreads();
 
-    // three product sums per token tile, added at the block's end: the xh * vh of the even
-    // and of the odd slices, and the small terms -- shorter chains of FP32 additions
-    // (relative error against 64 bits at 5 tokens x 4096 columns, Q6_K / Q4_K: 1.03e-7 /
-    // 1.19e-7, with one sum and a float reduction 1.63e-7 / 1.92e-7, the FP32 matvec 1.83e-7
-    // / 1.19e-7)
-    floatx4 cb[1][MT], c1[MT], cs[MT], acc[1][MT];
+    floatx4 acc[1][MT];
 #pragma unroll
-    for (int m = 0; m < MT; ++m) cb[0][m] = c1[m] = cs[m] = acc[0][m] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int m = 0; m < MT; ++m) acc[0][m] = floatx4{0.f, 0.f, 0.f, 0.f};
     int tile = first, bl = 0;
     auto compute = [&](const QRaw<T>& raw) {
-        uint32_t dblk[1], mins[1];
-        q_block_scales<CH>(raw, q, dblk[0], mins[0]);
-        const half8* A = reinterpret_cast<const half8*>(As + bl * AV);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            half8 wh[1][2], wl[1][2];
-            if constexpr (T == kQ6K) q6_unit(raw, j, wh[0], wl[0]);
-            else q4_unit<CH>(raw, q, j, wh[0]);
-            half8 xh[2][MT], xl[2][MT];
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-#pragma unroll
-                for (int m = 0; m < MT; ++m) {
-                    xh[h][m] = A[m * 1024 + (4 * j + 2 * h) * 64 + lane];
-                    xl[h][m] = A[m * 1024 + (4 * j + 2 * h + 1) * 64 + lane];
-                }
-#pragma unroll
-            for (int m = 0; m < MT; ++m) {
-                cb[0][m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[0][m], wh[0][0], cb[0][m], 0, 0, 0);
-                c1[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[1][m], wh[0][1], c1[m], 0, 0, 0);
-            }
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-#pragma unroll
-                for (int m = 0; m < MT; ++m) {
-                    cs[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl[h][m], wh[0][h], cs[m], 0, 0, 0);
-                    if constexpr (T == kQ6K)
-                        cs[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[h][m], wl[0][h], cs[m], 0, 0, 0);
-                }
-        }
-#pragma unroll
-        for (int m = 0; m < MT; ++m) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) cb[0][m][r] += c1[m][r] + cs[m][r];
-            c1[m] = cs[m] = floatx4{0.f, 0.f, 0.f, 0.f};
-        }
-        q_block_end<T, 1, MT>(Ss + bl * SV, lane, dblk, mins, cb, acc);
+        few_block<T, CH, MT>(raw, lds, bl, lane, acc);
         if (++bl == nbs) {
             q_store<1, MT>(a, tile * 16, 0, rj, q, acc);
 #pragma unroll
@@ -596,6 +615,45 @@ __global__ __launch_bounds__(1024) void gemm_q16_few_kernel(QGemmArgs a) {
         if (t + 1 < items) compute(r1);
         next(ld);
         q_load<CH>(r1, ld.row, nb, b0 + ld.b, q);
+    }
+}
+
+// The same sums without scratch for them (a graph being captured, which cannot grow it): a
+// workgroup stages one span after the other for its waves' row tiles and adds the spans'
+// sums in registers, in gemm_q16_reduce_kernel's order and precision. Grid: x as above.
+template <int T, bool CH, int MT>
+__global__ __launch_bounds__(512) void gemm_q16_few_serial_kernel(QGemmArgs a) {
+    __shared__ __align__(16) Few<T, MT> lds;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), q = lane >> 4, rj = lane & 15;
+    const int nb = a.K / kBlk, waves = blockDim.x >> 6, ntiles = (a.N + 15) >> 4;
+    for (int tile0 = blockIdx.x * waves; tile0 < ntiles; tile0 += gridDim.x * waves) {
+        const int tile = tile0 + wave;  // (tiles past the last read the last row; their results are not stored)
+        const uint8_t* row = q_row<T>(a, min(tile * 16 + rj, a.N - 1), nb);
+        double tot[MT][4] = {};
+        for (int b0 = 0; b0 < nb; b0 += kFewSpan) {
+            const int nbs = min(kFewSpan, nb - b0);
+            __syncthreads();
+            few_stage(a, b0, nbs, lds);
+            __syncthreads();
+            floatx4 acc[1][MT];
+#pragma unroll
+            for (int m = 0; m < MT; ++m) acc[0][m] = floatx4{0.f, 0.f, 0.f, 0.f};
+            for (int bl = 0; bl < nbs; ++bl) {
+                QRaw<T> raw;
+                q_load<CH>(raw, row, nb, b0 + bl, q);
+                few_block<T, CH, MT>(raw, lds, bl, lane, acc);
+            }
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) tot[m][r] += acc[0][m][r];
+        }
+        floatx4 acc[1][MT];
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[0][m][r] = (float)tot[m][r];
+        q_store<1, MT>(a, tile * 16, 0, rj, q, acc);
     }
 }
 
@@ -767,9 +825,11 @@ int tiles_for(int M) { return M <= 16 ? 1 : M <= 32 ? 2 : M <= 64 ? 4 : 8; }
 // 8-wave workgroups on half of the CUs 42.7).
 template <int T, bool CH, int MT> hipError_t launch_few(const QGemmArgs& a, int layers, hipStream_t stream) {
     const int ntiles = (a.N + 15) / 16, gx = std::min(std::max(1, kCUs / layers), ntiles);
-    const int per = (ntiles + gx - 1) / gx, rounds = (per + 15) / 16, waves = (per + rounds - 1) / rounds;
-    launch_kernel(gemm_q16_few_kernel<T, CH, MT>, dim3((ntiles + waves * rounds - 1) / (waves * rounds), 1, layers),
-                  dim3(waves * 64), 0, stream, a);
+    const int most = layers == a.spans ? 16 : 8;  // waves per workgroup
+    const int per = (ntiles + gx - 1) / gx, rounds = (per + most - 1) / most, waves = (per + rounds - 1) / rounds;
+    const dim3 grid((ntiles + waves * rounds - 1) / (waves * rounds), 1, layers), block(waves * 64);
+    if (layers == a.spans) launch_kernel(gemm_q16_few_kernel<T, CH, MT>, grid, block, 0, stream, a);
+    else launch_kernel(gemm_q16_few_serial_kernel<T, CH, MT>, grid, block, 0, stream, a);
     return launch_reduce(a, layers, stream);
 }
 
@@ -856,11 +916,11 @@ hipError_t launch_gemm_q16(uint32_t type, QGemmArgs a, hipStream_t stream) {
         return hipErrorInvalidValue;
     if (a.pair ? (a.nseg != 2 || a.N % 2 || a.row0[1] * 2 != a.N || a.ldy < a.N / 2) : a.ldy < a.N)
         return hipErrorInvalidValue;
-    const int nb = a.K / kBlk, layers = a.part || gemm_q16_few(a.M) ? gemm_q16_layers(a.M, a.N, a.K) : 1;
+    const int nb = a.K / kBlk, layers = a.part ? gemm_q16_layers(a.M, a.N, a.K) : 1;
     a.spans = gemm_q16_spans(a.M, a.K);
     a.span = (nb + a.spans - 1) / a.spans;
     if (gemm_q16_few(a.M) && a.span > kFewSpan) return hipErrorInvalidValue;
-    if (layers > 1 && (!a.part || a.M > 65535)) return hipErrorInvalidValue;
+    if (layers > 1 && a.M > 65535) return hipErrorInvalidValue;
     const bool ch = chunked_cols(a.K);
     if (type == kQ6K) return ch ? launch_type<kQ6K, true>(a, layers, stream) : launch_type<kQ6K, false>(a, layers, stream);
     return ch ? launch_type<kQ4K, true>(a, layers, stream) : launch_type<kQ4K, false>(a, layers, stream);

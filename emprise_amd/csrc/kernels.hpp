@@ -106,7 +106,8 @@ hipError_t launch_gemm_f32(const float* A, const float* B, float* C, int M, int 
 // one type whose rows follow each other in Y. launch_gemm_q16_split fills the activation
 // fields from X (fp16 hi/lo pieces of 2^-e x, e per row and 256 columns, and with `sums` the
 // pieces of its 32-column sums) in `scratch` (gemm_q16_split_bytes); the caller fills the
-// weights and, where gemm_q16_layers says more than one, `part` (layers * M * N floats).
+// weights and, where gemm_q16_layers says more than one, `part` (layers * M * N floats; without
+// it the spans run one after the other, with the same sums).
 struct QGemmArgs {
     const float* x;
     int ldx;

@@ -539,8 +539,8 @@ def test_linear_batch_forms(backend, wtype, tokens, rows, cols):
 @pytest.mark.parametrize("tokens", [5, 40, 200])
 def test_linear_batch_in_a_new_graph(tokens):
     """Captured with no earlier call of its size, so with no scratch of its own: the operands'
-    scratch is there from a larger call, partial sums stay in registers (or few rows go one
-    by one), and the replays agree with the eager call."""
+    scratch is there from a larger call, partial sums stay in registers, and the replays agree
+    with the eager call."""
     from emprise_amd import HipBackend
 
     rng = np.random.default_rng(tokens)
@@ -599,6 +599,37 @@ def test_graph_keeps_the_scratch_it_was_captured_with(tokens, cols):
         be.graph_destroy(g)
         be.linear_batch(w, x, y, tokens)
         assert np.array_equal(be.download(y, (tokens, rows)), eager)
+
+
+@pytest.mark.parametrize("wtype", [Q6_K, Q4_K])
+@pytest.mark.parametrize("q8,tokens,rows,cols", [(False, 5, 100, 4096), (False, 8, 33, 20480), (False, 17, 300, 2560),
+                                                 (True, 8, 200, 4096), (True, 32, 16, 1536)])
+def test_few_tokens_captured_without_scratch(wtype, q8, tokens, rows, cols):
+    """Few rows captured on a backend that has made no call: replays give the eager call's bits,
+    for two stacked weights and for gate and up of an FFN."""
+    from emprise_amd import HipBackend
+
+    rng = np.random.default_rng(tokens + cols)
+    with HipBackend(quantize_activations=q8) as be:
+        w = [be.upload_weight(wtype, cols, rows, matrix(rng, wtype, rows, cols)) for _ in range(2)]
+        x = be.to_device(rng.standard_normal((tokens, cols)).astype(np.float32))
+        y, f = be.alloc(tokens * 2 * rows * 4), be.alloc(tokens * rows * 4)
+
+        def run():
+            be.linear_batch_many(w, x, cols, y, 2 * rows, tokens)
+            be.ffn_gate_up_batch(w[0], w[1], x, cols, f, rows, tokens)
+        be.graph_begin()
+        run()
+        g = be.graph_end()
+        run()
+        want = be.download(y, (tokens, 2 * rows)), be.download(f, (tokens, rows))
+        assert np.all(np.isfinite(want[0])) and np.any(want[0])
+        for _ in range(3):
+            be.fill(y, 0.0, tokens * 2 * rows)
+            be.fill(f, 0.0, tokens * rows)
+            be.graph_launch(g)
+            assert np.array_equal(be.download(y, (tokens, 2 * rows)), want[0])
+            assert np.array_equal(be.download(f, (tokens, rows)), want[1])
 
 
 def _matvec_bound(W, x, rows_abs=0.0):
