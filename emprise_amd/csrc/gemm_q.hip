@@ -11,9 +11,11 @@
 //   most 63 * 15 = 945, exact in fp16 as it stands. The block scales d (and dmin) of each
 //   256 columns are applied in FP32 once per block.
 // - Activations. Each 256-column block of a row of X is scaled by a power of two 2^-e
-//   (exact) so that its largest magnitude lies in [2^8, 2^9) -- no fp16 overflow whatever
-//   the activations, in the values or in sums of 32 of them -- and split into xh = fp16(x)
-//   and xl = fp16(x - xh), which carry x to 22 significant bits.
+//   (exact) so that its largest magnitude lies in [2^14, 2^15) -- no fp16 overflow whatever
+//   the activations; sums of 32 of them are carried 2^-6 times as large -- and split into xh =
+//   fp16(x) and xl = fp16(x - xh), which carry 22 significant bits of every value down to 2^-16
+//   of the block's largest. For up to 8 tokens, which FP32 matvecs served before, a third piece
+//   carries the rest (split16).
 //
 // Per block the matrix cores accumulate, in FP32, sum v*xh + v*xl (+ vl*xh for Q6_K; the
 // dropped vl*xl is below 2^-21 of the term) and 2^e * d times that is added to the row's
@@ -66,13 +68,26 @@ constexpr int kTileHalves = 16 * kBlk * 2;  // a 16-token tile's pieces of one b
 
 // ---- activations: fp16 hi/lo pieces of 2^-e * x, and (for Q4_K) of its 32-column sums ----
 
+constexpr float kSumScale = 64.f;  // the unit sums are carried divided by this
+
 // One token's 16 columns 16c .. 16c+15 of a block, by thread c of the token's 16 threads (a
 // DPP row; all 16 call): slices 2(c%4), +1 of lane group q = c/4 into the tile's operands
 // (slice s, piece p, lane l -> halves ((2s + p)*64 + l)*8 .. +7), 2^e, and with `sums` lane
 // (i, q): the hi pieces of the sums over units 2q, 2q+1 (32 columns each), then their lo
 // pieces.
+//
+// EIGHT: for at most 8 tokens, whose pieces fill the tile: token i's high pieces are row i of
+// each slice's first operand, its low ones, carried 2^11 times as large, row i+8, and what
+// they leave row i+8 of the second operand (its rows 0..7 are zero; the sums' pieces alike).
+// So the products' rows 8..15 are the low part of tokens 0..7, to be added to rows 0..7, and
+// x is carried whole, 24 bits of every value down to 2^-26 of the block's largest (of unit
+// sums, 2^-20), as the FP32 matvecs that served these calls carried it. Error of an FFN's outputs
+// at 5 tokens against 64 bits, Q4_K 512 -> 1536 -> 512 / 4096 -> 12288 -> 4096: 1.25e-7 / 1.37e-7
+// (two pieces 1.65e-7 / 1.76e-7, the matvecs 1.30e-7 / 1.41e-7).
+template <bool EIGHT>
 __device__ __forceinline__ void split16(const float (&v)[16], int i, int c, _Float16* xf, float* xe, _Float16* xs,
                                         bool sums) {
+    constexpr float kLow = 2048.f;
     const int q = c >> 2;
     float mx = 0.f;
 #pragma unroll
@@ -84,33 +99,52 @@ __device__ __forceinline__ void split16(const float (&v)[16], int i, int c, _Flo
     int e = 0;
     if (mx > 0.f && mx < INFINITY) {
         (void)frexpf(mx, &e);      // mx = f * 2^e with f in [0.5, 1)
-        e = max(e - 9, -126);      // mx * 2^-e in [2^8, 2^9)
+        e = max(e - 15, -126);     // mx * 2^-e in [2^14, 2^15)
     }
     const float up = ldexpf(1.f, -e);
-    if (c == 0) xe[i] = ldexpf(1.f, e);
+    if (c == 0) {
+        xe[i] = ldexpf(1.f, e);
+        if constexpr (EIGHT) xe[i + 8] = ldexpf(1.f / kLow, e);
+    }
     _Float16* dst = xf + (q * 16 + i) * 8;
     float s = 0.f;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-        half8 hi, lo;
+        half8 hi, lo, rest;
+        float w[8];
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
-            const float w = v[8 * h + k] * up;
-            hi[k] = (_Float16)w;
-            lo[k] = (_Float16)(w - (float)hi[k]);
-            s += w;
+            w[k] = v[8 * h + k] * up;
+            hi[k] = (_Float16)w[k];
+            const float r = (w[k] - (float)hi[k]) * (EIGHT ? kLow : 1.f);
+            lo[k] = (_Float16)r;
+            rest[k] = (_Float16)(r - (float)lo[k]);
         }
-        const int slice = 2 * (c & 3) + h;
-        *reinterpret_cast<half8*>(dst + (2 * slice) * 512) = hi;
-        *reinterpret_cast<half8*>(dst + (2 * slice + 1) * 512) = lo;
+        s += ((w[0] + w[1]) + (w[2] + w[3])) + ((w[4] + w[5]) + (w[6] + w[7]));
+        _Float16* at = dst + (2 * (2 * (c & 3) + h)) * 512;
+        *reinterpret_cast<half8*>(at) = hi;
+        if constexpr (EIGHT) {
+            *reinterpret_cast<half8*>(at + 64) = lo;
+            *reinterpret_cast<half8*>(at + 512) = half8{};
+            *reinterpret_cast<half8*>(at + 512 + 64) = rest;
+        } else {
+            *reinterpret_cast<half8*>(at + 512) = lo;
+        }
     }
     if (sums) {
-        s += dpp_f<0xb1, 0xf>(0.f, s);                // the unit's two threads
+        s = (s + dpp_f<0xb1, 0xf>(0.f, s)) / kSumScale;  // the unit's two threads
         const float s1 = dpp_f<0x4e, 0xf>(0.f, s);    // lane group q's other unit
         if ((c & 3) == 0) {
             const _Float16 h0 = (_Float16)s, h1 = (_Float16)s1;
-            *reinterpret_cast<half4*>(xs + (q * 16 + i) * 4) =
-                half4{h0, h1, (_Float16)(s - (float)h0), (_Float16)(s1 - (float)h1)};
+            half4* at = reinterpret_cast<half4*>(xs + (q * 16 + i) * 4);
+            if constexpr (EIGHT) {
+                const float r0 = (s - (float)h0) * kLow, r1 = (s1 - (float)h1) * kLow;
+                const _Float16 l0 = (_Float16)r0, l1 = (_Float16)r1;
+                at[0] = half4{h0, h1, (_Float16)0.f, (_Float16)0.f};
+                at[8] = half4{l0, l1, (_Float16)(r0 - (float)l0), (_Float16)(r1 - (float)l1)};
+            } else {
+                at[0] = half4{h0, h1, (_Float16)(s - (float)h0), (_Float16)(s1 - (float)h1)};
+            }
         }
     }
 }
@@ -138,7 +172,7 @@ __global__ __launch_bounds__(256) void split_tiles_kernel(const float* __restric
     float v[16];
     load16(v, X, tile * 16 + i, M, ldx, blk * kBlk + 16 * c);
     const size_t at = (size_t)blk * tiles + tile;
-    split16(v, i, c, xf + at * kTileHalves, xe + at * 16, xs + at * 256, xs != nullptr);
+    split16<false>(v, i, c, xf + at * kTileHalves, xe + at * 16, xs + at * 256, xs != nullptr);
 }
 
 // ---- weights ---------------------------------------------------------------------------
@@ -251,7 +285,7 @@ __device__ __forceinline__ void q_block_end(const uint4* side, int lane, const u
                 const half2v mm = __builtin_bit_cast(half2v, mins[i]);
                 const half8 mv = {mm[0], mm[1], mm[0], mm[1], (_Float16)0.f, (_Float16)0.f, (_Float16)0.f, (_Float16)0.f};
                 cm = __builtin_amdgcn_mfma_f32_16x16x32_f16(xsum, mv, cm, 0, 0, 0);
-                dm = half_bits_to_float((uint16_t)(dblk[i] >> 16));
+                dm = half_bits_to_float((uint16_t)(dblk[i] >> 16)) * kSumScale;
             }
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
@@ -485,6 +519,7 @@ __global__ __launch_bounds__(WV * 64, OCC) void gemm_q16_kernel(QGemmArgs a) {
 // its span of the activations itself (no pass before it), keeps all of it in LDS, and its
 // waves then walk row tiles on their own.
 constexpr int kFewSpan = 4;
+constexpr int kEight = 8;  // tokens at most whose pieces share a 16-token tile (split16)
 template <int T, int MT> struct Few {
     static constexpr int AV = MT * 1024;                        // 16-byte pieces of a block's operands
     static constexpr int SV = MT * (T == kQ4K ? 36 : 4);        // of its side data
@@ -494,12 +529,23 @@ template <int T, int MT> struct Few {
 // Blocks b0 .. b0+nbs-1 of the activations.
 template <int T, int MT> __device__ __forceinline__ void few_stage(const QGemmArgs& a, int b0, int nbs, Few<T, MT>& lds) {
     using F = Few<T, MT>;
+    if (MT == 1 && a.M <= kEight) {
+        for (int t = threadIdx.x; t < nbs * 128; t += blockDim.x) {
+            const int bl = t >> 7, i = (t >> 4) & 7, c = t & 15;
+            float v[16];
+            load16(v, a.x, i, a.M, a.ldx, (b0 + bl) * kBlk + 16 * c);
+            uint4* side = lds.side + bl * F::SV;
+            split16<true>(v, i, c, reinterpret_cast<_Float16*>(lds.x + bl * F::AV), reinterpret_cast<float*>(side),
+                          reinterpret_cast<_Float16*>(side + 4), T == kQ4K);
+        }
+        return;
+    }
     for (int t = threadIdx.x; t < nbs * MT * 256; t += blockDim.x) {
         const int u = t >> 8, i = (t >> 4) & 15, c = t & 15, bl = u / MT, m = u - bl * MT;
         float v[16];
         load16(v, a.x, m * 16 + i, a.M, a.ldx, (b0 + bl) * kBlk + 16 * c);
         uint4* side = lds.side + bl * F::SV;
-        split16(v, i, c, reinterpret_cast<_Float16*>(lds.x + bl * F::AV + m * 1024), reinterpret_cast<float*>(side + 4 * m),
+        split16<false>(v, i, c, reinterpret_cast<_Float16*>(lds.x + bl * F::AV + m * 1024), reinterpret_cast<float*>(side + 4 * m),
                 reinterpret_cast<_Float16*>(side + 4 * MT + 32 * m), T == kQ4K);
     }
 }
@@ -555,6 +601,17 @@ __device__ __forceinline__ void few_block(const QRaw<T>& raw, const Few<T, MT>& 
     q_block_end<T, 1, MT>(lds.side + bl * F::SV, lane, dblk, mins, cb, acc);
 }
 
+// The tile's sums, of kEight tokens or fewer with their low part from the rows 8 further on
+// (lanes 32 further on; what this leaves in those lanes is not stored).
+template <int MT> __device__ __forceinline__ void few_finish(const QGemmArgs& a, floatx4 (&acc)[1][MT]) {
+    if (MT > 1 || a.M > kEight) return;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[0][0][r]), __float_as_uint(acc[0][0][r]), false, false);
+        acc[0][0][r] = __uint_as_float(s[0]) + __uint_as_float(s[1]);
+    }
+}
+
 // No barrier after the staging, two blocks' weights in flight per wave; each tile's sums over
 // the span go to part[z]. Grid: x = workgroups over the rows, z = spans of kFewSpan blocks.
 template <int T, bool CH, int MT>
@@ -601,6 +658,7 @@ __global__ __launch_bounds__(1024) void gemm_q16_few_kernel(QGemmArgs a) {
     auto compute = [&](const QRaw<T>& raw) {
         few_block<T, CH, MT>(raw, lds, bl, lane, acc);
         if (++bl == nbs) {
+            few_finish<MT>(a, acc);
             q_store<1, MT>(a, tile * 16, 0, rj, q, acc);
 #pragma unroll
             for (int m = 0; m < MT; ++m) acc[0][m] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -643,6 +701,7 @@ __global__ __launch_bounds__(512) void gemm_q16_few_serial_kernel(QGemmArgs a) {
                 q_load<CH>(raw, row, nb, b0 + bl, q);
                 few_block<T, CH, MT>(raw, lds, bl, lane, acc);
             }
+            few_finish<MT>(a, acc);
 #pragma unroll
             for (int m = 0; m < MT; ++m)
 #pragma unroll

@@ -602,6 +602,44 @@ def test_graph_keeps_the_scratch_it_was_captured_with(tokens, cols):
 
 
 @pytest.mark.parametrize("wtype", [Q6_K, Q4_K])
+@pytest.mark.parametrize("tokens,cols", [(2, 768), (5, 4096), (8, 1280), (9, 768), (70, 512), (200, 4096)])
+def test_small_activations_beside_large_ones(backend, wtype, tokens, cols):
+    """Of each 256 columns the first 32 are large and their weights zero, and one other value is
+    2^-down of theirs: up to 8 tokens carry it whole, more to 22 bits and at 2^-20 to 18. Q4_K's
+    unit sums are carried 2^-6 as large."""
+    rng = np.random.default_rng(tokens + cols)
+    down = (26 if tokens <= 8 else 20) - (6 if wtype == Q4_K else 0)
+    rows = 40
+    data = np.frombuffer(matrix(rng, wtype, rows, cols), np.uint8).reshape(rows * cols // 256, -1).copy()
+    if wtype == Q6_K:
+        data[:, 192:194] = 0  # the scales of the first two units
+    else:
+        data[:, 4] &= 0xC0    # scale and min of the first unit
+        data[:, 8] &= 0xC0
+    x = np.zeros((tokens, cols // 256, 256), np.float32)
+    x[:, :, :32] = rng.uniform(0.5, 1.0, (tokens, cols // 256, 32))
+    at = rng.integers(32, 256, cols // 256)
+    for b, i in enumerate(at):
+        x[:, b, i] = rng.uniform(0.5, 1.0, tokens) * 2.0**-down
+    x = x.reshape(tokens, cols)
+    w = backend.upload_weight(wtype, cols, rows, data.tobytes())
+    xd, yd, wd = backend.to_device(x), backend.alloc(tokens * rows * 4), backend.alloc(rows * cols * 4)
+    backend.linear_batch(w, xd, yd, tokens)
+    Y = backend.download(yd, (tokens, rows)).astype(np.float64)
+    backend.dequantize_rows(w, 0, rows, wd)
+    W = backend.download(wd, (rows, cols)).astype(np.float64)
+    small = np.abs(x) * (np.arange(cols) % 256 >= 32)
+    size = small.astype(np.float64) @ np.abs(W).T
+    if wtype == Q4_K:  # d*sc*q and dmin*m are summed apart, each at most |w| + dmin*m in size
+        size += small.sum(1, keepdims=True) * 2 * np.abs(W).max()
+    bits = 2.0**-23 if tokens <= 8 else 2.0**-18
+    assert np.all(np.abs(Y - x.astype(np.float64) @ W.T) <= (bits + 2.0**-24 * (2 * cols // 256 + 8)) * size)
+    for b in (xd, yd, wd):
+        backend.free(b)
+    backend.weight_free(w)
+
+
+@pytest.mark.parametrize("wtype", [Q6_K, Q4_K])
 @pytest.mark.parametrize("q8,tokens,rows,cols", [(False, 5, 100, 4096), (False, 8, 33, 20480), (False, 17, 300, 2560),
                                                  (True, 8, 200, 4096), (True, 32, 16, 1536)])
 def test_few_tokens_captured_without_scratch(wtype, q8, tokens, rows, cols):
