@@ -943,6 +943,15 @@ template <int G> __device__ __forceinline__ float sum_lanes(float v) {
     return v;
 }
 
+// 1 / sqrt(sum / n + eps), rounded once: its error is common to all outputs of the layer, which
+// is most of what they are off by. A Newton step in FP64 from the FP32 estimate.
+__device__ __forceinline__ float norm_scale(float sum, int n, float eps) {
+    const double t = (double)sum / (double)n + (double)eps;
+    const float y = rsqrtf((float)t);
+    const double z = (double)y * (1.5 - 0.5 * t * (double)y * (double)y);
+    return y > 0.f && y < INFINITY ? (float)z : y;
+}
+
 // xs and usum (stored_unit_sum of each unit, in order) from x + delta, normalised.
 template <int UNIT> __device__ __forceinline__ void stage_rows(const MvArgs& a, float4* xs, float* usum, float* red) {
     constexpr int TH = kRowWaves * 64;
@@ -973,7 +982,7 @@ template <int UNIT> __device__ __forceinline__ void stage_rows(const MvArgs& a, 
         }
     }
     float scale = 1.f;
-    if (w4) scale = 1.f / sqrtf(block_sum_lds(ss, red) / (float)a.cols + a.eps);
+    if (w4) scale = norm_scale(block_sum_lds(ss, red), a.cols, a.eps);
 #pragma unroll
     for (int k = 0; k < kRowStage; ++k) {
         if (k * TH >= n4) continue;
