@@ -77,10 +77,11 @@ template <int E> __device__ __forceinline__ void stv(float* p, const float (&v)[
 //
 // ranges: kAttnFew while they give every CU a workgroup and the range is short, else
 // kAttnSplit, two workgroups per CU, so that 16 waves' rows are in flight. The second 64
-// partials cost the merge a round trip behind the position read (4 KV heads x 256, us with
-// 128 and 64 ranges: 19.0 / 16.7 at 4000 positions, 27.6 / 22.3 at 8000, 32.3 / 36.2 at
-// 16000, 53.3 / 63.3 at 30000). Two KV heads fill the chip only with 128 (10.9 / 12.1 at
-// 4000, 28.8 / 48.5 at 30000).
+// partials cost the merge a round trip behind the position read (4 KV heads x 256, graph
+// replays, us with 128 and 64 ranges: 14.0 / 12.6 at 2000 positions, 17.1 / 16.2 at 4000, 19.6 /
+// 19.2 at 6000, 22.2 / 22.5 at 8000, 23.0 / 23.9 at 8250, 28.1 / 31.6 at 12000, 35.9 / 39.6 at
+// 16000; the empty workgroups of a short context cost nothing that shows, 8.6 at 200 either way).
+// Two KV heads fill the chip only with 128 (10.4 / 12.0 at 4000).
 __device__ __forceinline__ int attn_per(int len, int kv_heads) {
     const int nsub = (len + kAttnSub - 1) / kAttnSub;
     const int ranges = kv_heads * kAttnFew < 256 || nsub > kAttnLong ? kAttnSplit : kAttnFew;
