@@ -948,12 +948,20 @@ hipError_t launch_gemm_q16_split(const float* X, int M, int K, int ldx, void* sc
 
 bool gemm_q16_few(int M) { return M <= 32; }
 
-// Column spans of a product with M tokens and K columns.
+// Column spans of a product with M tokens and K columns. The rows may not enter (a row's sums
+// are the same bits whichever rows share its launch), so they are guessed from K. Wide inputs
+// are taken for those of down projections, with K/3 rows, and get spans for one workgroup of 128
+// x 128 per CU; narrower ones for the hidden state, whose projections have more rows and pay for
+// each span with partial sums. Where widths may be either, few spans are the smaller loss: FFNs
+// at 6144 hidden values or more are rare, and below that both kinds occur. us with few spans / with
+// the wide rule's, at 300 and 700 tokens: FFN 4096 -> 5632 -> 4096, Q4_K, 700 only, 378 / 447; 4096 ->
+// 5120 167 / 190 at 300; 5120 columns x 30720 rows, Q6_K, 350 / 437 and 606 / 759; but FFN 2048 -> 5888
+// 174 / 138 and 260 / 216, 1536 -> 4608 120 / 96 and 175 / 130 (rows near K/3, which the line gives up).
 int gemm_q16_spans(int M, int K) {
     const int nb = K / kBlk, groups = (M + 127) / 128;
     int spans;
     if (M <= 64) spans = (nb + kFewSpan - 1) / kFewSpan;
-    else if (K >= 6144) spans = std::max(1, 8 * 12288 / K / groups);
+    else if (K >= 6144) spans = std::max(1, 3 * 128 * kCUs / K / groups);
     else spans = groups == 1 ? 4 : groups <= 4 ? 2 : 1;
     spans = std::max(1, std::min(spans, nb / 2));
     const int span = (nb + spans - 1) / spans;  // blocks in each but the last
