@@ -359,46 +359,43 @@ __device__ __forceinline__ void q_store(const QGemmArgs& a, int n0, int t0, int 
     }
 }
 
-// The general form. A workgroup of WV waves covers WV*16*RT weight rows x 16*MT tokens; all
-// waves share the token operands, double-buffered in LDS UPS units (16 columns per lane) at
-// a time, one barrier per step; a wave decodes each weight once for its 16*MT tokens.
-// T: weight type; CH: chunked layout; MT: 16-token tiles and RT: 16-row tiles per wave; WV:
-// waves per workgroup; UPS: unit steps per LDS step; PF: the next block's weights are
+// The general form. A workgroup of MT waves covers 16*MT weight rows x 16*MT tokens; all waves
+// share the token operands, double-buffered in LDS one unit step (16 columns per lane) at a
+// time, one barrier per step; a wave decodes each weight once for its 16*MT tokens.
+// T: weight type; CH: chunked layout; MT: 16-token tiles; PF: the next block's weights are
 // loaded a whole block ahead (a second register set) instead of during the block's last
 // unit step. Grid: x = row groups, y = token groups, z = column spans. a.spans > 1 with one
 // z layer runs the spans one after the other, adding them in the order the reduction
 // would, so the results do not depend on which of the two forms ran.
-template <int T, bool CH, int MT, int RT, int WV, int UPS, bool PF, int OCC>
-__global__ __launch_bounds__(WV * 64, OCC) void gemm_q16_kernel(QGemmArgs a) {
-    constexpr int TH = WV * 64;                         // threads
-    constexpr int SPB = 4 / UPS;                        // steps per block
-    constexpr int AV = MT * UPS * 4096 / 16;            // 16-byte pieces of a step's operands
-    constexpr int AN = (AV + TH - 1) / TH;
+template <int T, bool CH, int MT, bool PF>
+__global__ __launch_bounds__(MT * 64, 2) void gemm_q16_kernel(QGemmArgs a) {
+    constexpr int TH = MT * 64;                         // threads
+    constexpr int AV = MT * 256;                        // 16-byte pieces of a step's operands
+    constexpr int AN = AV / TH;
     constexpr int SV = MT * (T == kQ4K ? 36 : 4);       // of a block's side data: 2^e, then the unit sums
     constexpr int SN = (SV + TH - 1) / TH;
-    constexpr int MP = MT >= 4 && RT == 1 ? 4 : MT >= 2 ? 2 : 1;
+    constexpr int MP = 4;
     __shared__ __align__(16) uint4 As[2][AV];
     __shared__ __align__(16) uint4 Ss[2][SV];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int q = lane >> 4, rj = lane & 15;
     const int tiles = (a.M + 15) >> 4, nb = a.K / kBlk;
-    const int t0 = blockIdx.y * MT, n0 = (blockIdx.x * WV + wave) * (16 * RT);
+    const int t0 = blockIdx.y * MT, n0 = (blockIdx.x * MT + wave) * 16;
     const int b0 = gridDim.z > 1 ? blockIdx.z * a.span : 0;
     const int b1 = gridDim.z > 1 ? min(b0 + a.span, nb) : nb;
 
-    const uint8_t* row[RT];  // (rows past N read the last row; their results are not stored)
-#pragma unroll
-    for (int i = 0; i < RT; ++i) row[i] = q_row<T>(a, min(n0 + 16 * i + rj, a.N - 1), nb);
+    // (rows past N read the last row; their results are not stored)
+    const uint8_t* row = q_row<T>(a, min(n0 + rj, a.N - 1), nb);
 
-    // step s (global numbering: block s / SPB, unit steps UPS * (s % SPB) ..)
+    // step s (global numbering): unit step s % 4 of block s / 4
     uint4 ra[AN], rs[SN];
     auto load_a = [&](int s) {
-        const int b = s / SPB, j = s - b * SPB;
+        const int b = s / 4, j = s - b * 4;
 #pragma unroll
         for (int k = 0; k < AN; ++k) {
-            const int v = min(k * TH + tid, AV - 1), tile = v / (UPS * 256), o = v - tile * (UPS * 256);
-            ra[k] = gld16(a.xf + ((size_t)b * tiles + min(t0 + tile, tiles - 1)) * kTileHalves + (size_t)(j * UPS * 256 + o) * 8);
+            const int v = min(k * TH + tid, AV - 1), tile = v / 256, o = v - tile * 256;
+            ra[k] = gld16(a.xf + ((size_t)b * tiles + min(t0 + tile, tiles - 1)) * kTileHalves + (size_t)(j * 256 + o) * 8);
         }
         if (j == 0) {
 #pragma unroll
@@ -406,11 +403,11 @@ __global__ __launch_bounds__(WV * 64, OCC) void gemm_q16_kernel(QGemmArgs a) {
         }
     };
     auto store_a = [&](int s, int buf) {
-        const int b = s / SPB, j = s - b * SPB;
+        const int b = s / 4, j = s - b * 4;
 #pragma unroll
         for (int k = 0; k < AN; ++k) {
             const int v = k * TH + tid;
-            if (AV % TH == 0 || v < AV) As[buf][v] = ra[k];
+            As[buf][v] = ra[k];
         }
         if (j == 0) {
 #pragma unroll
@@ -421,55 +418,40 @@ __global__ __launch_bounds__(WV * 64, OCC) void gemm_q16_kernel(QGemmArgs a) {
         }
     };
 
-    floatx4 cb[RT][MT], acc[RT][MT], tot[RT][MT];
+    floatx4 cb[1][MT], acc[1][MT], tot[MT];
 #pragma unroll
-    for (int i = 0; i < RT; ++i)
-#pragma unroll
-        for (int m = 0; m < MT; ++m) {
-            cb[i][m] = acc[i][m] = floatx4{0.f, 0.f, 0.f, 0.f};
-            tot[i][m] = floatx4{0.f, 0.f, 0.f, 0.f};
-        }
+    for (int m = 0; m < MT; ++m) cb[0][m] = acc[0][m] = tot[m] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-    QRaw<T> raw[RT], nxt[PF ? RT : 1];
-    const int s0 = b0 * SPB, s1 = b1 * SPB;
+    QRaw<T> raw, nxt;
+    const int s0 = b0 * 4, s1 = b1 * 4;
     load_a(s0);
-#pragma unroll
-    for (int i = 0; i < RT; ++i) q_load<CH>(raw[i], row[i], nb, b0, q);
+    q_load<CH>(raw, row, nb, b0, q);
     store_a(s0, s0 & 1);
     load_a(min(s0 + 1, s1 - 1));
     lds_barrier();
 
     for (int b = b0; b < b1; ++b) {
-        if constexpr (PF) {
+        if constexpr (PF) q_load<CH>(nxt, row, nb, min(b + 1, b1 - 1), q);
+        uint32_t dblk[1], mins[1];
+        q_block_scales<CH>(raw, q, dblk[0], mins[0]);
 #pragma unroll
-            for (int i = 0; i < RT; ++i) q_load<CH>(nxt[i], row[i], nb, min(b + 1, b1 - 1), q);
-        }
-        uint32_t dblk[RT], mins[RT];
-#pragma unroll
-        for (int i = 0; i < RT; ++i) q_block_scales<CH>(raw[i], q, dblk[i], mins[i]);
-#pragma unroll
-        for (int js = 0; js < SPB; ++js) {
-            const int s = b * SPB + js, buf = s & 1;
+        for (int j = 0; j < 4; ++j) {
+            const int s = b * 4 + j, buf = s & 1;
             // the next step's operands go into the buffer that every wave finished with
-            // before the last barrier; their loads had a whole step
-            if (s + 1 < s1) store_a(s + 1, buf ^ 1);
-            load_a(min(s + 2, s1 - 1));
+            // before the last barrier; their loads had a whole step (with PF behind the decode: FFN
+            // 2048 -> 6144 of 50 tokens, Q4_K, 51.2 us, before it 52.3)
+            auto stage = [&] {
+                if (s + 1 < s1) store_a(s + 1, buf ^ 1);
+                load_a(min(s + 2, s1 - 1));
+            };
+            if constexpr (!PF) stage();
             const half8* A = reinterpret_cast<const half8*>(As[buf]);
-#pragma unroll
-            for (int ju = 0; ju < UPS; ++ju) {
-                const int j = js * UPS + ju;
-                half8 wh[RT][2], wl[RT][2];
-#pragma unroll
-                for (int i = 0; i < RT; ++i) {
-                    if constexpr (T == kQ6K) q6_unit(raw[i], j, wh[i], wl[i]);
-                    else q4_unit<CH>(raw[i], q, j, wh[i]);
-                }
-                if constexpr (!PF) {
-                    if (j == 3) {
-#pragma unroll
-                        for (int i = 0; i < RT; ++i) q_load<CH>(raw[i], row[i], nb, min(b + 1, b1 - 1), q);
-                    }
-                }
+            auto products = [&] {
+                half8 wh[1][2], wl[1][2];
+                if constexpr (T == kQ6K) q6_unit(raw, j, wh[0], wl[0]);
+                else q4_unit<CH>(raw, q, j, wh[0]);
+                if constexpr (PF) stage();
+                else if (j == 3) q_load<CH>(raw, row, nb, min(b + 1, b1 - 1), q);
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
                     // MP token tiles at a time: consecutive MFMAs add to different accumulators
@@ -478,41 +460,35 @@ __global__ __launch_bounds__(WV * 64, OCC) void gemm_q16_kernel(QGemmArgs a) {
                         half8 xh[MP], xl[MP];
 #pragma unroll
                         for (int u = 0; u < MP; ++u) {
-                            xh[u] = A[(m + u) * (UPS * 256) + (ju * 4 + 2 * h) * 64 + lane];
-                            xl[u] = A[(m + u) * (UPS * 256) + (ju * 4 + 2 * h + 1) * 64 + lane];
+                            xh[u] = A[(m + u) * 256 + (2 * h) * 64 + lane];
+                            xl[u] = A[(m + u) * 256 + (2 * h + 1) * 64 + lane];
                         }
-                        q_products<T, RT, MP, MT>(xh, xl, wh, wl, h, m, cb);
+                        q_products<T, 1, MP, MT>(xh, xl, wh, wl, h, m, cb);
                     }
                 }
-            }
-            if (js == SPB - 1) {
-                q_block_end<T, RT, MT>(Ss[b & 1], lane, dblk, mins, cb, acc);
+            };
+            products();
+            if (j == 3) {
+                q_block_end<T, 1, MT>(Ss[b & 1], lane, dblk, mins, cb, acc);
                 if (gridDim.z == 1 && a.spans > 1 && ((b + 1) % a.span == 0 || b + 1 == b1)) {
 #pragma unroll
-                    for (int i = 0; i < RT; ++i)
+                    for (int m = 0; m < MT; ++m)
 #pragma unroll
-                        for (int m = 0; m < MT; ++m)
-#pragma unroll
-                            for (int r = 0; r < 4; ++r) {
-                                tot[i][m][r] += acc[i][m][r];
-                                acc[i][m][r] = 0.f;
-                            }
+                        for (int r = 0; r < 4; ++r) {
+                            tot[m][r] += acc[0][m][r];
+                            acc[0][m][r] = 0.f;
+                        }
                 }
             }
             lds_barrier();
         }
-        if constexpr (PF) {
-#pragma unroll
-            for (int i = 0; i < RT; ++i) raw[i] = nxt[i];
-        }
+        if constexpr (PF) raw = nxt;
     }
     if (gridDim.z == 1 && a.spans > 1) {
 #pragma unroll
-        for (int i = 0; i < RT; ++i)
-#pragma unroll
-            for (int m = 0; m < MT; ++m) acc[i][m] = tot[i][m];
+        for (int m = 0; m < MT; ++m) acc[0][m] = tot[m];
     }
-    q_store<RT, MT>(a, n0, t0, rj, q, acc);
+    q_store<1, MT>(a, n0, t0, rj, q, acc);
 }
 
 // The forms for up to 32 tokens, where the weights' bytes are the bound: a workgroup splits
@@ -901,23 +877,22 @@ hipError_t launch_grid(F kernel, int mt, int rows, int threads, const QGemmArgs&
     return launch_reduce(a, layers, stream);
 }
 
-template <int T, bool CH, int MT, int RT, int WV, int UPS, bool PF, int OCC>
-hipError_t launch_form(const QGemmArgs& a, int layers, hipStream_t stream) {
-    return launch_grid(gemm_q16_kernel<T, CH, MT, RT, WV, UPS, PF, OCC>, MT, WV * RT * 16, WV * 64, a, layers, stream);
+template <int T, bool CH, int MT, bool PF> hipError_t launch_form(const QGemmArgs& a, int layers, hipStream_t stream) {
+    return launch_grid(gemm_q16_kernel<T, CH, MT, PF>, MT, MT * 16, MT * 64, a, layers, stream);
 }
 
 template <int T, bool CH> hipError_t launch_type(const QGemmArgs& a, int layers, hipStream_t stream) {
     const int mt = tiles_for(a.M);
     if (mt == 1) return launch_few<T, CH, 1>(a, layers, stream);
     if (mt == 2) return launch_few<T, CH, 2>(a, layers, stream);
-    if (mt == 4) return launch_form<T, CH, 4, 1, 4, 1, true, 2>(a, layers, stream);
+    if (mt == 4) return launch_form<T, CH, 4, true>(a, layers, stream);
     // 256 rows per workgroup, or 128 where that fills the last round of workgroups better
     // (a workgroup of half the rows takes a bit over half the time)
     const int groups = ((a.M + 127) / 128) * layers;
     const int wide = (groups * ((a.N + 255) / 256) + kCUs - 1) / kCUs;
     const int half = (groups * ((a.N + 127) / 128) + kCUs - 1) / kCUs;
     if (half * 6 < wide * 10 || (layers == 1 && a.spans > 1) || a.M > (1 << 22))
-        return launch_form<T, CH, 8, 1, 8, 1, false, 2>(a, layers, stream);
+        return launch_form<T, CH, 8, false>(a, layers, stream);
     return launch_grid(gemm_q16_wide_kernel<T, CH>, 8, 256, 512, a, layers, stream);
 }
 
