@@ -536,6 +536,70 @@ def test_linear_batch_forms(backend, wtype, tokens, rows, cols):
     backend.weight_free(w)
 
 
+def _wide_form(tokens, rows, cols):
+    """Whether the GEMM takes its form of 256 weight rows per workgroup (launch_type's rule, with
+    gemm_q16_spans and gemm_q16_layers): where those workgroups fill their rounds of 256 better."""
+    blocks, groups = cols // 256, -(-tokens // 128)
+    spans = max(1, 98304 // cols // groups) if cols >= 6144 else 4 if groups == 1 else 2 if groups <= 4 else 1
+    spans = max(1, min(spans, blocks // 2))
+    spans = -(-blocks // -(-blocks // spans))
+    layers = 1 if rows >= 65536 or spans * tokens * rows > 64 << 20 else spans
+    wide, half = -(-groups * layers * -(-rows // 256) // 256), -(-groups * layers * -(-rows // 128) // 256)
+    return tokens > 64 and half * 6 >= wide * 10 and (layers > 1 or spans == 1)
+
+
+# the last workgroup's rows and tokens not full, one and two column spans, an odd number of blocks
+# in the last, weights that end inside a workgroup and inside a 16-row tile, both layouts
+@pytest.mark.parametrize("wtype", [Q6_K, Q4_K])
+@pytest.mark.parametrize("tokens,rows,cols", [(70, [33000], 256), (65, [17001], 1280), (2048, [2100], 768),
+                                              (1930, [1000, 7, 1094], 512), (2035, [2050], 4096), (600, [3000, 303], 8192),
+                                              (1100, [3, 3700], 2048)])
+def test_linear_batch_wide_form(backend, wtype, tokens, rows, cols):
+    """The prefill GEMM of 256-row workgroups against 64 bits."""
+    rng = np.random.default_rng(tokens + cols + wtype)
+    n, be = sum(rows), backend
+    assert _wide_form(tokens, n, cols)
+    data = [matrix(rng, wtype, r, cols) for r in rows]
+    w = [be.upload_weight(wtype, cols, r, d) for r, d in zip(rows, data)]
+    X = (rng.standard_normal((tokens, cols)) * 10.0 ** rng.uniform(-3, 3, (tokens, 1))).astype(np.float32)
+    xd, yd, wd = be.to_device(X), be.alloc(tokens * n * 4), be.alloc(max(rows) * cols * 4)
+    be.linear_batch_many(w, xd, cols, yd, n, tokens)
+    Y = be.download(yd, (tokens, n))
+    first = 0
+    for wt, r in zip(w, rows):
+        be.dequantize_rows(wt, 0, r, wd)
+        W = be.download(wd, (r, cols))
+        ref = X.astype(np.float64) @ W.astype(np.float64).T
+        extra = 2.0**-18 * np.abs(X).sum(1, keepdims=True) * np.abs(W).max() if wtype == Q4_K else 0.0
+        assert np.all(np.abs(Y[:, first:first + r] - ref) <= _gemm_bound(W, X, cols) + extra)
+        first += r
+    for b in (xd, yd, wd):
+        be.free(b)
+    for wt in w:
+        be.weight_free(wt)
+
+
+@pytest.mark.parametrize("wtype", [Q6_K, Q4_K])
+@pytest.mark.parametrize("tokens,rows,cols", [(2040, 1100, 768), (1500, 1400, 4096), (600, 1650, 8192)])
+def test_gate_up_wide_form(backend, wtype, tokens, rows, cols):
+    """Its SwiGLU epilogue against the two products, bit for bit."""
+    rng = np.random.default_rng(tokens + cols + wtype)
+    be = backend
+    assert _wide_form(tokens, 2 * rows, cols)
+    w = [be.upload_weight(wtype, cols, rows, matrix(rng, wtype, rows, cols)) for _ in range(2)]
+    xd = be.to_device(rng.standard_normal((tokens, cols)).astype(np.float32))
+    y = [be.alloc(tokens * rows * 4) for _ in range(3)]
+    be.ffn_gate_up_batch(w[0], w[1], xd, cols, y[0], rows, tokens)
+    be.linear_batch(w[0], xd, y[1], tokens)
+    be.linear_batch(w[1], xd, y[2], tokens)
+    be.swiglu(y[1], y[2], tokens * rows)
+    assert np.array_equal(be.download(y[0], tokens * rows), be.download(y[1], tokens * rows))
+    for b in [xd] + y:
+        be.free(b)
+    for wt in w:
+        be.weight_free(wt)
+
+
 @pytest.mark.parametrize("tokens", [5, 40, 200])
 def test_linear_batch_in_a_new_graph(tokens):
     """Captured with no earlier call of its size, so with no scratch of its own: the operands'
