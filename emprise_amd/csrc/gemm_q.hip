@@ -42,7 +42,7 @@
 // that decoded the weights into LDS for 128 x 128 tiles (chunked layout) or dequantised
 // them to FP32 (the others), graph replays over distinct weights, us, Q6_K gate+up rows
 // 24576 x 4096 and down rows 4096 x 12288: 5 tokens 34 + 26 (58 + 34 as small-batch
-// matvecs), 99 tokens 100 + 52 (the FFN 384 before, 158 now), 2048 tokens 980 + 515 (1276 +
+// matvecs), 99 tokens 100 + 52 (the FFN 384 before, 158 now), 2048 tokens 950 + 503 (1276 +
 // 620); Q4_K 12288 x 2048 and 2048 x 6144 at 700 tokens 148 + 85 (the FFN 1151 before, 219
 // now).
 //
@@ -698,15 +698,14 @@ __global__ __launch_bounds__(512) void gemm_q16_few_serial_kernel(QGemmArgs a) {
 // multiply phase of 96 (Q6_K) or 64 MFMAs with their LDS reads, a barrier after each.
 // Waves 4..7 run one phase behind waves 0..3 (one of each on every SIMD), so that one
 // group's vector work always runs beside the other's matrix work. Three operand buffers:
-// both groups write step s+1 while the slower one still reads step s-1. At 2048 tokens x
-// 24576 x 4096 the matrix cores are 59% busy at the 2.0 GHz the card holds there (1.2
-// PFLOP/s of fp16 products; a chain of MFMAs on registers alone holds 1.4 to 1.9 with data
-// like these): 980 us, 1050 with all eight waves in one phase. Without the decode, the
-// staging or the block scaling it would be 9%, 7% and 6% shorter; without its LDS reads no
-// shorter.
+// both groups write step s+1 while the slower one still reads step s-1. Bound by the matrix
+// cores and the registers: operands are read one pair ahead, not two, which for Q4_K spilled 33
+// to 60 of them (2048 tokens x 12352 x 4096, Q4_K / Q6_K, 542 / 628 us, with two 813 / 639; the kernel of
+// 128 x 128 tiles before this one 631 / 707). 2048 tokens x 24576 x 4096 in SwiGLU pairs 818 / 950 us:
+// 1.0 / 1.3 PFLOP/s of fp16 products, where an 8192^3 fp16 product of the library holds 1.1.
 template <int T, bool CH>
 __global__ __launch_bounds__(512, 2) void gemm_q16_wide_kernel(QGemmArgs a) {
-    constexpr int MT = 8, RT = 2, TH = 512, XD = 2;
+    constexpr int MT = 8, RT = 2, TH = 512, XD = 1;
     constexpr int AV = MT * 256, AN = AV / TH;
     constexpr int SV = MT * (T == kQ4K ? 36 : 4);
     __shared__ __align__(16) uint4 As[3][AV];
