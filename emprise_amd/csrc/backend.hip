@@ -631,17 +631,28 @@ static int small_batch(const emprise_hip* h, const Weight* wt) {
     return per;
 }
 
+// Whether two rows go one by one through this weight, of a width that the small-batch kernel does
+// not take: two matvecs against the GEMM and its reduction, which for small matrices is mostly
+// waiting (us, Q6_K: 512 x 1536 7.9 / 12.6, 2048 x 2048 7.9 / 13.0, 3072 x 3072 9.7 / 11.1, 2048 x 6144
+// 11.5 / 11.8; 512 columns 7.9 / 6.6, 2560 x 7680 14.9 / 13.7, 18432 x 3072 22.8 / 18.9; as gate and up,
+// Q4_K, 768 -> 2304 9.5 / 8.3, 1024 -> 3072 9.5 / 10.2, 1536 -> 4608 15.4 / 12.2). The matrix's own rows
+// count, not those it is called with, so its results are the same bits in every call.
+static bool by_row(const emprise_hip* h, const Weight* wt, int K) {
+    return K == 2 && !chunked_cols(wt->cols) && !(h->q8 && wt->type == kQ6K) && wt->cols > 512 &&
+           wt->rows * wt->cols <= (10u << 20);
+}
+
 // Whether K rows of X (16-byte aligned rows) go through this weight as a GEMM. Q6_K/Q4_K:
 // once the rows no longer fit one small-batch launch, which reads the weights once as well
 // (us, one launch against the GEMM's two: Q6_K 4096 x 4096 9.3 / 14.3 at 4 rows and 15.1 /
 // 14.4 at 5, 4096 x 12288 19.6 / 26.0 at 3 and 29.0 / 26.0 at 4); widths the small-batch
-// kernel does not take from 2 rows on (2048 x 6144 at 3 rows 27.4 as three matvecs, 14.0).
+// kernel does not take from 2 or 3 rows on (2048 x 6144 at 3 rows 27.4 as three matvecs, 14.0).
 // Q6_K under --fast-q8 keeps the single-input path, which quantises its input, up to
 // kGemmMinBatch, as do the unquantised types, whose GEMM fills 128-row tiles.
 static bool on_gemm(const emprise_hip* h, const Weight* wt, int K) {
     if (wt->type != kQ6K && wt->type != kQ4K) return K >= kGemmMinBatch && wt->cols % 16 == 0;
     if (K < kGemmMinBatch && ((h->q8 && wt->type == kQ6K) || wt->cols > kMatvecMaxCols)) return false;
-    return K > small_batch(h, wt);
+    return K > small_batch(h, wt) && !by_row(h, wt, K);
 }
 
 // Y[k] = [W_0; W_1; ...] X[k]: the weights' rows side by side in Y, for K rows of X. Where
@@ -675,7 +686,7 @@ static emprise_status linear_batch_rows(emprise_hip* h, int nw, const Weight* co
             const uint32_t type = wt->type;
             int j = i, nr = 0;
             qa.nseg = 0;
-            while (j < nw && ws[j]->type == type) {
+            while (j < nw && ws[j]->type == type && on_q16(ws[j])) {
                 qa.w[qa.nseg] = static_cast<const uint8_t*>(ws[j]->dev);
                 qa.row0[qa.nseg++] = nr;
                 nr += (int)ws[j]->rows;
@@ -779,6 +790,13 @@ emprise_status emprise_hip_ffn_gate_up_batch(emprise_hip* h, emprise_weight gate
         qa.ldy = (int)ldy;
         qa.pair = 1;
         return run_gemm_q16(h, g->type, qa, 4ull * K * cols * F);
+    }
+    if (X % 16 == 0 && ldx % 4 == 0 && u->type == g->type && (g->type == kQ6K || g->type == kQ4K) && by_row(h, g, K)) {
+        for (int k = 0; k < K; ++k) {
+            Proj p[2] = {{g, y + (size_t)k * ldy}, {u, nullptr}};
+            TRY(run_matvec(h, p, 2, kMvSwiglu, nullptr, reinterpret_cast<const float*>(X) + (size_t)k * ldx, nullptr, nullptr, 0, nullptr));
+        }
+        return EMPRISE_OK;
     }
     // otherwise the two projections (gate into Y, up into scratch), then swiglu per row
     void* ub;

@@ -666,6 +666,41 @@ def test_graph_keeps_the_scratch_it_was_captured_with(tokens, cols):
 
 
 @pytest.mark.parametrize("wtype", [Q6_K, Q4_K])
+@pytest.mark.parametrize("rows,cols", [(300, 768), (2049, 2048), (9000, 2048), (40, 512), (100, 7680)])
+def test_two_tokens_by_row_or_gemm(backend, wtype, rows, cols):
+    """Two rows: every call that a weight takes part in gives its rows the same bits -- alone, beside
+    a larger weight that goes the other way, and as gate and up of an FFN -- and right ones."""
+    rng = np.random.default_rng(rows + cols)
+    be, n = backend, 9000
+    data = [matrix(rng, wtype, r, cols) for r in (rows, rows, n)]
+    w = [be.upload_weight(wtype, cols, r, d) for r, d in zip((rows, rows, n), data)]
+    X = rng.standard_normal((2, cols + 4)).astype(np.float32)
+    xd = be.to_device(X)
+    y = [be.alloc(2 * rows * 4) for _ in range(3)]
+    many = be.alloc(2 * (2 * rows + n) * 4)
+    be.linear_batch_many([w[0]], xd, cols + 4, y[0], rows, 2)
+    be.linear_batch_many([w[1]], xd, cols + 4, y[1], rows, 2)
+    a, b = be.download(y[0], (2, rows)), be.download(y[1], (2, rows))
+    be.linear_batch_many([w[0], w[2], w[1]], xd, cols + 4, many, 2 * rows + n, 2)
+    m = be.download(many, (2, 2 * rows + n))
+    assert np.array_equal(m[:, :rows], a) and np.array_equal(m[:, rows + n:], b)
+    be.ffn_gate_up_batch(w[0], w[1], xd, cols + 4, y[2], rows, 2)
+    be.swiglu(y[0], y[1], 2 * rows)
+    assert np.array_equal(be.download(y[2], 2 * rows), be.download(y[0], 2 * rows))
+    wd = be.alloc(n * cols * 4)
+    for k, (got, r) in enumerate(((a, rows), (b, rows), (m[:, rows:rows + n], n))):
+        be.dequantize_rows(w[k], 0, r, wd)
+        W = be.download(wd, (r, cols))
+        ref = X[:, :cols].astype(np.float64) @ W.astype(np.float64).T
+        extra = 2.0**-18 * np.abs(X).sum(1, keepdims=True) * np.abs(W).max() if wtype == Q4_K else 0.0
+        assert np.all(np.abs(got - ref) <= _gemm_bound(W, X[:, :cols], cols) + extra)
+    for q in [xd, many, wd] + y:
+        be.free(q)
+    for q in w:
+        be.weight_free(q)
+
+
+@pytest.mark.parametrize("wtype", [Q6_K, Q4_K])
 @pytest.mark.parametrize("tokens,cols", [(2, 768), (5, 4096), (8, 1280), (9, 768), (70, 512), (200, 4096)])
 def test_small_activations_beside_large_ones(backend, wtype, tokens, cols):
     """Of each 256 columns the first 32 are large and their weights zero, and one other value is
