@@ -71,14 +71,13 @@ def test_linear_lm_head(backend, wtype):
                                                (Q6_K, 8, 4096, 4096), (Q6_K, 200, 300, 4096), (Q4_K, 129, 1000, 8192),
                                                (Q6_K, 40, 130, 12288), (Q4_K, 8, 128, 4096)])
 def test_linear_batch(backend, wtype, K, rows, cols):
-    """Backend::linear_batch (backend.hpp:20-24): Y[k] = W X[k]. From 8 tokens up it runs
-    on the matrix cores -- chunked Q6_K/Q4_K weights on exact fp16 pieces of weights and
-    activations with FP32 sums, other weights as an FP32 GEMM on exactly dequantised
-    weights; from 2 to 7 through a chunked Q6_K/Q4_K matrix as the small-batch matvec (up
-    to 4 inputs per launch, 3 at 12288 columns, the weights read once per launch); every
-    token must match the CPU matvec, and the single-token projection, to the per-op bar
-    (batched == sequential, reference tests/core.cpp:149-164). Token and row counts off
-    the 128 x 128 tiles included."""
+    """Backend::linear_batch (backend.hpp:20-24): Y[k] = W X[k]. Q6_K/Q4_K weights run on the
+    matrix cores from exact fp16 pieces with FP32 sums, once the tokens no longer fit one
+    small-batch matvec launch (chunked weights: 4 inputs, 3 at 12288 columns, the weights read
+    once per launch), or a matvec each; other weights from 8 tokens up as an FP32 GEMM on
+    exactly dequantised weights. Every token must match the CPU matvec, and the single-token
+    projection, to the per-op bar (batched == sequential, reference tests/core.cpp:149-164).
+    Token and row counts off the workgroups' tiles included."""
     rng = np.random.default_rng(K * 131 + rows + cols + wtype)
     raw = matrix(rng, wtype, rows, cols)
     X = rng.standard_normal((K, cols)).astype(np.float32)
