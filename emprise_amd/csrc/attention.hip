@@ -474,7 +474,7 @@ __global__ __launch_bounds__(256) void rope_table_kernel(float2* t, int context,
 //
 // Bound by the matrix cores and, about as much, by LDS reads (80 KiB per wave and tile): 2048
 // positions behind 4096 of the 9B shape (16 Q / 4 KV heads x 256) are 172 GFLOP, four and a half
-// times that in 16-bit products; 733 us for all the kernels here, of which the split 21 and the
+// times that in 16-bit products; 750 us for all the kernels here, of which the split 21 and the
 // prep 24. As two FP32 GEMMs per head with the scores in memory and a softmax pass between them it
 // took 2570 us and 805 MB of scratch, with 1.4e-6 of error against 64 bits, now 4e-7 (relative,
 // whole output). P.V from two fp16 pieces with an exponent per tile of values took 579 us, with

@@ -1174,7 +1174,7 @@ emprise_status emprise_hip_attention_batch(emprise_hip* h, const emprise_hip_att
         a.part = static_cast<float*>(part);
         a.stat = a.part + splits * hq;
     }
-    // K/V rows 0..first+count-1 read twice (scores, transpose), the new rows written
+    // K/V rows 0..first+count-1 read, written and read as operands (each counted at the rows' size)
     const uint64_t bytes = 3 * (uint64_t)(first_position + count) * p->kv_heads * p->head_dim * 4 + count * qkv_w * 4;
     return traced(h, "attention_batch", bytes, [&] { return launch_attention_batch(a, h->stream); });
 }
