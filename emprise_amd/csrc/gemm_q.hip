@@ -366,11 +366,14 @@ __device__ __forceinline__ void q_store(const QGemmArgs& a, int n0, int t0, int 
 // loaded a whole block ahead (a second register set) instead of during the block's last
 // unit step. Grid: x = row groups, y = token groups, z = column spans. a.spans > 1 with one
 // z layer runs the spans one after the other, adding them in the order the reduction
-// would, so the results do not depend on which of the two forms ran.
+// would, so the results do not depend on which of the two forms ran. (The loops of one round
+// are for the compiler's schedule. With / without them, us: FFN 4096 -> 12288 of 99 tokens,
+// Q6_K 157.8 / 158.9, Q4_K 138.1 / 140.0; 2048 -> 6144 of 50, 50.2 / 50.4, 50.9 / 51.2; 1024 ->
+// 3072 of 700, 233.9 / 234.5, 222.4 / 222.3.)
 template <int T, bool CH, int MT, bool PF>
 __global__ __launch_bounds__(MT * 64, 2) void gemm_q16_kernel(QGemmArgs a) {
     constexpr int TH = MT * 64;                         // threads
-    constexpr int AV = MT * 256;                        // 16-byte pieces of a step's operands
+    constexpr int AV = MT * 4096 / 16;                  // 16-byte pieces of a step's operands
     constexpr int AN = AV / TH;
     constexpr int SV = MT * (T == kQ4K ? 36 : 4);       // of a block's side data: 2^e, then the unit sums
     constexpr int SN = (SV + TH - 1) / TH;
@@ -385,8 +388,9 @@ __global__ __launch_bounds__(MT * 64, 2) void gemm_q16_kernel(QGemmArgs a) {
     const int b0 = gridDim.z > 1 ? blockIdx.z * a.span : 0;
     const int b1 = gridDim.z > 1 ? min(b0 + a.span, nb) : nb;
 
-    // (rows past N read the last row; their results are not stored)
-    const uint8_t* row = q_row<T>(a, min(n0 + rj, a.N - 1), nb);
+    const uint8_t* row[1];  // (rows past N read the last row; their results are not stored)
+#pragma unroll
+    for (int i = 0; i < 1; ++i) row[0] = q_row<T>(a, min(n0 + 16 * i + rj, a.N - 1), nb);
 
     // step s (global numbering): unit step s % 4 of block s / 4
     uint4 ra[AN], rs[SN];
@@ -418,40 +422,53 @@ __global__ __launch_bounds__(MT * 64, 2) void gemm_q16_kernel(QGemmArgs a) {
         }
     };
 
-    floatx4 cb[1][MT], acc[1][MT], tot[MT];
+    floatx4 cb[1][MT], acc[1][MT], tot[1][MT];
 #pragma unroll
-    for (int m = 0; m < MT; ++m) cb[0][m] = acc[0][m] = tot[m] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int m = 0; m < MT; ++m) {
+        cb[0][m] = acc[0][m] = floatx4{0.f, 0.f, 0.f, 0.f};
+        tot[0][m] = floatx4{0.f, 0.f, 0.f, 0.f};
+    }
 
-    QRaw<T> raw, nxt;
+    QRaw<T> raw[1], nxt[1];
     const int s0 = b0 * 4, s1 = b1 * 4;
     load_a(s0);
-    q_load<CH>(raw, row, nb, b0, q);
+#pragma unroll
+    for (int i = 0; i < 1; ++i) q_load<CH>(raw[0], row[0], nb, b0, q);
     store_a(s0, s0 & 1);
     load_a(min(s0 + 1, s1 - 1));
     lds_barrier();
 
     for (int b = b0; b < b1; ++b) {
-        if constexpr (PF) q_load<CH>(nxt, row, nb, min(b + 1, b1 - 1), q);
-        uint32_t dblk[1], mins[1];
-        q_block_scales<CH>(raw, q, dblk[0], mins[0]);
+        if constexpr (PF) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int s = b * 4 + j, buf = s & 1;
+            for (int i = 0; i < 1; ++i) q_load<CH>(nxt[0], row[0], nb, min(b + 1, b1 - 1), q);
+        }
+        uint32_t dblk[1], mins[1];
+#pragma unroll
+        for (int i = 0; i < 1; ++i) q_block_scales<CH>(raw[0], q, dblk[0], mins[0]);
+#pragma unroll
+        for (int js = 0; js < 4; ++js) {
+            const int s = b * 4 + js, buf = s & 1;
             // the next step's operands go into the buffer that every wave finished with
-            // before the last barrier; their loads had a whole step (with PF behind the decode: FFN
-            // 2048 -> 6144 of 50 tokens, Q4_K, 51.2 us, before it 52.3)
-            auto stage = [&] {
-                if (s + 1 < s1) store_a(s + 1, buf ^ 1);
-                load_a(min(s + 2, s1 - 1));
-            };
-            if constexpr (!PF) stage();
+            // before the last barrier; their loads had a whole step
+            if (s + 1 < s1) store_a(s + 1, buf ^ 1);
+            load_a(min(s + 2, s1 - 1));
             const half8* A = reinterpret_cast<const half8*>(As[buf]);
-            auto products = [&] {
+#pragma unroll
+            for (int ju = 0; ju < 1; ++ju) {
+                const int j = js + ju;
                 half8 wh[1][2], wl[1][2];
-                if constexpr (T == kQ6K) q6_unit(raw, j, wh[0], wl[0]);
-                else q4_unit<CH>(raw, q, j, wh[0]);
-                if constexpr (PF) stage();
-                else if (j == 3) q_load<CH>(raw, row, nb, min(b + 1, b1 - 1), q);
+#pragma unroll
+                for (int i = 0; i < 1; ++i) {
+                    if constexpr (T == kQ6K) q6_unit(raw[0], j, wh[0], wl[0]);
+                    else q4_unit<CH>(raw[0], q, j, wh[0]);
+                }
+                if constexpr (!PF) {
+                    if (j == 3) {
+#pragma unroll
+                        for (int i = 0; i < 1; ++i) q_load<CH>(raw[0], row[0], nb, min(b + 1, b1 - 1), q);
+                    }
+                }
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
                     // MP token tiles at a time: consecutive MFMAs add to different accumulators
@@ -466,27 +483,29 @@ __global__ __launch_bounds__(MT * 64, 2) void gemm_q16_kernel(QGemmArgs a) {
                         q_products<T, 1, MP, MT>(xh, xl, wh, wl, h, m, cb);
                     }
                 }
-            };
-            products();
-            if (j == 3) {
+            }
+            if (js == 3) {
                 q_block_end<T, 1, MT>(Ss[b & 1], lane, dblk, mins, cb, acc);
                 if (gridDim.z == 1 && a.spans > 1 && ((b + 1) % a.span == 0 || b + 1 == b1)) {
 #pragma unroll
                     for (int m = 0; m < MT; ++m)
 #pragma unroll
                         for (int r = 0; r < 4; ++r) {
-                            tot[m][r] += acc[0][m][r];
+                            tot[0][m][r] += acc[0][m][r];
                             acc[0][m][r] = 0.f;
                         }
                 }
             }
             lds_barrier();
         }
-        if constexpr (PF) raw = nxt;
+        if constexpr (PF) {
+#pragma unroll
+            for (int i = 0; i < 1; ++i) raw[0] = nxt[0];
+        }
     }
     if (gridDim.z == 1 && a.spans > 1) {
 #pragma unroll
-        for (int m = 0; m < MT; ++m) acc[0][m] = tot[m];
+        for (int m = 0; m < MT; ++m) acc[0][m] = tot[0][m];
     }
     q_store<1, MT>(a, n0, t0, rj, q, acc);
 }
